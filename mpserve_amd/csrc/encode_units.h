@@ -1,0 +1,527 @@
+// The sidecar builder's passes over the elements, one *unit* of one bucket a
+// workgroup (included by fp8_encode.hip, inside its namespace).
+//
+// A bucket's elements share one scale, so inside a bucket a (key, symbol) pair
+// is 24 bits, and a scale has a few thousand distinct pairs: they fit one LDS
+// hash table. A unit is a run of whole steps (k_eff elements, one a substream)
+// of one bucket, so the same units serve every pass:
+//   unit_hist    counts a unit's pairs in LDS and writes them as a list;
+//   merge_lists  adds up the lists of one scale (one q range of it) in LDS and
+//                sorts them by (q, count, symbol): the builder's item order;
+//   scan_parts, number_keys   table ids of the keys, in (scale, q) order;
+//   (the codebooks, from the sorted entries, fp8_encode.hip)
+//   unit_codes   maps a unit's elements to code words through an LDS table of
+//                the scale's pairs, stores them (16 bits an element, in bucket
+//                order) and sums each substream's bits within the unit;
+//   bucket_starts, bucket_bases   start bits of the substreams and buckets;
+//   unit_pack    writes each substream's piece of the unit into the bitstream.
+// Every pass has as many workgroups as units, so a tensor of few buckets, or
+// of few substreams a bucket, fills the chip too: a piece of a substream
+// starts at its substream's start bit plus the bits of its earlier pieces.
+//
+// Measured against one work-item a substream over a hash table in global
+// memory (the general path of fp8_encode.hip, for the calls this one does not
+// take), one 14336 x 4096 FP8 weight, k = 1024: counting 1.89 ms -> 69 us,
+// grouping and sorting 1.38 ms -> 80 us, code words and bits 1.60 ms -> 101 us,
+// packing 0.57 -> 0.26 ms; the whole call 10.7 -> 2.8 ms.
+#pragma once
+
+constexpr int kUnitThreads = 1024;
+constexpr uint32_t kPairSlots = 8192;   // LDS slots of a unit's, or a part's, pairs
+constexpr uint32_t kUnitRows = 1024;    // a unit spans at most this many rows (groups), + 2 partial ones
+constexpr uint32_t kNoPair = 0xFFFFFFFFu;
+constexpr uint32_t kMaxProbes = 256;
+
+struct Unit {
+  uint32_t bucket;
+  uint32_t i0, i1;  // steps: elements [i0 * k_eff, min(i1 * k_eff, total)) of the bucket
+  uint32_t sidx;    // the bucket's scale
+};
+
+struct UnitArgs {
+  const Unit *units;
+  const uint16_t *bf16;
+  const uint8_t *q;
+  uint32_t m;
+  uint32_t qmask;
+  const int32_t *row_offsets;
+  const int32_t *row_indices;
+  const int32_t *col_start;  // by bucket (null with row_col)
+  const int32_t *col_len;
+  const int32_t *row_col;    // by row: column start of each group (by-scale layout), or null
+  uint32_t k;
+  int32_t vec8;  // 8 elements of a row can be loaded at once (widths, starts and pointers are multiples)
+};
+
+struct UnitGeom {
+  uint32_t cl, k_eff, total;  // the bucket
+  uint32_t e0, e1, r0;        // the unit's elements and its first row
+};
+
+// Where a pair's probes start: the symbol's sign and low bits. The symbols of
+// one scale span some 20 of the 32 octaves these bits tell apart, so pairs of
+// different symbols start at different slots; a symbol's second q value (at a
+// rounding boundary) steps away.
+template <uint32_t kSlots>
+__device__ __forceinline__ uint32_t pair_slot(uint32_t pair) {
+  static_assert(kSlots == 8192 || kSlots == 16384, "sign + 12 or 13 low bits");
+  return kSlots == 8192 ? (pair & 0xFFFu) | ((pair >> 3) & 0x1000u) : (pair & 0x1FFFu) | ((pair >> 2) & 0x2000u);
+}
+__device__ __forceinline__ uint32_t pair_step(uint32_t pair) { return ((pair >> 16) * 0x2F2u + 0x4D7u) | 1u; }
+
+// Elements of bucket `b` are counted in 32 bits: a tensor has fewer than 2^32.
+// Stages the unit's row offsets (first element of each row's column range) in LDS.
+__device__ __forceinline__ UnitGeom unit_geom(const UnitArgs &a, const Unit &u, uint32_t *s_base) {
+  UnitGeom g;
+  const int32_t ra = a.row_offsets[u.bucket];
+  const uint32_t rows = (uint32_t)(a.row_offsets[u.bucket + 1] - ra);
+  g.cl = (uint32_t)a.col_len[u.bucket];
+  g.total = rows * g.cl;
+  g.k_eff = a.k < g.total ? a.k : (g.total > 0 ? g.total : 1u);
+  g.e0 = u.i0 * g.k_eff;
+  const uint64_t end = (uint64_t)u.i1 * g.k_eff;
+  g.e1 = end < g.total ? (uint32_t)end : g.total;
+  g.r0 = g.e0 / g.cl;
+  const uint32_t nrows = g.e1 > g.e0 ? (g.e1 - 1u) / g.cl - g.r0 + 1u : 0u;
+  const uint32_t c0 = a.row_col ? 0u : (uint32_t)a.col_start[u.bucket];
+  for (uint32_t r = threadIdx.x; r < nrows; r += kUnitThreads) {
+    const int32_t at = ra + (int32_t)(g.r0 + r);
+    s_base[r] = (uint32_t)a.row_indices[at] * a.m + (a.row_col ? (uint32_t)a.row_col[at] : c0);
+  }
+  return g;
+}
+
+// Adds `add` to a pair's count; false when no slot was found.
+__device__ __forceinline__ bool pair_add(uint32_t *s_key, uint32_t *s_cnt, uint32_t pair, uint32_t add) {
+  uint32_t h = pair_slot<kPairSlots>(pair);
+  for (uint32_t i = 0; i < kMaxProbes; ++i) {
+    uint32_t cur = s_key[h];
+    if (cur == kNoPair) {
+      cur = atomicCAS(&s_key[h], kNoPair, pair);
+      if (cur == kNoPair) cur = pair;
+    }
+    if (cur == pair) {
+      atomicAdd(&s_cnt[h], add);
+      return true;
+    }
+    h = (h + pair_step(pair)) & (kPairSlots - 1u);
+  }
+  return false;
+}
+
+// One unit's pairs and counts -> lists[list_off[u] ..] (list_n[u] of them, any
+// order). Bound by the LDS: a read and an add an element, at random banks.
+__global__ __launch_bounds__(kUnitThreads) void unit_hist(UnitArgs a, const uint32_t *__restrict__ list_off,
+                                                          uint2 *__restrict__ lists, uint32_t *__restrict__ list_n,
+                                                          uint32_t *overflow) {
+  __shared__ uint32_t s_key[kPairSlots], s_cnt[kPairSlots], s_base[kUnitRows + 2], s_n;
+  const uint32_t tid = threadIdx.x;
+  const Unit u = a.units[blockIdx.x];
+  const UnitGeom g = unit_geom(a, u, s_base);
+  for (uint32_t i = tid; i < kPairSlots; i += kUnitThreads) {
+    s_key[i] = kNoPair;
+    s_cnt[i] = 0u;
+  }
+  if (tid == 0) s_n = 0u;
+  __syncthreads();
+  bool ok = true;
+  uint32_t done = g.e0;
+  if (a.vec8 && g.e0 % 8u == 0u) {
+    done = g.e1 & ~7u;
+    for (uint32_t e = g.e0 + 8u * tid; e < done; e += 8u * kUnitThreads) {
+      const uint32_t r = e / g.cl;
+      const uint32_t idx = s_base[r - g.r0] + (e - r * g.cl);
+      const uint4 b = *reinterpret_cast<const uint4 *>(a.bf16 + idx);
+      const uint2 q = *reinterpret_cast<const uint2 *>(a.q + idx);
+      const uint32_t bw[4] = {b.x, b.y, b.z, b.w}, qw[2] = {q.x, q.y};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t sym = (bw[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
+        const uint32_t qv = (qw[j / 4] >> (8 * (j & 3))) & a.qmask;
+        ok &= pair_add(s_key, s_cnt, (qv << 16) | sym, 1u);
+      }
+    }
+    if (done < g.e0) done = g.e0;
+  }
+  for (uint32_t e = done + tid; e < g.e1; e += kUnitThreads) {
+    const uint32_t r = e / g.cl;
+    const uint32_t idx = s_base[r - g.r0] + (e - r * g.cl);
+    ok &= pair_add(s_key, s_cnt, ((uint32_t)(a.q[idx] & a.qmask) << 16) | a.bf16[idx], 1u);
+  }
+  if (!ok) atomicOr(overflow, 1u);
+  __syncthreads();
+  uint2 *out = lists + list_off[blockIdx.x];
+  const int lane = (int)(tid & 63u);
+  for (uint32_t i = tid; i < kPairSlots; i += kUnitThreads) {
+    const uint32_t key = s_key[i];
+    const uint64_t live = __ballot(key != kNoPair);
+    uint32_t base = 0;
+    if (lane == 0 && live) base = atomicAdd(&s_n, (uint32_t)__popcll(live));
+    base = (uint32_t)__shfl((int)base, 0);
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    if (key != kNoPair) out[base + (uint32_t)__popcll(live & below)] = make_uint2(key, s_cnt[i]);
+  }
+  __syncthreads();
+  if (tid == 0) list_n[blockIdx.x] = s_n;
+}
+
+// Part p of scale s (blockIdx.x = s * parts + p): the pairs with q in
+// [p * qvals / parts, (p + 1) * qvals / parts), added up over the scale's unit
+// lists and sorted by (q, count as int, symbol) into skeys[part_off ..]; the
+// keys' entry counts and first entries (tcount, toff, indexed s * 256 + q).
+// Sorted in LDS (bitonic, over the pairs found), which bounds it; the parts
+// keep the sorts short and the workgroups many when the scales are few.
+__global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__restrict__ scale_unit_off,
+                                                            const uint32_t *__restrict__ unit_of_scale,
+                                                            const uint32_t *__restrict__ list_off,
+                                                            const uint32_t *__restrict__ list_n,
+                                                            const uint2 *__restrict__ lists, uint32_t parts,
+                                                            uint32_t qvals, const uint32_t *__restrict__ part_off,
+                                                            uint64_t *__restrict__ skeys, uint32_t *__restrict__ tcount,
+                                                            uint32_t *__restrict__ toff, uint32_t *__restrict__ part_n,
+                                                            uint32_t *__restrict__ part_keys, uint32_t *overflow) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_pairs[2 * kPairSlots];
+  __shared__ uint32_t s_n, s_keys;
+  uint32_t *s_key = s_pairs, *s_cnt = s_pairs + kPairSlots;
+  uint64_t *s_sort = reinterpret_cast<uint64_t *>(s_pairs);
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t s = blockIdx.x / parts, p = blockIdx.x % parts;
+  const uint32_t q0 = p * qvals / parts, q1 = (p + 1u) * qvals / parts;
+  for (uint32_t i = tid; i < kPairSlots; i += kUnitThreads) {
+    s_key[i] = kNoPair;
+    s_cnt[i] = 0u;
+  }
+  if (tid == 0) s_n = s_keys = 0u;
+  __syncthreads();
+  bool ok = true;
+  for (uint32_t i = scale_unit_off[s] + wave; i < scale_unit_off[s + 1]; i += kUnitThreads / 64) {
+    const uint32_t u = unit_of_scale[i];
+    const uint32_t n = list_n[u];
+    const uint2 *l = lists + list_off[u];
+    for (uint32_t j = lane; j < n; j += 64u) {
+      const uint2 e = l[j];
+      const uint32_t q = e.x >> 16;
+      if (q >= q0 && q < q1) ok &= pair_add(s_key, s_cnt, e.x, e.y);
+    }
+  }
+  if (!ok) atomicOr(overflow, 1u);
+  __syncthreads();
+  // The pairs as sort keys, in place: read into registers, then written back dense.
+  constexpr int kPer = kPairSlots / kUnitThreads;
+  uint64_t v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint32_t key = s_key[tid + i * kUnitThreads], cnt = s_cnt[tid + i * kUnitThreads];
+    v[i] = key == kNoPair ? ~0ull : ((uint64_t)(key >> 16) << 48) | item_key(cnt, key & 0xFFFFu);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const uint64_t live = __ballot(v[i] != ~0ull);
+    uint32_t base = 0;
+    if (lane == 0 && live) base = atomicAdd(&s_n, (uint32_t)__popcll(live));
+    base = (uint32_t)__shfl((int)base, 0);
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64u - lane));
+    if (v[i] != ~0ull) s_sort[base + (uint32_t)__popcll(live & below)] = v[i];
+  }
+  __syncthreads();
+  const uint32_t n = s_n;
+  uint32_t np = 1;
+  while (np < n) np <<= 1;
+  for (uint32_t i = n + tid; i < np; i += kUnitThreads) s_sort[i] = ~0ull;
+  __syncthreads();
+  for (uint32_t size = 2; size <= np; size <<= 1) {
+    for (uint32_t d = size >> 1; d > 0; d >>= 1) {
+      for (uint32_t i = tid; i < np / 2; i += kUnitThreads) {
+        const uint32_t x = ((i & ~(d - 1u)) << 1) | (i & (d - 1u)), y = x + d;
+        const uint64_t vx = s_sort[x], vy = s_sort[y];
+        if ((vx > vy) == ((x & size) == 0u)) {
+          s_sort[x] = vy;
+          s_sort[y] = vx;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  const uint32_t off = part_off[blockIdx.x];
+  for (uint32_t i = tid; i < n; i += kUnitThreads) skeys[off + i] = s_sort[i];
+  if (tid < q1 - q0) {
+    auto first = [&](uint32_t q) {  // first entry with a q of at least this one
+      uint32_t lo = 0, hi = n;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if ((uint32_t)(s_sort[mid] >> 48) < q) lo = mid + 1u;
+        else hi = mid;
+      }
+      return lo;
+    };
+    const uint32_t a = first(q0 + tid), b = first(q0 + tid + 1u);
+    tcount[s * 256u + q0 + tid] = b - a;
+    toff[s * 256u + q0 + tid] = off + a;
+    if (b > a) atomicAdd(&s_keys, 1u);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    part_n[blockIdx.x] = n;
+    part_keys[blockIdx.x] = s_keys;
+  }
+}
+
+// Exclusive sums of the parts' key counts (in place), and in res: [0] keys in
+// all, [1] entries in all, [2] most entries of one scale. One workgroup.
+__global__ __launch_bounds__(kScanBlock) void scan_parts(uint32_t *part_keys, const uint32_t *part_n, uint32_t scales,
+                                                         uint32_t parts, uint32_t *res) {
+  __shared__ uint32_t s_tmp[16], s_most, s_sum;
+  const uint32_t n = scales * parts, tid = threadIdx.x;
+  if (tid == 0) s_most = s_sum = 0u;
+  uint32_t run = 0;
+  for (uint32_t b = 0; b < n; b += kScanBlock) {
+    const uint32_t v = b + tid < n ? part_keys[b + tid] : 0u;
+    uint32_t total = 0;
+    const uint32_t ex = block_exclusive_scan(v, s_tmp, &total);
+    if (b + tid < n) part_keys[b + tid] = run + ex;
+    run += total;
+  }
+  __syncthreads();
+  for (uint32_t s = tid; s < scales; s += kScanBlock) {
+    uint32_t d = 0;
+    for (uint32_t p = 0; p < parts; ++p) d += part_n[s * parts + p];
+    atomicAdd(&s_sum, d);
+    atomicMax(&s_most, d);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    res[0] = run;
+    res[1] = s_sum;
+    res[2] = s_most;
+  }
+}
+
+// Table ids of scale blockIdx.x's keys, and their size classes' lists.
+__global__ __launch_bounds__(256) void number_keys(const uint32_t *__restrict__ tcount,
+                                                   const uint32_t *__restrict__ part_keys, uint32_t parts, uint32_t T,
+                                                   uint32_t qvals, uint32_t *__restrict__ tgid,
+                                                   uint32_t *__restrict__ gid_tkey, uint32_t *lists, uint32_t cap,
+                                                   uint32_t *n3) {
+  __shared__ uint32_t s_tmp[16];
+  const uint32_t tk = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t ni = threadIdx.x < qvals ? tcount[tk] : 0u;
+  const uint32_t gid = part_keys[blockIdx.x * parts] + block_exclusive_scan(ni ? 1u : 0u, s_tmp, nullptr);
+  if (ni) {
+    tgid[tk] = gid;
+    gid_tkey[gid] = tk;
+  }
+  cb_append(gid, ni ? cb_class(ni, T) : -1, lists, cap, n3);
+}
+
+// Code word of an element, 16 bits (L <= 11): code | length << 11 | raw16 << 15.
+__device__ __forceinline__ uint32_t cw16(uint32_t cw) {
+  return (cw & 0x7FFu) | (cw_len(cw) << 11) | ((cw & kRaw) ? 0x8000u : 0u);
+}
+__device__ __forceinline__ uint32_t cw16_len(uint32_t c) { return (c >> 11) & 0xFu; }
+
+// Pieces of a unit: piece j of substream t is steps [i0 + j * per, + per) of the
+// unit, up to 1024 / k_eff pieces side by side; thread j * k_eff + t has it.
+__device__ __forceinline__ uint32_t piece_steps(const Unit &u, uint32_t k_eff) {
+  const uint32_t nsub = kUnitThreads / k_eff;
+  return (u.i1 - u.i0 + nsub - 1u) / nsub;
+}
+struct UnitPiece {
+  uint32_t lane, i, iend;  // substream, first step and end (none: i >= iend)
+};
+__device__ __forceinline__ UnitPiece unit_piece(const Unit &u, uint32_t k_eff) {
+  const uint32_t sub = threadIdx.x / k_eff, per = piece_steps(u, k_eff);
+  UnitPiece p;
+  p.lane = threadIdx.x - sub * k_eff;
+  p.i = u.i0 + sub * per;
+  p.iend = sub >= kUnitThreads / k_eff ? 0u : p.i + per < u.i1 ? p.i + per : u.i1;
+  return p;
+}
+
+// The unit's elements as code words (codes[bucket_elem[b] + e], e in bucket
+// order) and each piece's bits (piece_bits[unit * 1024 + thread]).
+template <uint32_t kSlots>
+__global__ __launch_bounds__(kUnitThreads) void unit_codes(UnitArgs a, uint32_t parts,
+                                                           const uint32_t *__restrict__ part_off,
+                                                           const uint32_t *__restrict__ part_n,
+                                                           const uint64_t *__restrict__ skeys,
+                                                           const uint32_t *__restrict__ entry_cw,
+                                                           const uint32_t *__restrict__ bucket_elem,
+                                                           uint16_t *__restrict__ codes,
+                                                           uint32_t *__restrict__ piece_bits, uint32_t *err) {
+  __shared__ uint2 s_map[kSlots];  // pair, code word
+  __shared__ uint32_t s_base[kUnitRows + 2];
+  const uint32_t tid = threadIdx.x;
+  const Unit u = a.units[blockIdx.x];
+  const UnitGeom g = unit_geom(a, u, s_base);
+  for (uint32_t i = tid; i < kSlots; i += kUnitThreads) s_map[i] = make_uint2(kNoPair, 0u);
+  __syncthreads();
+  for (uint32_t p = 0; p < parts; ++p) {
+    const uint32_t off = part_off[u.sidx * parts + p], n = part_n[u.sidx * parts + p];
+    for (uint32_t i = tid; i < n; i += kUnitThreads) {
+      const uint64_t key = skeys[off + i];
+      const uint32_t pair = ((uint32_t)(key >> 48) << 16) | cb_sym(key);
+      const uint32_t cw = cw16(entry_cw[off + i]);
+      uint32_t h = pair_slot<kSlots>(pair);
+      while (atomicCAS(&s_map[h].x, kNoPair, pair) != kNoPair) h = (h + pair_step(pair)) & (kSlots - 1u);
+      s_map[h].y = cw;
+    }
+  }
+  __syncthreads();
+  const UnitPiece pc = unit_piece(u, g.k_eff);
+  uint32_t bits = 0;
+  bool found = true;
+  uint16_t *out = codes + bucket_elem[u.bucket];
+  constexpr int kB = 8;  // elements in flight a work-item
+  for (uint32_t i = pc.i; i < pc.iend; i += kB) {
+    uint32_t pair[kB], e[kB];
+#pragma unroll
+    for (int j = 0; j < kB; ++j) {
+      e[j] = pc.lane + (i + j) * g.k_eff;
+      const bool in = i + j < pc.iend && e[j] < g.e1;
+      const uint32_t ee = in ? e[j] : g.e0;  // past the end: the unit's first element, not stored
+      e[j] = in ? e[j] : kNoPair;
+      const uint32_t r = ee / g.cl;
+      const uint32_t idx = s_base[r - g.r0] + (ee - r * g.cl);
+      pair[j] = ((uint32_t)(a.q[idx] & a.qmask) << 16) | a.bf16[idx];
+    }
+#pragma unroll
+    for (int j = 0; j < kB; ++j) {
+      uint32_t h = pair_slot<kSlots>(pair[j]);
+      uint2 s = s_map[h];
+      while (s.x != pair[j] && s.x != kNoPair) {
+        h = (h + pair_step(pair[j])) & (kSlots - 1u);
+        s = s_map[h];
+      }
+      found &= s.x == pair[j];
+      if (e[j] != kNoPair) {
+        out[e[j]] = (uint16_t)s.y;
+        bits += cw16_len(s.y) + ((s.y >> 15) << 4);
+      }
+    }
+  }
+  piece_bits[(uint64_t)blockIdx.x * kUnitThreads + tid] = bits;
+  if (!found) atomicOr(err, 4u);
+}
+
+// Bucket blockIdx.x's substreams: start bits (k + 1 of them) from the pieces'
+// bits, each piece's offset from its substream's start (in place), and the
+// bucket's bits.
+__global__ __launch_bounds__(kUnitThreads) void bucket_starts(const Unit *__restrict__ units,
+                                                              const uint32_t *__restrict__ bucket_unit,
+                                                              const uint32_t *__restrict__ lane_base, uint32_t k,
+                                                              uint32_t *__restrict__ piece_bits,
+                                                              uint32_t *__restrict__ startbit,
+                                                              uint32_t *__restrict__ bucket_bits) {
+  __shared__ uint32_t s_tmp[16];
+  const uint32_t b = blockIdx.x, t = threadIdx.x;
+  const uint32_t k_eff = lane_base[b + 1] - lane_base[b];
+  uint32_t acc = 0;
+  if (t < k_eff) {
+    for (uint32_t i = bucket_unit[b]; i < bucket_unit[b + 1]; ++i) {
+      const Unit u = units[i];
+      const uint32_t per = piece_steps(u, k_eff), np = (u.i1 - u.i0 + per - 1u) / per;
+      uint32_t *pb = piece_bits + (uint64_t)i * kUnitThreads + t;
+      for (uint32_t j0 = 0; j0 < np; j0 += 4) {  // four loads at a time
+        uint32_t v[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) v[j] = j0 + j < np ? pb[(j0 + j) * k_eff] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+          if (j0 + j < np) pb[(j0 + j) * k_eff] = acc;
+          acc += v[j];
+        }
+      }
+    }
+  }
+  uint32_t total = 0;
+  const uint32_t ex = block_exclusive_scan(acc, s_tmp, &total);
+  uint32_t *sb = startbit + (uint64_t)b * (k + 1u);
+  if (t == 0) {
+    sb[0] = 0u;
+    bucket_bits[b] = total;
+  }
+  if (t < k) sb[t + 1] = t < k_eff ? ex + acc : total;
+}
+
+// 64-bit aligned bucket bases, and the end of the last bucket unaligned
+// (build_huffman.cu:813-818). One workgroup.
+__global__ __launch_bounds__(kScanBlock) void bucket_bases(const uint32_t *__restrict__ bucket_bits, uint32_t B,
+                                                           int64_t *__restrict__ bit_base) {
+  __shared__ uint32_t s_tmp[16];
+  const uint32_t tid = threadIdx.x;
+  uint64_t run = 0;  // 64-bit words
+  for (uint32_t b = 0; b < B; b += kScanBlock) {
+    const uint32_t bits = b + tid < B ? bucket_bits[b + tid] : 0u;
+    const uint32_t words = (uint32_t)(((uint64_t)bits + 63u) >> 6);
+    uint32_t total = 0;
+    const uint32_t ex = block_exclusive_scan(words, s_tmp, &total);
+    if (b + tid < B) bit_base[b + tid] = (int64_t)((run + ex) << 6);
+    if (b + tid + 1u == B) bit_base[B] = (int64_t)(((run + ex) << 6) + bits);
+    run += total;
+  }
+}
+
+// The unit's pieces into the (zeroed) bitstream, MSB-first in 32-bit chunks
+// (chunk c of the stream is u32 c ^ 1: a 64-bit word's first half is its high
+// half). A piece's first and last chunk may be shared with its neighbours and
+// are merged with atomicOr; the chunks between are its own.
+__global__ __launch_bounds__(kUnitThreads) void unit_pack(UnitArgs a, const uint32_t *__restrict__ bucket_elem,
+                                                          const uint16_t *__restrict__ codes,
+                                                          const uint32_t *__restrict__ piece_at,
+                                                          const uint32_t *__restrict__ startbit,
+                                                          const int64_t *__restrict__ bit_base,
+                                                          uint32_t *__restrict__ chunks) {
+  const Unit u = a.units[blockIdx.x];
+  const int32_t ra = a.row_offsets[u.bucket];
+  const uint32_t cl = (uint32_t)a.col_len[u.bucket];
+  const uint32_t total = (uint32_t)(a.row_offsets[u.bucket + 1] - ra) * cl;
+  const uint32_t k_eff = a.k < total ? a.k : total;
+  const UnitPiece pc = unit_piece(u, k_eff);
+  if (pc.i >= pc.iend) return;
+  const uint64_t p0 = (uint64_t)bit_base[u.bucket] + startbit[(uint64_t)u.bucket * (a.k + 1u) + pc.lane] +
+                      piece_at[(uint64_t)blockIdx.x * kUnitThreads + threadIdx.x];
+  uint64_t c = p0 >> 5;
+  uint64_t acc = 0;                       // bits from the top: `used` of them
+  uint32_t used = (uint32_t)(p0 & 31u);   // < 32 between elements
+  bool shared = true;                     // the chunk being filled may hold others' bits
+  auto flush = [&]() {
+    const uint32_t v = (uint32_t)(acc >> 32);
+    if (shared) atomicOr(chunks + (c ^ 1u), v);
+    else chunks[c ^ 1u] = v;
+    shared = false;
+    ++c;
+    acc <<= 32;
+    used -= 32u;
+  };
+  auto put = [&](uint32_t v, uint32_t n) {
+    acc |= (uint64_t)v << (64u - used - n);
+    used += n;
+    if (used >= 32u) flush();
+  };
+  const uint16_t *in = codes + bucket_elem[u.bucket];
+  constexpr int kB = 8;
+  for (uint32_t i = pc.i; i < pc.iend; i += kB) {
+    uint32_t w[kB];
+#pragma unroll
+    for (int j = 0; j < kB; ++j) {
+      const uint32_t e = pc.lane + (i + j) * k_eff;
+      w[j] = i + j < pc.iend && e < total ? in[e] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kB; ++j) {
+      const uint32_t len = cw16_len(w[j]);
+      if (len) put(w[j] & 0x7FFu, len);
+      if (w[j] & 0x8000u) {
+        const uint32_t e = pc.lane + (i + j) * k_eff, r = e / cl;
+        const int32_t at = ra + (int32_t)r;
+        const uint32_t col = (uint32_t)(a.row_col ? a.row_col[at] : a.col_start[u.bucket]) + (e - r * cl);
+        put(a.bf16[(uint64_t)(uint32_t)a.row_indices[at] * a.m + col], 16u);
+      }
+    }
+  }
+  if (used) {
+    const uint32_t v = (uint32_t)(acc >> 32);
+    if (v) atomicOr(chunks + (c ^ 1u), v);
+  }
+}

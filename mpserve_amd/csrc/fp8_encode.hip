@@ -2,18 +2,19 @@
 //
 // Produces byte for byte what the reference's host builder
 // huffman_build_fp8_decode_tables_entry (kernel/build_huffman.cu:292-969) produces:
-//   1. histogram of (scale, fp8) keys x BF16 symbols    (:392-401)   -> LDS-atomic pre-aggregation
-//                                                                        into a global open-addressing table
-//   2. keys in ascending order -> table id (gid)         (:403-412)   -> ballot/prefix-scan compaction,
-//                                                                        counting sort by key, scans
-//   3. per key: ESC selection, package-merge lengths,    (:445-578)   -> one work-item per key
+//   1. histogram of (scale, fp8) keys x BF16 symbols    (:392-401)
+//   2. keys in ascending order -> table id (gid)         (:403-412)
+//   3. per key: ESC selection, package-merge lengths,    (:445-578)   -> one wave per key, in LDS
 //      canonical codes in (count asc, sym asc) order,
 //      decode LUT and packed 4-bit lengths
-//   4. row buckets, bucket_table, U/uniq/uidx            (:582-783)   -> host (O(rows)) + one work-item
-//                                                                        per bucket
-//   5. per-lane bit counts, u32 lane starts, 64-bit      (:786-925)   -> two passes over the lanes with a
-//      aligned bucket bases, MSB-first packing                           scan between them; words shared by
-//                                                                        two lanes are merged with atomicOr
+//   4. row buckets, bucket_table, U/uniq/uidx            (:582-783)   -> host (O(rows)) + a kernel
+//   5. per-lane bit counts, u32 lane starts, 64-bit      (:786-925)
+//      aligned bucket bases, MSB-first packing
+// Steps 1, 2 and 5 run on units of one bucket over tables in LDS
+// (encode_units.h). The general path further down, over hash tables in global
+// memory with a work-item a substream, takes the calls the units do not: codes
+// longer than 11 bits, fewer than 32 substreams, tensors past 2^31 elements,
+// very small buckets, and scales with more pairs than an LDS table holds.
 // The reference is single-threaded; here every O(N) pass runs on the GPU.
 #include <hip/hip_runtime.h>
 
@@ -657,6 +658,7 @@ __global__ void codebook_kernel(CodebookArgs a) {
 // left to another launch.
 // ---------------------------------------------------------------------------
 constexpr int kCbLanes = 64;
+constexpr int kCbSmall = 64;  // the smallest NMAX: keys of at most this many entries and no ESC
 
 __device__ __forceinline__ uint32_t cb_count(uint64_t k) { return key_count(k); }
 __device__ __forceinline__ uint32_t cb_sym(uint64_t k) { return (uint32_t)(k & 0xFFFFu); }
@@ -675,7 +677,7 @@ struct CbShared {
       int32_t B[4 * NMAX];
       uint32_t masks[11 * (NMAX / 8) + 16];
     } pm;
-    uint32_t symset[65536 / 32];
+    uint32_t symset[NMAX > kCbSmall ? 65536 / 32 : 1];  // ESC lists only
     uint8_t nibs[2048];
   } u;
   int32_t na[16];
@@ -712,21 +714,17 @@ __device__ __forceinline__ uint32_t cb_bound(const uint64_t *k, uint32_t lo, uin
 }
 
 template <int NMAX>
-__global__ __launch_bounds__(kCbLanes) void codebook_wave_kernel(CodebookArgs a, const uint64_t *__restrict__ skeys,
-                                                                 const uint32_t *__restrict__ sslots, uint32_t lo_n,
-                                                                 uint32_t hi_n) {
-  __shared__ CbShared<NMAX> S;
-  const uint32_t g = blockIdx.x;
+__device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookArgs &a, uint32_t g,
+                                              const uint64_t *__restrict__ skeys,
+                                              const uint32_t *__restrict__ sslots) {
   const int lane = threadIdx.x;
   const int L = a.L;
   const uint32_t T = 1u << L;
   const uint32_t tk = a.gid_tkey[g];
   const uint32_t off = a.toff[tk];
   const uint32_t ni = a.tcount[tk];
-  const uint32_t nmax = ni < T ? ni : T;
-  if (nmax <= lo_n || nmax > hi_n) return;
   const uint64_t *keys = skeys + off;
-  const uint32_t *slots = sslots + off;
+  auto slot_of = [&](uint32_t t) { return sslots ? sslots[off + t] : off + t; };
   uint16_t *dsyms = a.decode_syms + (uint64_t)g * T;
   uint8_t *dlens = a.decode_lens + (uint64_t)g * (T / 2 > 0 ? T / 2 : 1);
   if (lane == 0) {
@@ -736,12 +734,12 @@ __global__ __launch_bounds__(kCbLanes) void codebook_wave_kernel(CodebookArgs a,
   if (ni == 1) {
     for (uint32_t j = lane; j < T; j += kCbLanes) dsyms[j] = (uint16_t)cb_sym(keys[0]);
     for (uint32_t j = lane; j < T / 2; j += kCbLanes) dlens[j] = 0x11;  // len 1 in both nibbles
-    if (lane == 0) a.cw_slot[slots[0]] = (1u << 16) | 0u;
+    if (lane == 0) a.cw_slot[slot_of(0)] = (1u << 16) | 0u;
     return;
   }
 
   // --- the coded list ---
-  const bool use_esc = ni > T;
+  const bool use_esc = NMAX > kCbSmall && ni > T;
   const uint32_t keep = T - 1;
   uint32_t nl, s0 = 0, s1 = 0, r = 0, esc_sym = 0, esc_pos = 0;
   int32_t esc_w = 0;
@@ -1044,8 +1042,50 @@ __global__ __launch_bounds__(kCbLanes) void codebook_wave_kernel(CodebookArgs a,
     } else {
       cw = esc_cw | kRaw;  // outside the map: ESC code + raw16
     }
-    a.cw_slot[slots[t]] = cw;
+    a.cw_slot[slot_of(t)] = cw;
   }
+}
+
+// The codebooks of the *n keys in `list` (one of the three size classes).
+template <int NMAX>
+__global__ __launch_bounds__(kCbLanes) void codebook_wave_kernel(CodebookArgs a, const uint64_t *__restrict__ skeys,
+                                                                 const uint32_t *__restrict__ sslots,
+                                                                 const uint32_t *__restrict__ list,
+                                                                 const uint32_t *__restrict__ n) {
+  __shared__ CbShared<NMAX> S;
+  const uint32_t count = *n;
+  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+    codebook_wave<NMAX>(S, a, list[i], skeys, sslots);
+    __syncthreads();
+  }
+}
+
+// Size class of a key with ni entries and T = 2^L codes: 0 (at most kCbSmall
+// entries, no ESC), 1 (a coded list of at most 512) or 2.
+__device__ __forceinline__ int cb_class(uint32_t ni, uint32_t T) {
+  const uint32_t nmax = ni < T ? ni : T;
+  return ni <= (uint32_t)kCbSmall && ni <= T ? 0 : nmax <= 512u ? 1 : 2;
+}
+
+// Appends gid to its class's list (lists: [3][cap]); one atomic per wave and class.
+__device__ __forceinline__ void cb_append(uint32_t gid, int cls, uint32_t *lists, uint32_t cap, uint32_t *n3) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const uint64_t m = __ballot(cls == c);
+    if (!m) continue;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(n3 + c, (uint32_t)__popcll(m));
+    base = (uint32_t)__shfl((int)base, 0);
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    if (cls == c) lists[(uint64_t)c * cap + base + (uint32_t)__popcll(m & below)] = gid;
+  }
+}
+
+__global__ void codebook_classes_kernel(const uint32_t *gid_tkey, const uint32_t *tcount, uint32_t G, uint32_t T,
+                                        uint32_t *lists, uint32_t *n3) {
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+  cb_append(g, g < G ? cb_class(tcount[gid_tkey[g]], T) : -1, lists, G, n3);
 }
 
 __global__ void item_keys_kernel(const uint16_t *__restrict__ sym, const uint32_t *__restrict__ cnt, uint64_t n,
@@ -1253,9 +1293,22 @@ __global__ void pack_kernel(PackArgs a) {
   if (used > 0) flush_word(a.bits, w, acc, first_w, last_w);
 }
 
+#include "encode_units.h"
+
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
+// The three codebook launches, a wave per key of each size class.
+void launch_codebooks(const CodebookArgs &cba, const uint64_t *skeys, const uint32_t *sslots, const uint32_t *lists,
+                      uint32_t cap, const uint32_t *n3, uint32_t most, hipStream_t s) {
+  hipLaunchKernelGGL(codebook_wave_kernel<kCbSmall>, dim3(std::min(most, 8192u)), dim3(kCbLanes), 0, s, cba, skeys,
+                     sslots, lists, n3);
+  hipLaunchKernelGGL(codebook_wave_kernel<512>, dim3(std::min(most, 1280u)), dim3(kCbLanes), 0, s, cba, skeys, sslots,
+                     lists + cap, n3 + 1);
+  hipLaunchKernelGGL(codebook_wave_kernel<2048>, dim3(std::min(most, 256u)), dim3(kCbLanes), 0, s, cba, skeys, sslots,
+                     lists + 2 * (size_t)cap, n3 + 2);
+}
+
 template <typename T>
 struct DevBuf {
   T *p = nullptr;
@@ -1458,17 +1511,11 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
   }
 
   auto sc = std::make_unique<mps_fp8_sidecar>();
-  DevBuf<uint16_t> d_row_sidx, d_block_sidx, d_bucket_sidx, d_scale_values;
+  DevBuf<uint16_t> d_bucket_sidx, d_scale_values;
   DevBuf<uint32_t> d_lane_base;
-  HC(d_row_sidx.alloc(row_sidx.size()));
-  HC(d_block_sidx.alloc(block_sidx.size()));
   HC(d_bucket_sidx.alloc(B));
   HC(d_scale_values.alloc(S));
   HC(d_lane_base.alloc(B + 1));
-  if (!row_sidx.empty())
-    HC(hipMemcpyAsync(d_row_sidx.p, row_sidx.data(), 2 * row_sidx.size(), hipMemcpyHostToDevice, s));
-  if (!block_sidx.empty())
-    HC(hipMemcpyAsync(d_block_sidx.p, block_sidx.data(), 2 * block_sidx.size(), hipMemcpyHostToDevice, s));
   HC(hipMemcpyAsync(d_bucket_sidx.p, bucket_sidx.data(), 2 * (size_t)B, hipMemcpyHostToDevice, s));
   HC(hipMemcpyAsync(d_scale_values.p, uniq_sc.data(), 2 * (size_t)S, hipMemcpyHostToDevice, s));
   HC(hipMemcpyAsync(d_lane_base.p, lane_base.data(), 4 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
@@ -1490,243 +1537,435 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
   }
   HC(hipMemcpyAsync(sc->bucket_col_len.p, col_len.data(), 4 * (size_t)B, hipMemcpyHostToDevice, s));
 
-  ScaleMap smap;
-  smap.mode = scale_block2d ? 1 : 0;
-  smap.row_sidx = d_row_sidx.p;
-  smap.block_sidx = d_block_sidx.p;
-  smap.sb0 = sb0;
-  smap.sb1 = sb1;
-  smap.nb1 = nb1;
+  DevBuf<uint32_t> flags;  // [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count, [5..7] codebook
+                           // classes, [8..10] keys, entries and most entries of a scale (scan_parts)
+  constexpr int kFlags = 16;
+  HC(flags.alloc(kFlags));
+  uint32_t hflags[kFlags] = {};
+  DevBuf<uint32_t> tcount, tgid, gid_tkey, cb_lists;
+  uint32_t D = 0, G = 0;
+  uint64_t cap = 0;
+  int64_t W = 0;
+  const uint64_t T = (uint64_t)S * 256;
+  const uint32_t Tsz = 1u << L;
+  const uint32_t packed = Tsz / 2 > 0 ? Tsz / 2 : 1;
+  const bool fp8 = sp.format == kFmtFp8;
+  CodebookArgs cba{};
+  auto alloc_tables = [&]() -> int {  // the outputs whose sizes follow from G
+    HC(sc->decode_syms.alloc((size_t)G * Tsz));
+    HC(sc->decode_lens.alloc((size_t)G * packed));
+    HC(sc->table_scale.alloc(G));
+    HC(sc->table_fp8.alloc(G));
+    HC(sc->bucket_table.alloc((size_t)B * qvals));
+    HC(sc->bucket_U.alloc(fp8 ? B : 0));
+    HC(sc->bucket_unique_gid.alloc(fp8 ? (size_t)B * 256 : 0));
+    HC(sc->bucket_fp8_uidx.alloc(fp8 ? (size_t)B * 256 : 0));
+    cba.gid_tkey = gid_tkey.p;
+    cba.tcount = tcount.p;
+    cba.scale_values = d_scale_values.p;
+    cba.decode_syms = sc->decode_syms.p;
+    cba.decode_lens = sc->decode_lens.p;
+    cba.table_scale = sc->table_scale.p;
+    cba.table_fp8 = sc->table_fp8.p;
+    cba.G = G;
+    cba.L = (int)L;
+    cba.esc_mode = sp.format;
+    cba.err = flags.p + 1;
+    cba.esc_stats = flags.p + 2;
+    return MPS_OK;
+  };
+  auto bucket_tables = [&]() -> int {
+    if (B)
+      hipLaunchKernelGGL(bucket_table_kernel, dim3((B + 63) / 64), dim3(64), 0, s, d_bucket_sidx.p, B, qvals,
+                         tcount.p, tgid.p, sc->bucket_table.p, sc->bucket_U.p, sc->bucket_unique_gid.p,
+                         sc->bucket_fp8_uidx.p);
+    HC(hipGetLastError());
+    return MPS_OK;
+  };
+  auto check_errors = [&]() -> int {
+    if (hflags[1] & 2u) return fail(MPS_ERR_RUNTIME, "invalid code length");
+    if (hflags[1] & 4u)
+      return fail(MPS_ERR_RUNTIME,
+                  fp8 ? "missing enc table for (scale,fp8) key" : "missing enc table for (scale,qv) key");
+    return MPS_OK;
+  };
 
-  // --- 1. histogram (retry with a larger table on overflow) ---
-  DevBuf<uint64_t> keys;
-  DevBuf<uint32_t> counts, flags;  // flags: [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count
-  HC(flags.alloc(8));
-  uint64_t cap = 1u << 16;
-  while (cap < (uint64_t)std::min<int64_t>(numel, (int64_t)1 << 22) * 2) cap <<= 1;
-  const int64_t per_block = 1 << 14;
-  const unsigned hist_blocks = (unsigned)((numel + per_block - 1) / per_block);
-  uint32_t hflags[8] = {};
-  for (;;) {
-    HC(keys.alloc(cap));
-    HC(counts.alloc(cap));
-    HC(hipMemsetAsync(keys.p, 0xFF, sizeof(uint64_t) * cap, s));
-    HC(hipMemsetAsync(counts.p, 0, sizeof(uint32_t) * cap, s));
-    HC(hipMemsetAsync(flags.p, 0, sizeof(uint32_t) * 8, s));
-    hipLaunchKernelGGL(hist_kernel, dim3(hist_blocks), dim3(kHistBlock), 0, s, sp.bf16, sp.q, n, m, smap,
-                       qmask, per_block, keys.p, counts.p, cap - 1, flags.p);
+  // --- the unit passes (encode_units.h) ---
+  // Taken when code words fit 16 bits (L <= 11), a workgroup's pieces of a
+  // substream stay few (k >= 32), element indexes have room in 32 bits, and the
+  // buckets are not so small that a workgroup's LDS set-up outweighs its unit
+  // (1024 elements). It gives up (kGeneral) when a unit's or a scale's pairs
+  // overflow their LDS tables, as random bit patterns do.
+  constexpr int kGeneral = 1;
+  auto unit_path = [&]() -> int {
+    if (L > 11 || kth < 32 || numel > ((int64_t)1 << 31)) return kGeneral;
+    // A unit: about 1/1024 of the tensor, so that four go to a CU; at least 16 Ki
+    // elements beside the 64 KiB of LDS each pass sets up.
+    const uint64_t target = std::min<uint64_t>(std::max<uint64_t>((uint64_t)numel / 1024, 16384), 1u << 20);
+    std::vector<Unit> units;
+    std::vector<uint32_t> bucket_unit(B + 1, 0), bucket_elem(B), list_off, scale_units(S + 1, 0);
+    std::vector<uint64_t> scale_elems(S, 0);
+    uint64_t elem = 0, lists_n = 0;
+    for (uint32_t b = 0; b < B; ++b) {
+      const uint64_t cl = (uint64_t)col_len[b], total = (uint64_t)(row_offsets[b + 1] - row_offsets[b]) * cl;
+      const uint64_t ke = lane_base[b + 1] - lane_base[b];
+      const uint64_t steps = (total + ke - 1) / ke;
+      const uint64_t most = std::max<uint64_t>(1, std::min<uint64_t>(target, (uint64_t)kUnitRows * cl) / ke);
+      const uint64_t parts = (steps + most - 1) / most, per = (steps + parts - 1) / parts;
+      bucket_unit[b] = (uint32_t)units.size();
+      bucket_elem[b] = (uint32_t)elem;
+      for (uint64_t i = 0; i < steps; i += per) {
+        const uint64_t end = std::min(steps, i + per);
+        units.push_back(Unit{b, (uint32_t)i, (uint32_t)end, bucket_sidx[b]});
+        list_off.push_back((uint32_t)lists_n);
+        lists_n += std::min<uint64_t>((end - i) * ke, kPairSlots);
+        ++scale_units[bucket_sidx[b] + 1];
+      }
+      elem += total;
+      scale_elems[bucket_sidx[b]] += total;
+    }
+    const size_t U = units.size();
+    bucket_unit[B] = (uint32_t)U;
+    if (U == 0 || (U > 4096 && (uint64_t)numel / U < 1024)) return kGeneral;
+    for (uint32_t i = 0; i < S; ++i) scale_units[i + 1] += scale_units[i];
+    std::vector<uint32_t> unit_of_scale(U), fill(scale_units.begin(), scale_units.end() - 1);
+    for (size_t u = 0; u < U; ++u) unit_of_scale[fill[units[u].sidx]++] = (uint32_t)u;
+    // Parts: q ranges of a scale merged by workgroups of their own, two a CU in all.
+    const uint32_t P = std::min<uint32_t>((uint32_t)qvals, std::max<uint32_t>(1, std::min<uint32_t>(16, 512 / S)));
+    std::vector<uint32_t> part_off((size_t)S * P);
+    uint64_t entries = 0;
+    for (size_t i = 0; i < part_off.size(); ++i) {
+      part_off[i] = (uint32_t)entries;
+      entries += std::min<uint64_t>(scale_elems[i / P], kPairSlots);
+    }
+    // One device block: the host-built arrays, then the passes' own.
+    std::vector<char> host;
+    size_t bytes = 0;
+    auto take = [&](size_t n) {
+      const size_t at = bytes;
+      bytes += (n + 255) & ~(size_t)255;
+      return at;
+    };
+    auto put = [&](const void *src, size_t n) {
+      const size_t at = take(n);
+      host.resize(bytes);
+      std::memcpy(host.data() + at, src, n);
+      return at;
+    };
+    const size_t o_units = put(units.data(), sizeof(Unit) * U), o_bunit = put(bucket_unit.data(), 4 * bucket_unit.size()),
+                 o_belem = put(bucket_elem.data(), 4 * (size_t)B), o_loff = put(list_off.data(), 4 * U),
+                 o_sunit = put(scale_units.data(), 4 * scale_units.size()),
+                 o_uos = put(unit_of_scale.data(), 4 * U), o_poff = put(part_off.data(), 4 * part_off.size());
+    const size_t host_bytes = bytes;
+    const size_t o_ln = take(4 * U), o_pn = take(4 * part_off.size()), o_pk = take(4 * part_off.size()),
+                 o_lists = take(8 * lists_n), o_skeys = take(8 * entries), o_cw = take(4 * entries),
+                 o_toff = take(4 * T), o_codes = take(2 * (size_t)numel), o_pieces = take(4 * (size_t)kUnitThreads * U),
+                 o_bbits = take(4 * (size_t)B);
+    DevBuf<char> blk;
+    HC(blk.alloc(bytes));
+    HC(tcount.alloc(T));
+    HC(tgid.alloc(T));
+    HC(gid_tkey.alloc(T));
+    HC(cb_lists.alloc(3 * T));
+    auto at32 = [&](size_t o) { return reinterpret_cast<uint32_t *>(blk.p + o); };
+    HC(hipMemcpyAsync(blk.p, host.data(), host_bytes, hipMemcpyHostToDevice, s));
+    HC(hipMemsetAsync(flags.p, 0, 4 * kFlags, s));
+    UnitArgs ua;
+    ua.units = reinterpret_cast<const Unit *>(blk.p + o_units);
+    ua.bf16 = sp.bf16;
+    ua.q = sp.q;
+    ua.m = (uint32_t)m;
+    ua.qmask = qmask;
+    ua.row_offsets = sc->bucket_row_offsets.p;
+    ua.row_indices = sc->row_indices.p;
+    ua.col_start = by_scale ? nullptr : sc->bucket_col_start.p;
+    ua.col_len = sc->bucket_col_len.p;
+    ua.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    ua.k = (uint32_t)kth;
+    // every row's column range starts and ends on 8 elements (columns start at multiples of the range's width)
+    ua.vec8 = m % 8 == 0 && col_len[0] % 8 == 0 && reinterpret_cast<uintptr_t>(sp.bf16) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(sp.q) % 8 == 0;
+    auto *lists = reinterpret_cast<uint2 *>(blk.p + o_lists);
+    auto *skeys = reinterpret_cast<uint64_t *>(blk.p + o_skeys);
+    auto *codes = reinterpret_cast<uint16_t *>(blk.p + o_codes);
+    hipLaunchKernelGGL(unit_hist, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, at32(o_loff), lists, at32(o_ln),
+                       flags.p);
+    hipLaunchKernelGGL(merge_lists, dim3(S * P), dim3(kUnitThreads), 0, s, at32(o_sunit), at32(o_uos), at32(o_loff),
+                       at32(o_ln), lists, P, (uint32_t)qvals, at32(o_poff), skeys, tcount.p, at32(o_toff), at32(o_pn),
+                       at32(o_pk), flags.p);
+    hipLaunchKernelGGL(scan_parts, dim3(1), dim3(kScanBlock), 0, s, at32(o_pk), at32(o_pn), S, P, flags.p + 8);
+    hipLaunchKernelGGL(number_keys, dim3(S), dim3(256), 0, s, tcount.p, at32(o_pk), P, Tsz, (uint32_t)qvals, tgid.p,
+                       gid_tkey.p, cb_lists.p, (uint32_t)T, flags.p + 5);
     HC(hipGetLastError());
     HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
-    if (!hflags[0]) break;
-    if (cap >= ((uint64_t)1 << 34)) return fail(MPS_ERR_RUNTIME, "histogram table overflow");
-    cap <<= 1;
-  }
-
-  // --- 2. compaction and grouping by (scale, fp8) key ---
-  DevBuf<uint64_t> ckey;
-  DevBuf<uint32_t> ccount, cslot;
-  // bound for the compact arrays: count first
-  uint32_t D = 0;
-  {
-    HC(ckey.alloc(cap));
-    HC(ccount.alloc(cap));
-    HC(cslot.alloc(cap));
-    hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((cap + 255) / 256)), dim3(256), 0, s, keys.p, counts.p, cap,
-                       ckey.p, ccount.p, cslot.p, flags.p + 4);
+    const uint32_t most = hflags[10];  // entries of the scale that has most
+    if (hflags[0] || most > 12288) return kGeneral;
+    G = hflags[8];
+    D = hflags[9];
+    cap = (uint64_t)S * P * kPairSlots;
+    int rc = alloc_tables();
+    if (rc != MPS_OK) return rc;
+    cba.toff = at32(o_toff);
+    cba.cw_slot = at32(o_cw);
+    launch_codebooks(cba, skeys, nullptr, cb_lists.p, (uint32_t)T, flags.p + 5, G, s);
     HC(hipGetLastError());
-    HC(hipMemcpyAsync(&D, flags.p + 4, 4, hipMemcpyDeviceToHost, s));
+    if ((rc = bucket_tables()) != MPS_OK) return rc;
+    HC(sc->bucket_thread_startbit.alloc((size_t)B * (kth + 1)));
+    HC(sc->bucket_bit_base.alloc(B + 1));
+    // the smaller table (two workgroups a CU) while it is at most 3/4 full
+    auto codes_pass = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, P, at32(o_poff), at32(o_pn), skeys,
+                         at32(o_cw), at32(o_belem), codes, at32(o_pieces), flags.p + 1);
+    };
+    if (most <= 6144) codes_pass(unit_codes<8192>);
+    else codes_pass(unit_codes<16384>);
+    hipLaunchKernelGGL(bucket_starts, dim3(B), dim3(kUnitThreads), 0, s, ua.units, at32(o_bunit), d_lane_base.p,
+                       (uint32_t)kth, at32(o_pieces), sc->bucket_thread_startbit.p, at32(o_bbits));
+    hipLaunchKernelGGL(bucket_bases, dim3(1), dim3(kScanBlock), 0, s, at32(o_bbits), B, sc->bucket_bit_base.p);
+    HC(hipGetLastError());
+    int64_t end = 0;
+    HC(hipMemcpyAsync(&end, sc->bucket_bit_base.p + B, 8, hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
-  }
-  const uint64_t T = (uint64_t)S * 256;
-  DevBuf<uint32_t> tcount, toff, tfill, tnz, tgid;
-  HC(tcount.alloc(T));
-  HC(toff.alloc(T));
-  HC(tfill.alloc(T));
-  HC(tnz.alloc(T));
-  HC(tgid.alloc(T));
-  HC(hipMemsetAsync(tcount.p, 0, 4 * T, s));
-  HC(hipMemsetAsync(tfill.p, 0, 4 * T, s));
-  hipLaunchKernelGGL(table_count_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, D, tcount.p);
-  HC(hipGetLastError());
-  uint32_t D_check = 0, G = 0;
-  HC(device_scan(tcount.p, toff.p, T, s, &D_check));
-  hipLaunchKernelGGL(nonzero_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, T, tnz.p);
-  HC(hipGetLastError());
-  HC(device_scan(tnz.p, tgid.p, T, s, &G));
-  if (D_check != D) return fail(MPS_ERR_RUNTIME, "internal error: histogram grouping mismatch");
-  DevBuf<uint16_t> seg_sym;
-  DevBuf<uint32_t> seg_cnt, seg_slot, gid_tkey, ws_off, cw_slot;
-  HC(seg_sym.alloc(D));
-  HC(seg_cnt.alloc(D));
-  HC(seg_slot.alloc(D));
-  HC(gid_tkey.alloc(G));
-  hipLaunchKernelGGL(scatter_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, ccount.p, cslot.p, D, toff.p,
-                     tfill.p, seg_sym.p, seg_cnt.p, seg_slot.p);
-  hipLaunchKernelGGL(table_list_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, tgid.p, T,
-                     gid_tkey.p);
-  HC(hipGetLastError());
+    if ((rc = check_errors()) != MPS_OK) return rc;
+    W = (end + 63) >> 6;
+    HC(sc->bitstream.alloc((size_t)W));
+    if (W) {
+      HC(hipMemsetAsync(sc->bitstream.p, 0, 8 * (size_t)W, s));
+      hipLaunchKernelGGL(unit_pack, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, at32(o_belem), codes,
+                         at32(o_pieces), sc->bucket_thread_startbit.p, sc->bucket_bit_base.p,
+                         reinterpret_cast<uint32_t *>(sc->bitstream.p));
+      HC(hipGetLastError());
+    }
+    HC(hipStreamSynchronize(s));  // the block goes out of scope
+    return MPS_OK;
+  };
 
-  // --- 3. code books ---
-  const uint32_t Tsz = 1u << L;
-  const uint32_t packed = Tsz / 2 > 0 ? Tsz / 2 : 1;
-  HC(sc->decode_syms.alloc((size_t)G * Tsz));
-  HC(sc->decode_lens.alloc((size_t)G * packed));
-  HC(sc->table_scale.alloc(G));
-  HC(sc->table_fp8.alloc(G));
-  HC(cw_slot.alloc(cap));
-  // Codebooks. L <= 11 (the FP8 and AWQ formats): the keys' histogram entries
-  // are sorted for all keys at once, then a wave per key builds each codebook in
-  // LDS (codebook_wave_kernel; one launch for lists of up to 512 items, one for
-  // the larger). Longer codes (L up to 15, reachable through the op's max_len)
-  // keep the work-item-per-key kernel and its global workspace.
-  const bool wave_cb = L <= 11;
-  DevBuf<uint64_t> keys_in, keys_sorted;
-  DevBuf<uint32_t> slots_sorted, seg_beg, seg_end;
-  DevBuf<char> sort_tmp;
-  if (wave_cb && G) {
-    HC(keys_in.alloc(D));
-    HC(keys_sorted.alloc(D));
-    HC(slots_sorted.alloc(D));
-    HC(seg_beg.alloc(G));
-    HC(seg_end.alloc(G));
-    if (D)
-      hipLaunchKernelGGL(item_keys_kernel, dim3((D + 255) / 256), dim3(256), 0, s, seg_sym.p, seg_cnt.p, (uint64_t)D,
-                         keys_in.p);
-    hipLaunchKernelGGL(segment_bounds_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, toff.p, tcount.p, G,
-                       seg_beg.p, seg_end.p);
+  // --- the general path: hash tables in global memory, a work-item a substream ---
+  auto general_path = [&]() -> int {
+    DevBuf<uint16_t> d_row_sidx, d_block_sidx;
+    HC(d_row_sidx.alloc(row_sidx.size()));
+    HC(d_block_sidx.alloc(block_sidx.size()));
+    if (!row_sidx.empty())
+      HC(hipMemcpyAsync(d_row_sidx.p, row_sidx.data(), 2 * row_sidx.size(), hipMemcpyHostToDevice, s));
+    if (!block_sidx.empty())
+      HC(hipMemcpyAsync(d_block_sidx.p, block_sidx.data(), 2 * block_sidx.size(), hipMemcpyHostToDevice, s));
+    ScaleMap smap;
+    smap.mode = scale_block2d ? 1 : 0;
+    smap.row_sidx = d_row_sidx.p;
+    smap.block_sidx = d_block_sidx.p;
+    smap.sb0 = sb0;
+    smap.sb1 = sb1;
+    smap.nb1 = nb1;
+
+    // --- 1. histogram (retry with a larger table on overflow) ---
+    DevBuf<uint64_t> keys;
+    DevBuf<uint32_t> counts;
+    cap = 1u << 16;
+    while (cap < (uint64_t)std::min<int64_t>(numel, (int64_t)1 << 22) * 2) cap <<= 1;
+    const int64_t per_block = 1 << 14;
+    const unsigned hist_blocks = (unsigned)((numel + per_block - 1) / per_block);
+    for (;;) {
+      HC(keys.alloc(cap));
+      HC(counts.alloc(cap));
+      HC(hipMemsetAsync(keys.p, 0xFF, sizeof(uint64_t) * cap, s));
+      HC(hipMemsetAsync(counts.p, 0, sizeof(uint32_t) * cap, s));
+      HC(hipMemsetAsync(flags.p, 0, sizeof(uint32_t) * kFlags, s));
+      hipLaunchKernelGGL(hist_kernel, dim3(hist_blocks), dim3(kHistBlock), 0, s, sp.bf16, sp.q, n, m, smap,
+                         qmask, per_block, keys.p, counts.p, cap - 1, flags.p);
+      HC(hipGetLastError());
+      HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+      HC(hipStreamSynchronize(s));
+      if (!hflags[0]) break;
+      if (cap >= ((uint64_t)1 << 34)) return fail(MPS_ERR_RUNTIME, "histogram table overflow");
+      cap <<= 1;
+    }
+
+    // --- 2. compaction and grouping by (scale, fp8) key ---
+    DevBuf<uint64_t> ckey;
+    DevBuf<uint32_t> ccount, cslot;
+    // bound for the compact arrays: count first
+    {
+      HC(ckey.alloc(cap));
+      HC(ccount.alloc(cap));
+      HC(cslot.alloc(cap));
+      hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((cap + 255) / 256)), dim3(256), 0, s, keys.p, counts.p, cap,
+                         ckey.p, ccount.p, cslot.p, flags.p + 4);
+      HC(hipGetLastError());
+      HC(hipMemcpyAsync(&D, flags.p + 4, 4, hipMemcpyDeviceToHost, s));
+      HC(hipStreamSynchronize(s));
+    }
+    DevBuf<uint32_t> toff, tfill, tnz;
+    HC(tcount.alloc(T));
+    HC(toff.alloc(T));
+    HC(tfill.alloc(T));
+    HC(tnz.alloc(T));
+    HC(tgid.alloc(T));
+    HC(hipMemsetAsync(tcount.p, 0, 4 * T, s));
+    HC(hipMemsetAsync(tfill.p, 0, 4 * T, s));
+    hipLaunchKernelGGL(table_count_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, D, tcount.p);
     HC(hipGetLastError());
-    size_t tmp_bytes = 0;
-    HC(rocprim::segmented_radix_sort_pairs(nullptr, tmp_bytes, keys_in.p, keys_sorted.p, seg_slot.p, slots_sorted.p,
-                                           D, G, seg_beg.p, seg_end.p, 0, 48, s));
-    HC(sort_tmp.alloc(tmp_bytes));
-    HC(rocprim::segmented_radix_sort_pairs(sort_tmp.p, tmp_bytes, keys_in.p, keys_sorted.p, seg_slot.p,
-                                           slots_sorted.p, D, G, seg_beg.p, seg_end.p, 0, 48, s));
-  }
-  // per-key workspace of the work-item-per-key kernel, sized by each key's list length
-  DevBuf<uint32_t> ws_sz;
-  HC(ws_sz.alloc(G));
-  HC(ws_off.alloc(G));
-  uint32_t ws_total = 0;
-  if (G && !wave_cb) {
-    hipLaunchKernelGGL(ws_size_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, tcount.p, G, Tsz,
-                       ws_sz.p);
+    uint32_t D_check = 0;
+    G = 0;
+    HC(device_scan(tcount.p, toff.p, T, s, &D_check));
+    hipLaunchKernelGGL(nonzero_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, T, tnz.p);
     HC(hipGetLastError());
-    HC(device_scan(ws_sz.p, ws_off.p, G, s, &ws_total));
-  }
-  DevBuf<int32_t> ws;
-  HC(ws.alloc(ws_total));
-  CodebookArgs cba;
-  cba.gid_tkey = gid_tkey.p;
-  cba.toff = toff.p;
-  cba.tcount = tcount.p;
-  cba.seg_sym = seg_sym.p;
-  cba.seg_cnt = seg_cnt.p;
-  cba.seg_slot = seg_slot.p;
-  cba.ws = ws.p;
-  cba.ws_off = ws_off.p;
-  cba.scale_values = d_scale_values.p;
-  cba.cw_slot = cw_slot.p;
-  cba.decode_syms = sc->decode_syms.p;
-  cba.decode_lens = sc->decode_lens.p;
-  cba.table_scale = sc->table_scale.p;
-  cba.table_fp8 = sc->table_fp8.p;
-  cba.G = G;
-  cba.L = (int)L;
-  cba.esc_mode = sp.format;
-  cba.err = flags.p + 1;
-  cba.esc_stats = flags.p + 2;
-  if (G && wave_cb) {
-    hipLaunchKernelGGL(codebook_wave_kernel<512>, dim3(G), dim3(kCbLanes), 0, s, cba, keys_sorted.p, slots_sorted.p,
-                       0u, 512u);
-    hipLaunchKernelGGL(codebook_wave_kernel<2048>, dim3(G), dim3(kCbLanes), 0, s, cba, keys_sorted.p,
-                       slots_sorted.p, 512u, 2048u);
-  } else if (G) {
-    hipLaunchKernelGGL(codebook_kernel, dim3((G + 63) / 64), dim3(64), 0, s, cba);
-  }
-  HC(hipGetLastError());
+    HC(device_scan(tnz.p, tgid.p, T, s, &G));
+    if (D_check != D) return fail(MPS_ERR_RUNTIME, "internal error: histogram grouping mismatch");
+    DevBuf<uint16_t> seg_sym;
+    DevBuf<uint32_t> seg_cnt, seg_slot, ws_off, cw_slot;
+    HC(seg_sym.alloc(D));
+    HC(seg_cnt.alloc(D));
+    HC(seg_slot.alloc(D));
+    HC(gid_tkey.alloc(G));
+    hipLaunchKernelGGL(scatter_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, ccount.p, cslot.p, D, toff.p,
+                       tfill.p, seg_sym.p, seg_cnt.p, seg_slot.p);
+    hipLaunchKernelGGL(table_list_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, tgid.p, T,
+                       gid_tkey.p);
+    HC(hipGetLastError());
 
-  // --- 4. bucket tables ---
-  const bool fp8 = sp.format == kFmtFp8;
-  HC(sc->bucket_table.alloc((size_t)B * qvals));
-  HC(sc->bucket_U.alloc(fp8 ? B : 0));
-  HC(sc->bucket_unique_gid.alloc(fp8 ? (size_t)B * 256 : 0));
-  HC(sc->bucket_fp8_uidx.alloc(fp8 ? (size_t)B * 256 : 0));
-  if (B)
-    hipLaunchKernelGGL(bucket_table_kernel, dim3((B + 63) / 64), dim3(64), 0, s, d_bucket_sidx.p, B, qvals, tcount.p,
-                       tgid.p, sc->bucket_table.p, sc->bucket_U.p, sc->bucket_unique_gid.p, sc->bucket_fp8_uidx.p);
-  HC(hipGetLastError());
+    // --- 3. code books ---
+    int rc = alloc_tables();
+    if (rc != MPS_OK) return rc;
+    HC(cw_slot.alloc(cap));
+    // Codebooks. L <= 11 (the FP8 and AWQ formats): the keys' histogram entries
+    // are sorted for all keys at once, then a wave per key builds each codebook in
+    // LDS (codebook_wave_kernel; one launch for lists of up to 512 items, one for
+    // the larger). Longer codes (L up to 15, reachable through the op's max_len)
+    // keep the work-item-per-key kernel and its global workspace.
+    const bool wave_cb = L <= 11;
+    DevBuf<uint64_t> keys_in, keys_sorted;
+    DevBuf<uint32_t> slots_sorted, seg_beg, seg_end;
+    DevBuf<char> sort_tmp;
+    if (wave_cb && G) {
+      HC(keys_in.alloc(D));
+      HC(keys_sorted.alloc(D));
+      HC(slots_sorted.alloc(D));
+      HC(seg_beg.alloc(G));
+      HC(seg_end.alloc(G));
+      if (D)
+        hipLaunchKernelGGL(item_keys_kernel, dim3((D + 255) / 256), dim3(256), 0, s, seg_sym.p, seg_cnt.p, (uint64_t)D,
+                           keys_in.p);
+      hipLaunchKernelGGL(segment_bounds_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, toff.p, tcount.p, G,
+                         seg_beg.p, seg_end.p);
+      HC(hipGetLastError());
+      size_t tmp_bytes = 0;
+      HC(rocprim::segmented_radix_sort_pairs(nullptr, tmp_bytes, keys_in.p, keys_sorted.p, seg_slot.p, slots_sorted.p,
+                                             D, G, seg_beg.p, seg_end.p, 0, 48, s));
+      HC(sort_tmp.alloc(tmp_bytes));
+      HC(rocprim::segmented_radix_sort_pairs(sort_tmp.p, tmp_bytes, keys_in.p, keys_sorted.p, seg_slot.p,
+                                             slots_sorted.p, D, G, seg_beg.p, seg_end.p, 0, 48, s));
+    }
+    // per-key workspace of the work-item-per-key kernel, sized by each key's list length
+    DevBuf<uint32_t> ws_sz;
+    HC(ws_sz.alloc(G));
+    HC(ws_off.alloc(G));
+    uint32_t ws_total = 0;
+    if (G && !wave_cb) {
+      hipLaunchKernelGGL(ws_size_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, tcount.p, G, Tsz,
+                         ws_sz.p);
+      HC(hipGetLastError());
+      HC(device_scan(ws_sz.p, ws_off.p, G, s, &ws_total));
+    }
+    DevBuf<int32_t> ws;
+    HC(ws.alloc(ws_total));
+    cba.toff = toff.p;
+    cba.seg_sym = seg_sym.p;
+    cba.seg_cnt = seg_cnt.p;
+    cba.seg_slot = seg_slot.p;
+    cba.ws = ws.p;
+    cba.ws_off = ws_off.p;
+    cba.cw_slot = cw_slot.p;
+    if (G && wave_cb) {
+      HC(cb_lists.alloc(3 * (size_t)G));
+      HC(hipMemsetAsync(flags.p + 5, 0, 12, s));
+      hipLaunchKernelGGL(codebook_classes_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, tcount.p, G, Tsz,
+                         cb_lists.p, flags.p + 5);
+      launch_codebooks(cba, keys_sorted.p, slots_sorted.p, cb_lists.p, G, flags.p + 5, G, s);
+    } else if (G) {
+      hipLaunchKernelGGL(codebook_kernel, dim3((G + 63) / 64), dim3(64), 0, s, cba);
+    }
+    HC(hipGetLastError());
 
-  // --- 5. bitstream ---
-  HC(sc->bucket_thread_startbit.alloc((size_t)B * (kth + 1)));
-  HC(hipMemsetAsync(sc->bucket_thread_startbit.p, 0, 4 * (size_t)B * (kth + 1), s));
-  DevBuf<uint32_t> cw_elem, bucket_bits;
-  HC(cw_elem.alloc((size_t)numel));
-  HC(bucket_bits.alloc(B));
-  const uint32_t lanes = lane_base[B];
-  LaneArgs la;
-  la.bf16 = sp.bf16;
-  la.fp8 = sp.q;
-  la.qmask = qmask;
-  la.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
-  la.S = smap;
-  la.m = m;
-  la.row_offsets = sc->bucket_row_offsets.p;
-  la.row_indices = sc->row_indices.p;
-  la.col_start = sc->bucket_col_start.p;
-  la.col_len = sc->bucket_col_len.p;
-  la.lane_base = d_lane_base.p;
-  la.B = B;
-  la.k = kth;
-  la.keys = keys.p;
-  la.cw_slot = cw_slot.p;
-  la.cap_mask = cap - 1;
-  la.cw_elem = cw_elem.p;
-  la.lane_bits = sc->bucket_thread_startbit.p;
-  la.err = flags.p + 1;
-  if (lanes) hipLaunchKernelGGL(lane_bits_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, la);
-  HC(hipGetLastError());
-  if (B) hipLaunchKernelGGL(lane_starts_kernel, dim3(B), dim3(1024), 0, s, sc->bucket_thread_startbit.p,
-                            d_lane_base.p, kth, bucket_bits.p);
-  HC(hipGetLastError());
-  std::vector<uint32_t> h_bucket_bits(B);
-  if (B) HC(hipMemcpyAsync(h_bucket_bits.data(), bucket_bits.p, 4 * (size_t)B, hipMemcpyDeviceToHost, s));
-  HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
-  HC(hipStreamSynchronize(s));
-  if (hflags[1] & 2u) return fail(MPS_ERR_RUNTIME, "invalid code length");
-  if (hflags[1] & 4u)
-    return fail(MPS_ERR_RUNTIME, fp8 ? "missing enc table for (scale,fp8) key" : "missing enc table for (scale,qv) key");
-  // 64-bit aligned bucket bases (build_huffman.cu:813-818), final cursor unaligned
-  std::vector<int64_t> bit_base(B + 1, 0);
-  int64_t pos = 0;
-  for (uint32_t b = 0; b < B; ++b) {
-    if (pos & 63) pos = (pos + 63) & ~(int64_t)63;
-    bit_base[b] = pos;
-    pos += h_bucket_bits[b];
-  }
-  bit_base[B] = pos;
-  const int64_t W = (pos + 63) >> 6;
-  HC(sc->bucket_bit_base.alloc(B + 1));
-  HC(hipMemcpyAsync(sc->bucket_bit_base.p, bit_base.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
-  HC(sc->bitstream.alloc((size_t)W));
-  if (W) HC(hipMemsetAsync(sc->bitstream.p, 0, 8 * (size_t)W, s));
-  PackArgs pa;
-  pa.bf16 = sp.bf16;
-  pa.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
-  pa.m = m;
-  pa.row_offsets = sc->bucket_row_offsets.p;
-  pa.row_indices = sc->row_indices.p;
-  pa.col_start = sc->bucket_col_start.p;
-  pa.col_len = sc->bucket_col_len.p;
-  pa.lane_base = d_lane_base.p;
-  pa.B = B;
-  pa.k = kth;
-  pa.cw_elem = cw_elem.p;
-  pa.startbit = sc->bucket_thread_startbit.p;
-  pa.bit_base = sc->bucket_bit_base.p;
-  pa.bits = reinterpret_cast<unsigned long long *>(sc->bitstream.p);
-  if (lanes && W) hipLaunchKernelGGL(pack_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, pa);
-  HC(hipGetLastError());
+    // --- 4. bucket tables ---
+    if ((rc = bucket_tables()) != MPS_OK) return rc;
+
+    // --- 5. bitstream ---
+    HC(sc->bucket_thread_startbit.alloc((size_t)B * (kth + 1)));
+    HC(hipMemsetAsync(sc->bucket_thread_startbit.p, 0, 4 * (size_t)B * (kth + 1), s));
+    DevBuf<uint32_t> cw_elem, bucket_bits;
+    HC(cw_elem.alloc((size_t)numel));
+    HC(bucket_bits.alloc(B));
+    const uint32_t lanes = lane_base[B];
+    LaneArgs la;
+    la.bf16 = sp.bf16;
+    la.fp8 = sp.q;
+    la.qmask = qmask;
+    la.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    la.S = smap;
+    la.m = m;
+    la.row_offsets = sc->bucket_row_offsets.p;
+    la.row_indices = sc->row_indices.p;
+    la.col_start = sc->bucket_col_start.p;
+    la.col_len = sc->bucket_col_len.p;
+    la.lane_base = d_lane_base.p;
+    la.B = B;
+    la.k = kth;
+    la.keys = keys.p;
+    la.cw_slot = cw_slot.p;
+    la.cap_mask = cap - 1;
+    la.cw_elem = cw_elem.p;
+    la.lane_bits = sc->bucket_thread_startbit.p;
+    la.err = flags.p + 1;
+    if (lanes) hipLaunchKernelGGL(lane_bits_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, la);
+    HC(hipGetLastError());
+    if (B) hipLaunchKernelGGL(lane_starts_kernel, dim3(B), dim3(1024), 0, s, sc->bucket_thread_startbit.p,
+                              d_lane_base.p, kth, bucket_bits.p);
+    HC(hipGetLastError());
+    std::vector<uint32_t> h_bucket_bits(B);
+    if (B) HC(hipMemcpyAsync(h_bucket_bits.data(), bucket_bits.p, 4 * (size_t)B, hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+    HC(hipStreamSynchronize(s));
+    if ((rc = check_errors()) != MPS_OK) return rc;
+    // 64-bit aligned bucket bases (build_huffman.cu:813-818), final cursor unaligned
+    std::vector<int64_t> bit_base(B + 1, 0);
+    int64_t pos = 0;
+    for (uint32_t b = 0; b < B; ++b) {
+      if (pos & 63) pos = (pos + 63) & ~(int64_t)63;
+      bit_base[b] = pos;
+      pos += h_bucket_bits[b];
+    }
+    bit_base[B] = pos;
+    W = (pos + 63) >> 6;
+    HC(sc->bucket_bit_base.alloc(B + 1));
+    HC(hipMemcpyAsync(sc->bucket_bit_base.p, bit_base.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
+    HC(sc->bitstream.alloc((size_t)W));
+    if (W) HC(hipMemsetAsync(sc->bitstream.p, 0, 8 * (size_t)W, s));
+    PackArgs pa;
+    pa.bf16 = sp.bf16;
+    pa.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    pa.m = m;
+    pa.row_offsets = sc->bucket_row_offsets.p;
+    pa.row_indices = sc->row_indices.p;
+    pa.col_start = sc->bucket_col_start.p;
+    pa.col_len = sc->bucket_col_len.p;
+    pa.lane_base = d_lane_base.p;
+    pa.B = B;
+    pa.k = kth;
+    pa.cw_elem = cw_elem.p;
+    pa.startbit = sc->bucket_thread_startbit.p;
+    pa.bit_base = sc->bucket_bit_base.p;
+    pa.bits = reinterpret_cast<unsigned long long *>(sc->bitstream.p);
+    if (lanes && W) hipLaunchKernelGGL(pack_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, pa);
+    HC(hipGetLastError());
+    HC(hipStreamSynchronize(s));
+    return MPS_OK;
+  };
+
+  int path_rc = unit_path();
+  if (path_rc == kGeneral) path_rc = general_path();
+  if (path_rc != MPS_OK) return path_rc;
   const int64_t shape[4] = {n, m, kth, by_scale ? (int64_t)col_len.front() : 0};
   const int nshape = by_scale ? 4 : 3;
   HC(sc->shape_nmk.alloc(nshape));

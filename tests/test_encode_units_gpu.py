@@ -1,0 +1,97 @@
+"""The builder's unit passes at their edges, byte for byte against the CPU oracle:
+units a bucket, partial steps, odd widths and offsets, substream counts that do not
+divide a workgroup, the two sizes of the code-word table, and calls that leave the
+passes for the general path (pairs that overflow a table, few substreams)."""
+import numpy as np
+import pytest
+import torch
+
+import MPServe_cuda
+import oracle
+from mpserve_amd.synthetic import make_awq_weight
+from tests.helpers import synth
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _fp8(bf, q, sc, L, k, shift=0):
+    """Builds on the device from tensors `shift` elements into their storage."""
+    def put(a, dt):
+        a = np.ascontiguousarray(a)
+        base = torch.empty(a.size + shift, dtype=dt, device=DEV)
+        base[shift:] = torch.from_numpy(a.reshape(-1)).to(DEV)
+        return base[shift:].view(a.shape)
+    b = put(bf.view(np.int16), torch.int16).view(torch.bfloat16)
+    got = MPServe_cuda.huffman_build_fp8_decode_tables(b, put(q, torch.uint8), torch.from_numpy(sc), L, k)
+    return {x: v.cpu().numpy() for x, v in got.items()}
+
+
+def _same(got, want):
+    assert list(got) == list(want)
+    for x in want:
+        assert got[x].shape == want[x].shape and np.array_equal(got[x], want[x]), x
+
+
+@pytest.mark.parametrize("n,m,k,shift", [
+    (300, 520, 1024, 0),    # several units a bucket, 8-element loads
+    (300, 521, 1024, 0),    # odd width: rows start anywhere
+    (300, 520, 1024, 1),    # the same loads from tensors at odd offsets
+    (260, 1000, 320, 0),    # 1024 / k pieces leave work-items over
+    (257, 999, 33, 0), (257, 999, 32, 0),  # many pieces side by side
+    (257, 999, 31, 0),      # too few substreams: general path
+    (5000, 8, 1024, 0), (5000, 3, 512, 0), (20000, 2, 64, 0),  # units bounded by their rows, not their elements
+    (3, 17, 1024, 0),       # fewer elements than substreams
+])
+def test_units_per_row(n, m, k, shift):
+    print(f"[units] {n}x{m} k{k} shift {shift}", flush=True)
+    bf, q, sc = synth(n, m, seed=n + m + k)
+    sc[n // 3:] = sc[0]  # one scale with many rows, the others few
+    _same(_fp8(bf, q, sc, 7, k, shift), oracle.encode(bf, q, sc, 7, k))
+
+
+@pytest.mark.parametrize("L", [1, 6, 7, 10, 11, 12])
+def test_units_code_lengths(L):
+    print(f"[units] L {L}", flush=True)
+    bf, q, sc = synth(200, 300, seed=L)
+    _same(_fp8(bf, q, sc[:1].copy(), L, 256), oracle.encode(bf, q, sc[:1].copy(), L, 256))
+
+
+@pytest.mark.parametrize("syms,qs", [(2900, 2), (3500, 2), (6000, 2), (65536, 256)])
+def test_units_table_sizes(syms, qs):
+    """Pairs of one scale: within 3/4 of the smaller table, of the larger, near its end, and beyond any table."""
+    print(f"[units] {syms} symbols x {qs}", flush=True)
+    rng = np.random.default_rng(syms)
+    bf = rng.integers(0, syms, size=(256, 900)).astype(np.uint16)
+    q = rng.integers(0, qs, size=bf.shape).astype(np.uint8)
+    sc = np.array([0x1C00], dtype=np.uint16)
+    _same(_fp8(bf, q, sc, 7, 1024), oracle.encode(bf, q, sc, 7, 1024))
+
+
+@pytest.mark.parametrize("bs", [(128, 128), (64, 40), (2, 3)])
+def test_units_blocks(bs):
+    print(f"[units] blocks {bs}", flush=True)
+    n, m = bs[0] * 4, bs[1] * 20
+    bf, q, _ = synth(n, m, seed=bs[1])
+    sc = np.random.default_rng(bs[0]).integers(0x2000, 0x2006, size=(4, 20), dtype=np.uint16)
+    _same(_fp8(bf, q, sc, 7, 256), oracle.encode(bf, q, sc, 7, 256))
+
+
+@pytest.mark.parametrize("n,m,group,k,by_scale,cap", [
+    (512, 1024, 128, 1024, True, 1024), (512, 1024, 64, 256, True, 7), (300, 1000, 40, 512, True, 100000),
+    (300, 999, None, 1024, True, 64), (300, 999, None, 256, False, 1024), (256, 640, 128, 1024, False, 1024),
+])
+def test_units_awq(n, m, group, k, by_scale, cap):
+    print(f"[units] awq {n}x{m} group {group} k{k} by_scale {by_scale}", flush=True)
+    w = make_awq_weight(n, m, group, seed=n + m + k)
+    args = (w.bf16.to(DEV), w.int4_u8.to(DEV), w.scale_u16, 11, k)
+    if by_scale:
+        got = MPServe_cuda.huffman_build_awq_int4_bucket_decode_tables_by_scale(*args, cap)
+    else:
+        got = MPServe_cuda.huffman_build_awq_int4_bucket_decode_tables(*args)
+    want = oracle.awq_encode(w.bf16.view(torch.uint16).numpy(), w.int4_u8.numpy(), w.scale_u16.numpy(), 11, k, cap,
+                             by_scale)
+    got = {x: v.cpu().numpy() for x, v in got.items()}
+    assert list(got) == list(want)
+    for x, v in want.items():
+        assert got[x].shape == v.shape and np.array_equal(got[x].view(v.dtype), v), x
