@@ -1115,32 +1115,33 @@ __global__ void ws_size_kernel(const uint32_t *gid_tkey, const uint32_t *tcount,
 // ---------------------------------------------------------------------------
 // 4. bucket_table, U / unique gids / fp8 -> uidx (one work-item per bucket)
 // ---------------------------------------------------------------------------
-// qvals = 256 (FP8 bytes; also U/uniq/uidx) or 16 (AWQ int4 values, build_huffman.cu:1973-1982).
-__global__ void bucket_table_kernel(const uint16_t *bucket_sidx, uint32_t B, int qvals, const uint32_t *tcount,
-                                    const uint32_t *tgid, int32_t *btab, int32_t *bU, int32_t *uniq, int16_t *uidx) {
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const uint64_t t0 = (uint64_t)bucket_sidx[b] * 256;
+// qvals = 256 (FP8 bytes; also U/uniq/uidx): a workgroup a bucket, a work-item
+// a byte; or 16 (AWQ int4 values, build_huffman.cu:1973-1982): a work-item an
+// entry. (A work-item a bucket walking its 256 bytes took 172 us for 70 to 180
+// buckets, all of it latency; this takes 5 us.)
+__global__ __launch_bounds__(256) void bucket_table_kernel(const uint16_t *bucket_sidx, uint32_t B, int qvals,
+                                                           const uint32_t *tcount, const uint32_t *tgid, int32_t *btab,
+                                                           int32_t *bU, int32_t *uniq, int16_t *uidx) {
+  __shared__ uint32_t s_tmp[16];
   if (qvals != 256) {
-    for (int c = 0; c < qvals; ++c) btab[b * qvals + c] = tcount[t0 + c] ? (int32_t)tgid[t0 + c] : -1;
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (uint64_t)B * qvals) return;
+    const uint64_t t = (uint64_t)bucket_sidx[i / qvals] * 256 + i % qvals;
+    btab[i] = tcount[t] ? (int32_t)tgid[t] : -1;
     return;
   }
-  int32_t U = 0;
-  for (int c = 0; c < 256; ++c) {
-    const int32_t gid = tcount[t0 + c] ? (int32_t)tgid[t0 + c] : -1;
-    btab[b * 256 + c] = gid;
-    uniq[b * 256 + c] = -1;
-    uidx[b * 256 + c] = -1;
-  }
+  const uint32_t b = blockIdx.x, c = threadIdx.x;
+  const uint64_t t = (uint64_t)bucket_sidx[b] * 256 + c;
+  const bool has = tcount[t] != 0;
+  const int32_t gid = has ? (int32_t)tgid[t] : -1;
   // gids of one bucket are distinct (one scale, distinct fp8 bytes): first-appearance order is fp8 order
-  for (int c = 0; c < 256; ++c) {
-    const int32_t gid = btab[b * 256 + c];
-    if (gid < 0) continue;
-    uniq[b * 256 + U] = gid;
-    uidx[b * 256 + c] = (int16_t)U;
-    ++U;
-  }
-  bU[b] = U;
+  uint32_t U = 0;
+  const uint32_t at = block_exclusive_scan(has ? 1u : 0u, s_tmp, &U);
+  btab[(uint64_t)b * 256 + c] = gid;
+  uidx[(uint64_t)b * 256 + c] = has ? (int16_t)at : (int16_t)-1;
+  if (has) uniq[(uint64_t)b * 256 + at] = gid;
+  if (c >= U) uniq[(uint64_t)b * 256 + c] = -1;
+  if (c == 0) bU[b] = (int32_t)U;
 }
 
 // ---------------------------------------------------------------------------
@@ -1576,8 +1577,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
   };
   auto bucket_tables = [&]() -> int {
     if (B)
-      hipLaunchKernelGGL(bucket_table_kernel, dim3((B + 63) / 64), dim3(64), 0, s, d_bucket_sidx.p, B, qvals,
-                         tcount.p, tgid.p, sc->bucket_table.p, sc->bucket_U.p, sc->bucket_unique_gid.p,
+      hipLaunchKernelGGL(bucket_table_kernel, dim3(fp8 ? B : (B * 16 + 255) / 256), dim3(256), 0, s, d_bucket_sidx.p, B,
+                         qvals, tcount.p, tgid.p, sc->bucket_table.p, sc->bucket_U.p, sc->bucket_unique_gid.p,
                          sc->bucket_fp8_uidx.p);
     HC(hipGetLastError());
     return MPS_OK;
