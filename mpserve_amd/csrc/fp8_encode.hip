@@ -1733,8 +1733,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     W = (end + 63) >> 6;
     HC(sc->bitstream.alloc((size_t)W));
     if (W) {
-      HC(hipMemsetAsync(sc->bitstream.p, 0, 8 * (size_t)W, s));
-      hipLaunchKernelGGL(unit_pack, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, at32(o_belem), codes,
+      hipLaunchKernelGGL(unit_pack, dim3((unsigned)(U + 7) / 8 * 8), dim3(kUnitThreads), 0, s, ua, (uint32_t)U,
+                         at32(o_belem), codes,
                          at32(o_pieces), sc->bucket_thread_startbit.p, sc->bucket_bit_base.p,
                          reinterpret_cast<uint32_t *>(sc->bitstream.p));
       HC(hipGetLastError());
