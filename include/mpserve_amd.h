@@ -263,6 +263,23 @@ typedef struct mps_awq_encode_in {
  * and slot 13 shape_nmkg_i64 (slot 9 is empty). Slots 14-16 are empty. */
 int mps_awq_encode(const mps_awq_encode_in *in, void *stream, mps_fp8_sidecar **out);
 
+/* The same builds into the caller's memory, without a handle. `alloc` is asked
+ * for device memory on the current device, usable on `stream`, 256-byte
+ * aligned: each non-empty output once, by its slot (0..16, the handle's order),
+ * and workspaces as slot -1; it returns NULL when it has none (then
+ * MPS_ERR_NO_MEMORY). Called on the calling thread. sizes17 and stats4 are as
+ * mps_fp8_sidecar_sizes and mps_fp8_sidecar_stats give them. Work on `stream`
+ * may still be running on return: the caller frees workspaces (and, after an
+ * error, outputs) in stream order. Host arrays of the caller are not used after
+ * the return. No counterpart in the reference, whose outputs are host tensors;
+ * it spares a serving or compressing program, whose allocator caches memory,
+ * the builder's own device allocations and the copies out of a handle. */
+typedef void *(*mps_encode_alloc)(void *ctx, int32_t slot, int64_t bytes);
+int mps_fp8_encode_alloc(const mps_fp8_encode_in *in, void *stream, mps_encode_alloc alloc, void *ctx,
+                         int64_t *sizes17, int64_t *stats4);
+int mps_awq_encode_alloc(const mps_awq_encode_in *in, void *stream, mps_encode_alloc alloc, void *ctx,
+                         int64_t *sizes17, int64_t *stats4);
+
 /* Element counts of the 17 outputs, in the reference's order (kernel/wrapper.cpp:429-446):
  * decode_syms_u16, decode_lens_u8, table_scale_u16, table_fp8_u16, bucket_scale_u16,
  * bucket_row_offsets_i32, row_indices_i32, bucket_table_i32, bucket_col_start_i32,

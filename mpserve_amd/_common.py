@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from typing import Dict, Optional
 
 import torch
 
@@ -42,3 +43,43 @@ def _maybe_check_status(device: torch.device, op: str = "huffman_decode_fp8") ->
         if st:
             raise RuntimeError(f"{op}: sidecar integrity flags 0x{st:x} "
                                "(1=bucket range, 2=row index, 4=table id, 8=lane bit desync)")
+
+
+class BuilderOutputs:
+    """A sidecar builder's device memory, from torch's allocator: the outputs it asks for by
+    slot and its workspaces, all on ``device`` and of the current stream (whose order makes
+    it safe to drop the workspaces when the call returns)."""
+
+    def __init__(self, device: torch.device, dtypes: Dict[int, torch.dtype]):
+        self._device, self._dtypes = device, dtypes
+        self._out: Dict[int, torch.Tensor] = {}
+        self._work: list = []
+        self._error: Optional[BaseException] = None
+
+    def _alloc(self, _ctx, slot: int, nbytes: int):
+        try:
+            dtype = self._dtypes.get(slot, torch.uint8)
+            t = torch.empty(nbytes // dtype.itemsize, dtype=dtype, device=self._device)
+            if slot >= 0:
+                self._out[slot] = t
+            else:
+                self._work.append(t)
+            return t.data_ptr()
+        except BaseException as e:  # raised again once the native call has returned
+            self._error = e
+            return None
+
+    def build(self, entry, args, stream: int):
+        """Runs ``entry`` (mps_*_encode_alloc); (sizes, stats) of its outputs."""
+        sizes, stats = (ctypes.c_int64 * 17)(), (ctypes.c_int64 * 4)()
+        rc = entry(ctypes.byref(args), ctypes.c_void_p(stream), _native.ENCODE_ALLOC(self._alloc), None, sizes, stats)
+        if self._error is not None:
+            raise self._error
+        _native.check(rc)
+        return sizes, stats
+
+    def tensor(self, slot: int, shape, on_host: bool) -> torch.Tensor:
+        t = self._out.get(slot)
+        if t is None:
+            t = torch.empty(0, dtype=self._dtypes[slot], device=self._device)
+        return t.view(shape).cpu() if on_host else t.view(shape)

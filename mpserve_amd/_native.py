@@ -76,6 +76,9 @@ class MpsAwqEncodeIn(ctypes.Structure):
     ]
 
 
+#: mps_encode_alloc: (ctx, slot, bytes) -> device pointer, or None for no memory
+ENCODE_ALLOC = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, _i64)
+
 _lib = None
 
 
@@ -107,6 +110,9 @@ def lib():
         L.mps_fp8_sidecar_copy.argtypes = [_p, ctypes.POINTER(_p), _p]
         L.mps_fp8_sidecar_free.argtypes = [_p]
         L.mps_fp8_sidecar_stats.argtypes = [_p, ctypes.POINTER(_i64)]
+    encode_alloc = [_p, ENCODE_ALLOC, _p, ctypes.POINTER(_i64), ctypes.POINTER(_i64)]
+    L.mps_fp8_encode_alloc.argtypes = [ctypes.POINTER(MpsFp8EncodeIn)] + encode_alloc
+    L.mps_awq_encode_alloc.argtypes = [ctypes.POINTER(MpsAwqEncodeIn)] + encode_alloc
     L.mps_awq_decode.argtypes = [ctypes.POINTER(MpsAwqTensor), _i64, _p]
     L.mps_awq_encode.argtypes = [ctypes.POINTER(MpsAwqEncodeIn), _p, ctypes.POINTER(_p)]
     L.mps_awq_plan_create.argtypes = [ctypes.POINTER(MpsAwqTensor), _i64, _p, ctypes.POINTER(_p)]
@@ -118,7 +124,7 @@ def lib():
     for name in ("mps_clock_rate_khz", "mps_fp8_decode", "mps_fp8_plan_create", "mps_fp8_plan_decode",
                  "mps_fp8_plan_decode_into", "mps_fp8_plan_info", "mps_fp8_plan_read_status",
                  "mps_fp8_plan_destroy", "mps_fp8_read_status", "mps_fp8_decode_batch_noalloc", "mps_stream_capture_id",
-                 "mps_awq_decode", "mps_awq_encode",
+                 "mps_awq_decode", "mps_awq_encode", "mps_fp8_encode_alloc", "mps_awq_encode_alloc",
                  "mps_awq_plan_create", "mps_awq_plan_decode", "mps_awq_plan_decode_into", "mps_awq_plan_info", "mps_awq_plan_read_status",
                  "mps_awq_plan_destroy"):
         getattr(L, name).restype = ctypes.c_int

@@ -24,7 +24,7 @@ from typing import Dict
 import torch
 
 from . import _native
-from ._common import _check_cuda_contig, _maybe_check_status, _stream_handle
+from ._common import BuilderOutputs, _check_cuda_contig, _maybe_check_status, _stream_handle
 
 # Dict keys in the reference's order (wrapper.cpp:268-281, :301-313) and the
 # builder-handle slot each comes from.
@@ -97,28 +97,14 @@ def _build(bf16, int4, scales, max_len, threads, group_cap, by_scale: bool, with
     a.scale_numel = sc.numel()
     a.by_scale = int(by_scale)
     a.max_len, a.threads_per_block, a.group_cap = int(max_len), int(threads), int(group_cap)
-    lib = _native.lib()
-    handle = ctypes.c_void_p()
     keys = BY_SCALE_KEYS if by_scale else BUCKET_KEYS
+    mem = BuilderOutputs(dev, {slot: dt for _, slot, dt in keys})
     with torch.cuda.device(dev):
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        _native.check(lib.mps_awq_encode(ctypes.byref(a), stream, ctypes.byref(handle)))
-        try:
-            sizes = (ctypes.c_int64 * 17)()
-            _native.check(lib.mps_fp8_sidecar_sizes(handle, sizes))
-            G, B, L = int(sizes[2]), int(sizes[4]), int(max_len)
-            shape = {0: (G, 1 << L), 1: (G, max(1, (1 << L) // 2)), 7: (B, 16), 10: (B, int(threads) + 1)}
-            ptrs = (ctypes.c_void_p * 17)()
-            out: Dict[str, torch.Tensor] = {}
-            for key, slot, dt in keys:
-                t = torch.empty(shape.get(slot, (int(sizes[slot]),)), dtype=dt, device="cpu" if on_host else dev)
-                out[key] = t
-                ptrs[slot] = t.data_ptr() if t.numel() else None
-            _native.check(lib.mps_fp8_sidecar_copy(handle, ptrs, stream))
-            stats = (ctypes.c_int64 * 4)()
-            _native.check(lib.mps_fp8_sidecar_stats(handle, stats))
-        finally:
-            lib.mps_fp8_sidecar_free(handle)
+        sizes, stats = mem.build(_native.lib().mps_awq_encode_alloc, a, _stream_handle(dev))
+        G, B, L = int(sizes[2]), int(sizes[4]), int(max_len)
+        shape = {0: (G, 1 << L), 1: (G, max(1, (1 << L) // 2)), 7: (B, 16), 10: (B, int(threads) + 1)}
+        out: Dict[str, torch.Tensor] = {key: mem.tensor(slot, shape.get(slot, (int(sizes[slot]),)), on_host)
+                                        for key, slot, _ in keys}
     if with_stats:
         return out, {"esc_keys": int(stats[0]), "esc_collisions": int(stats[1])}
     return out

@@ -23,7 +23,9 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -1359,18 +1361,21 @@ hipError_t device_scan(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_
 
 using namespace mps;
 
-// Result object: device arrays in the reference's 17-output order.
+// A handle's result: device arrays in the reference's 17-output order.
 struct mps_fp8_sidecar {
-  DevBuf<uint16_t> decode_syms, table_scale, table_fp8, bucket_scale;
-  DevBuf<uint8_t> decode_lens;
-  DevBuf<int32_t> bucket_row_offsets, row_indices, bucket_table, bucket_col_start, bucket_col_len, bucket_U,
-      bucket_unique_gid;
-  DevBuf<uint32_t> bucket_thread_startbit;
-  DevBuf<int64_t> bucket_bit_base, shape_nmk;
-  DevBuf<uint64_t> bitstream;
-  DevBuf<int16_t> bucket_fp8_uidx;
+  void *out[17] = {};
   int64_t sizes[17] = {};
   int64_t stats[4] = {};  // esc keys, esc collision elements, distinct (key, symbol) pairs, hash capacity
+  std::vector<void *> work;
+  ~mps_fp8_sidecar() {
+    for (void *p : out)
+      if (p) (void)hipFree(p);
+    free_work();
+  }
+  void free_work() {
+    for (void *p : work) (void)hipFree(p);
+    work.clear();
+  }
 };
 
 namespace mps {
@@ -1390,7 +1395,26 @@ struct EncodeSpec {
   int format;
 };
 
-int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
+constexpr int kOutBytes[17] = {2, 1, 2, 2, 2, 4, 4, 4, 4, 4, 4, 8, 8, 8, 4, 4, 2};  // of an element of each output
+
+// Arrays built on the host travel in one block; those that are outputs are
+// copied from it to their own buffers by one launch.
+struct Placed {
+  const char *src[6];
+  char *dst[6];
+  uint64_t bytes[6];
+};
+__global__ void place_kernel(Placed p) {
+  const int a = (int)blockIdx.y;
+  const uint64_t n = p.bytes[a], at = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (at + 4 <= n) *reinterpret_cast<uint32_t *>(p.dst[a] + at) = *reinterpret_cast<const uint32_t *>(p.src[a] + at);
+  else if (at + 2 <= n) *reinterpret_cast<uint16_t *>(p.dst[a] + at) = *reinterpret_cast<const uint16_t *>(p.src[a] + at);
+}
+
+// Runs the builder. Device memory comes from `alloc` (the 17 outputs by slot,
+// workspaces as slot -1); the last kernels may still run when this returns.
+int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, void *ctx, int64_t *sizes17,
+                int64_t *stats4) {
   const int64_t n = sp.n, m = sp.m, numel = n * m, L = sp.L, kth = sp.k, scale_numel = sp.scale_numel;
   const bool scale_scalar = sp.scalar, scale_block2d = sp.block2d;
   const int64_t nb0 = sp.nb0, nb1 = sp.nb1, sb0 = sp.sb0, sb1 = sp.sb1;
@@ -1401,185 +1425,192 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
   do {                                                          \
     if ((e = (x)) != hipSuccess) return hip_fail(e, #x);        \
   } while (0)
+// The output of a slot: `count` elements from the caller's allocator (null for none).
+#define OUT(name, T, slot, count)                                                                   \
+  T *name = nullptr;                                                                                \
+  {                                                                                                 \
+    const size_t out_n = (count);                                                                   \
+    if (out_n && !(name = static_cast<T *>(alloc(ctx, slot, (int64_t)(sizeof(T) * out_n)))))        \
+      return fail(MPS_ERR_NO_MEMORY, "no device memory for output %d of the sidecar builder", slot); \
+  }
 
   // --- scales to host, dense scale index (sorted unique values) ---
   std::vector<uint16_t> hsc((size_t)scale_numel);
   HC(hipMemcpyAsync(hsc.data(), sp.scales, sizeof(uint16_t) * scale_numel, hipMemcpyDeviceToHost, s));
   HC(hipStreamSynchronize(s));
-  std::vector<uint16_t> uniq_sc(hsc);
-  std::sort(uniq_sc.begin(), uniq_sc.end());
-  uniq_sc.erase(std::unique(uniq_sc.begin(), uniq_sc.end()), uniq_sc.end());
+  std::vector<uint16_t> rank(65536, 0), uniq_sc;
+  {
+    std::vector<uint8_t> seen(65536, 0);
+    for (uint16_t v : hsc) seen[v] = 1;
+    for (uint32_t v = 0; v < 65536; ++v)
+      if (seen[v]) {
+        rank[v] = (uint16_t)uniq_sc.size();
+        uniq_sc.push_back((uint16_t)v);
+      }
+  }
   const uint32_t S = (uint32_t)uniq_sc.size();
-  auto sidx_of_value = [&](uint16_t v) -> uint16_t {
-    return (uint16_t)(std::lower_bound(uniq_sc.begin(), uniq_sc.end(), v) - uniq_sc.begin());
-  };
 
   // --- buckets (build_huffman.cu:611-696), host ---
-  std::vector<int32_t> row_indices, row_offsets{0}, col_start, col_len;
-  std::vector<uint16_t> bucket_scale;
-  std::vector<uint16_t> row_sidx, block_sidx;
-  std::vector<int32_t> group_col;  // by scale: column start of each group
+  // Rows (groups, by scale) are dealt to their scales by counting: ascending
+  // scales, rows in order within one, which is the reference's stable sort.
   const bool by_scale = sp.format == kFmtAwqByScale;
-  if (by_scale) {
-    // quantisation groups (row, column start) bucketed by exact scale, scales
-    // ascending, groups in (row, column) order, <= group_cap a bucket
-    // (build_huffman.cu:1350-1385)
-    const int64_t gsz = scale_block2d ? sb1 : m;
-    const int64_t gpr = scale_block2d ? nb1 : 1;
-    if (!scale_block2d) {
-      row_sidx.resize((size_t)n);
-      for (int64_t r = 0; r < n; ++r) row_sidx[(size_t)r] = sidx_of_value(scale_scalar ? hsc[0] : hsc[(size_t)r]);
-    } else {
-      block_sidx.resize((size_t)(nb0 * nb1));
-      for (int64_t i = 0; i < nb0 * nb1; ++i) block_sidx[(size_t)i] = sidx_of_value(hsc[(size_t)i]);
-    }
-    std::vector<uint64_t> gk((size_t)(n * gpr));
-    for (int64_t r = 0; r < n; ++r)
-      for (int64_t bc = 0; bc < gpr; ++bc) {
-        const uint16_t v = scale_scalar ? hsc[0] : !scale_block2d ? hsc[(size_t)r] : hsc[(size_t)((r / sb0) * nb1 + bc)];
-        gk[(size_t)(r * gpr + bc)] = ((uint64_t)v << 40) | (uint64_t)(r * gpr + bc);
+  const int64_t width = scale_block2d ? sb1 : m;               // columns of a row (group) of a bucket
+  const int64_t per_row = by_scale && scale_block2d ? nb1 : 1;  // groups of a row
+  std::vector<int32_t> row_offsets{0};
+  std::vector<uint32_t> lane_base{0};
+  std::vector<uint16_t> bucket_sidx, bucket_scale;
+  std::vector<int32_t> row_indices, cols;  // cols: by bucket, or (by scale) by group
+  if (by_scale || !scale_block2d) {
+    std::vector<int64_t> at(S + 1, 0);  // first row (group) of each scale
+    if (scale_block2d)
+      for (uint16_t v : hsc) at[rank[v] + 1] += sb0;
+    else if (scale_scalar) at[1] = n;
+    else
+      for (uint16_t v : hsc) at[rank[v] + 1] += 1;
+    const int64_t cap_rows = by_scale ? sp.group_cap : 128;
+    for (uint32_t i = 0; i < S; ++i) {
+      const int64_t rows = at[i + 1];
+      for (int64_t off = 0; off < rows; off += std::min(cap_rows, rows - off)) {
+        bucket_sidx.push_back((uint16_t)i);
+        row_offsets.push_back(row_offsets.back() + (int32_t)std::min(cap_rows, rows - off));
       }
-    std::sort(gk.begin(), gk.end());
-    size_t i = 0;
-    while (i < gk.size()) {
-      size_t j = i;
-      while (j < gk.size() && (gk[j] >> 40) == (gk[i] >> 40)) ++j;
-      for (size_t off = i; off < j; off += (size_t)sp.group_cap) {
-        const size_t take = std::min<size_t>((size_t)sp.group_cap, j - off);
-        for (size_t q = 0; q < take; ++q) {
-          const int64_t gi = (int64_t)(gk[off + q] & 0xFFFFFFFFFFull);
-          row_indices.push_back((int32_t)(gi / gpr));
-          group_col.push_back((int32_t)((gi % gpr) * gsz));
-        }
-        bucket_scale.push_back((uint16_t)(gk[i] >> 40));
-        col_start.push_back(0);
-        col_len.push_back((int32_t)gsz);
-        row_offsets.push_back((int32_t)row_indices.size());
-      }
-      i = j;
+      at[i + 1] += at[i];
     }
-  } else if (!scale_block2d) {
-    row_sidx.resize((size_t)n);
-    std::vector<std::pair<uint16_t, int32_t>> order((size_t)n);
+    row_indices.resize((size_t)(n * per_row));
+    if (by_scale) cols.resize(row_indices.size());
+    std::vector<uint16_t> ranks(hsc.size());
+    for (size_t i = 0; i < ranks.size(); ++i) ranks[i] = rank[hsc[i]];
     for (int64_t r = 0; r < n; ++r) {
-      const uint16_t v = scale_scalar ? hsc[0] : hsc[(size_t)r];
-      order[(size_t)r] = {v, (int32_t)r};
-      row_sidx[(size_t)r] = sidx_of_value(v);
-    }
-    std::stable_sort(order.begin(), order.end(),
-                     [](const std::pair<uint16_t, int32_t> &x, const std::pair<uint16_t, int32_t> &y) {
-                       return x.first < y.first;
-                     });
-    size_t i = 0;
-    while (i < order.size()) {
-      size_t j = i;
-      while (j < order.size() && order[j].first == order[i].first) ++j;
-      for (size_t off = i; off < j; off += 128) {
-        const size_t take = std::min<size_t>(128, j - off);
-        for (size_t q = 0; q < take; ++q) row_indices.push_back(order[off + q].second);
-        bucket_scale.push_back(order[i].first);
-        col_start.push_back(0);
-        col_len.push_back((int32_t)m);
-        row_offsets.push_back((int32_t)row_indices.size());
+      const uint16_t *rk = ranks.data() + (scale_scalar ? 0 : scale_block2d ? r / sb0 * nb1 : r);
+      for (int64_t c = 0; c < per_row; ++c) {
+        const size_t to = (size_t)at[rk[c]]++;
+        row_indices[to] = (int32_t)r;
+        if (by_scale) cols[to] = (int32_t)(c * width);
       }
-      i = j;
     }
+    if (!by_scale) cols.assign(bucket_sidx.size(), 0);
   } else {
-    block_sidx.resize((size_t)(nb0 * nb1));
-    for (int64_t i = 0; i < nb0 * nb1; ++i) block_sidx[(size_t)i] = sidx_of_value(hsc[(size_t)i]);
     for (int64_t br = 0; br < nb0; ++br) {
       for (int64_t bc = 0; bc < nb1; ++bc) {
-        const uint16_t sc = hsc[(size_t)(br * nb1 + bc)];
         for (int64_t off = 0; off < sb0; off += 128) {
           const int64_t take = std::min<int64_t>(128, sb0 - off);
           for (int64_t q = 0; q < take; ++q) row_indices.push_back((int32_t)(br * sb0 + off + q));
-          bucket_scale.push_back(sc);
-          col_start.push_back((int32_t)(bc * sb1));
-          col_len.push_back((int32_t)sb1);
+          bucket_sidx.push_back(rank[hsc[(size_t)(br * nb1 + bc)]]);
+          cols.push_back((int32_t)(bc * sb1));
           row_offsets.push_back((int32_t)row_indices.size());
         }
       }
     }
   }
-  const uint32_t B = (uint32_t)bucket_scale.size();
-  std::vector<uint32_t> lane_base(B + 1, 0);
-  std::vector<uint16_t> bucket_sidx(B);
+  const uint32_t B = (uint32_t)bucket_sidx.size();
+  const std::vector<int32_t> col_len(B, (int32_t)width);
   for (uint32_t b = 0; b < B; ++b) {
-    const int64_t total = (int64_t)(row_offsets[b + 1] - row_offsets[b]) * col_len[b];
-    const int64_t k_eff = std::min<int64_t>(kth, std::max<int64_t>(1, total));
-    lane_base[b + 1] = lane_base[b] + (uint32_t)k_eff;
-    bucket_sidx[b] = sidx_of_value(bucket_scale[b]);
+    const int64_t total = (int64_t)(row_offsets[b + 1] - row_offsets[b]) * width;
+    lane_base.push_back(lane_base[b] + (uint32_t)std::min<int64_t>(kth, std::max<int64_t>(1, total)));
+    bucket_scale.push_back(uniq_sc[bucket_sidx[b]]);
   }
+  const bool fp8 = sp.format == kFmtFp8;
+  const int64_t shape[4] = {n, m, kth, by_scale ? width : 0};
+  const size_t nshape = by_scale ? 4 : 3;
 
-  auto sc = std::make_unique<mps_fp8_sidecar>();
-  DevBuf<uint16_t> d_bucket_sidx, d_scale_values;
-  DevBuf<uint32_t> d_lane_base;
-  HC(d_bucket_sidx.alloc(B));
-  HC(d_scale_values.alloc(S));
-  HC(d_lane_base.alloc(B + 1));
-  HC(hipMemcpyAsync(d_bucket_sidx.p, bucket_sidx.data(), 2 * (size_t)B, hipMemcpyHostToDevice, s));
-  HC(hipMemcpyAsync(d_scale_values.p, uniq_sc.data(), 2 * (size_t)S, hipMemcpyHostToDevice, s));
-  HC(hipMemcpyAsync(d_lane_base.p, lane_base.data(), 4 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
-
-  HC(sc->bucket_scale.alloc(B));
-  HC(sc->bucket_row_offsets.alloc(B + 1));
-  HC(sc->row_indices.alloc(row_indices.size()));
-  HC(sc->bucket_col_start.alloc(by_scale ? group_col.size() : (size_t)B));
-  HC(sc->bucket_col_len.alloc(B));
-  HC(hipMemcpyAsync(sc->bucket_scale.p, bucket_scale.data(), 2 * (size_t)B, hipMemcpyHostToDevice, s));
-  HC(hipMemcpyAsync(sc->bucket_row_offsets.p, row_offsets.data(), 4 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
-  if (!row_indices.empty())
-    HC(hipMemcpyAsync(sc->row_indices.p, row_indices.data(), 4 * row_indices.size(), hipMemcpyHostToDevice, s));
-  if (by_scale) {
-    if (!group_col.empty())
-      HC(hipMemcpyAsync(sc->bucket_col_start.p, group_col.data(), 4 * group_col.size(), hipMemcpyHostToDevice, s));
-  } else {
-    HC(hipMemcpyAsync(sc->bucket_col_start.p, col_start.data(), 4 * (size_t)B, hipMemcpyHostToDevice, s));
-  }
-  HC(hipMemcpyAsync(sc->bucket_col_len.p, col_len.data(), 4 * (size_t)B, hipMemcpyHostToDevice, s));
-
-  DevBuf<uint32_t> flags;  // [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count, [5..7] codebook
-                           // classes, [8..10] keys, entries and most entries of a scale (scan_parts)
+  // --- one device block: the host-built arrays (`put`), then work memory (`take`) ---
+  // flags: [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count, [5..7] codebook
+  // classes, [8..10] keys, entries and most entries of a scale (scan_parts)
   constexpr int kFlags = 16;
-  HC(flags.alloc(kFlags));
   uint32_t hflags[kFlags] = {};
-  DevBuf<uint32_t> tcount, tgid, gid_tkey, cb_lists;
+  std::vector<char> host;
+  size_t bytes = 0;
+  auto take = [&](size_t sz) {
+    const size_t at = bytes;
+    bytes += (sz + 255) & ~(size_t)255;
+    return at;
+  };
+  auto put = [&](const void *src, size_t sz) {
+    const size_t at = take(sz);
+    host.resize(bytes);
+    std::memcpy(host.data() + at, src, sz);
+    return at;
+  };
+  const size_t o_flags = put(hflags, sizeof(hflags)), o_scale_values = put(uniq_sc.data(), 2 * (size_t)S),
+               o_sidx = put(bucket_sidx.data(), 2 * (size_t)B), o_lane_base = put(lane_base.data(), 4 * lane_base.size()),
+               o_bscale = put(bucket_scale.data(), 2 * (size_t)B),
+               o_rowoff = put(row_offsets.data(), 4 * row_offsets.size()),
+               o_rows = put(row_indices.data(), 4 * row_indices.size()), o_cols = put(cols.data(), 4 * cols.size()),
+               o_clen = put(col_len.data(), 4 * (size_t)B), o_shape = put(shape, 8 * nshape);
+  char *blk = nullptr;
+  bool placed = false;  // the outputs among the host-built arrays are made once
+  uint32_t *flags = nullptr, *d_lane_base = nullptr, *tcount = nullptr, *tgid = nullptr, *gid_tkey = nullptr;
+  int32_t *d_row_offsets = nullptr, *d_row_indices = nullptr, *d_cols = nullptr, *d_col_len = nullptr;
+  auto at32 = [&](size_t o) { return reinterpret_cast<uint32_t *>(blk + o); };
+  // Allocates the block as laid out so far, uploads it and places the outputs it holds.
+  auto upload = [&]() -> int {
+    if (!(blk = static_cast<char *>(alloc(ctx, -1, (int64_t)bytes))))
+      return fail(MPS_ERR_NO_MEMORY, "no device memory for the sidecar builder's workspace (%zu bytes)", bytes);
+    HC(hipMemcpyAsync(blk, host.data(), host.size(), hipMemcpyHostToDevice, s));
+    flags = at32(o_flags);
+    d_lane_base = at32(o_lane_base);
+    d_row_offsets = reinterpret_cast<int32_t *>(blk + o_rowoff);
+    d_row_indices = reinterpret_cast<int32_t *>(blk + o_rows);
+    d_cols = reinterpret_cast<int32_t *>(blk + o_cols);
+    d_col_len = reinterpret_cast<int32_t *>(blk + o_clen);
+    if (placed) return MPS_OK;
+    placed = true;
+    OUT(x4, uint16_t, 4, (size_t)B);
+    OUT(x5, int32_t, 5, row_offsets.size());
+    OUT(x6, int32_t, 6, row_indices.size());
+    OUT(x8, int32_t, 8, cols.size());
+    OUT(x9, int32_t, 9, by_scale ? (size_t)0 : (size_t)B);
+    OUT(x13, int64_t, 13, nshape);
+    Placed pl = {{blk + o_bscale, blk + o_rowoff, blk + o_rows, blk + o_cols, blk + o_clen, blk + o_shape},
+                 {(char *)x4, (char *)x5, (char *)x6, (char *)x8, (char *)x9, (char *)x13},
+                 {2ull * B, 4 * row_offsets.size(), 4 * row_indices.size(), 4 * cols.size(), by_scale ? 0ull : 4ull * B,
+                  8 * nshape}};
+    const uint64_t longest = *std::max_element(pl.bytes, pl.bytes + 6);
+    hipLaunchKernelGGL(place_kernel, dim3((unsigned)((longest + 1023) / 1024), 6), dim3(256), 0, s, pl);
+    HC(hipGetLastError());
+    return MPS_OK;
+  };
+
   uint32_t D = 0, G = 0;
   uint64_t cap = 0;
   int64_t W = 0;
   const uint64_t T = (uint64_t)S * 256;
   const uint32_t Tsz = 1u << L;
   const uint32_t packed = Tsz / 2 > 0 ? Tsz / 2 : 1;
-  const bool fp8 = sp.format == kFmtFp8;
   CodebookArgs cba{};
+  int32_t *btab = nullptr, *bU = nullptr, *uniq = nullptr;
+  int16_t *uidx = nullptr;
   auto alloc_tables = [&]() -> int {  // the outputs whose sizes follow from G
-    HC(sc->decode_syms.alloc((size_t)G * Tsz));
-    HC(sc->decode_lens.alloc((size_t)G * packed));
-    HC(sc->table_scale.alloc(G));
-    HC(sc->table_fp8.alloc(G));
-    HC(sc->bucket_table.alloc((size_t)B * qvals));
-    HC(sc->bucket_U.alloc(fp8 ? B : 0));
-    HC(sc->bucket_unique_gid.alloc(fp8 ? (size_t)B * 256 : 0));
-    HC(sc->bucket_fp8_uidx.alloc(fp8 ? (size_t)B * 256 : 0));
-    cba.gid_tkey = gid_tkey.p;
-    cba.tcount = tcount.p;
-    cba.scale_values = d_scale_values.p;
-    cba.decode_syms = sc->decode_syms.p;
-    cba.decode_lens = sc->decode_lens.p;
-    cba.table_scale = sc->table_scale.p;
-    cba.table_fp8 = sc->table_fp8.p;
+    OUT(syms, uint16_t, 0, (size_t)G * Tsz);
+    OUT(lens, uint8_t, 1, (size_t)G * packed);
+    OUT(tscale, uint16_t, 2, (size_t)G);
+    OUT(tq, uint16_t, 3, (size_t)G);
+    OUT(x7, int32_t, 7, (size_t)B * qvals);
+    OUT(x14, int32_t, 14, fp8 ? (size_t)B : 0);
+    OUT(x15, int32_t, 15, fp8 ? (size_t)B * 256 : 0);
+    OUT(x16, int16_t, 16, fp8 ? (size_t)B * 256 : 0);
+    btab = x7;
+    bU = x14;
+    uniq = x15;
+    uidx = x16;
+    cba.gid_tkey = gid_tkey;
+    cba.tcount = tcount;
+    cba.scale_values = reinterpret_cast<const uint16_t *>(blk + o_scale_values);
+    cba.decode_syms = syms;
+    cba.decode_lens = lens;
+    cba.table_scale = tscale;
+    cba.table_fp8 = tq;
     cba.G = G;
     cba.L = (int)L;
     cba.esc_mode = sp.format;
-    cba.err = flags.p + 1;
-    cba.esc_stats = flags.p + 2;
+    cba.err = flags + 1;
+    cba.esc_stats = flags + 2;
     return MPS_OK;
   };
   auto bucket_tables = [&]() -> int {
     if (B)
-      hipLaunchKernelGGL(bucket_table_kernel, dim3(fp8 ? B : (B * 16 + 255) / 256), dim3(256), 0, s, d_bucket_sidx.p, B,
-                         qvals, tcount.p, tgid.p, sc->bucket_table.p, sc->bucket_U.p, sc->bucket_unique_gid.p,
-                         sc->bucket_fp8_uidx.p);
+      hipLaunchKernelGGL(bucket_table_kernel, dim3(fp8 ? B : (B * 16 + 255) / 256), dim3(256), 0, s,
+                         reinterpret_cast<const uint16_t *>(blk + o_sidx), B, qvals, tcount, tgid, btab, bU, uniq, uidx);
     HC(hipGetLastError());
     return MPS_OK;
   };
@@ -1608,7 +1639,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     std::vector<uint64_t> scale_elems(S, 0);
     uint64_t elem = 0, lists_n = 0;
     for (uint32_t b = 0; b < B; ++b) {
-      const uint64_t cl = (uint64_t)col_len[b], total = (uint64_t)(row_offsets[b + 1] - row_offsets[b]) * cl;
+      const uint64_t cl = (uint64_t)width, total = (uint64_t)(row_offsets[b + 1] - row_offsets[b]) * cl;
       const uint64_t ke = lane_base[b + 1] - lane_base[b];
       const uint64_t steps = (total + ke - 1) / ke;
       const uint64_t most = std::max<uint64_t>(1, std::min<uint64_t>(target, (uint64_t)kUnitRows * cl) / ke);
@@ -1640,111 +1671,103 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
       entries += std::min<uint64_t>(scale_elems[i / P], kPairSlots);
     }
     // One device block: the host-built arrays, then the passes' own.
-    std::vector<char> host;
-    size_t bytes = 0;
-    auto take = [&](size_t n) {
-      const size_t at = bytes;
-      bytes += (n + 255) & ~(size_t)255;
-      return at;
-    };
-    auto put = [&](const void *src, size_t n) {
-      const size_t at = take(n);
-      host.resize(bytes);
-      std::memcpy(host.data() + at, src, n);
-      return at;
-    };
     const size_t o_units = put(units.data(), sizeof(Unit) * U), o_bunit = put(bucket_unit.data(), 4 * bucket_unit.size()),
                  o_belem = put(bucket_elem.data(), 4 * (size_t)B), o_loff = put(list_off.data(), 4 * U),
                  o_sunit = put(scale_units.data(), 4 * scale_units.size()),
                  o_uos = put(unit_of_scale.data(), 4 * U), o_poff = put(part_off.data(), 4 * part_off.size());
-    const size_t host_bytes = bytes;
     const size_t o_ln = take(4 * U), o_pn = take(4 * part_off.size()), o_pk = take(4 * part_off.size()),
                  o_lists = take(8 * lists_n), o_skeys = take(8 * entries), o_cw = take(4 * entries),
-                 o_toff = take(4 * T), o_codes = take(2 * (size_t)numel), o_pieces = take(4 * (size_t)kUnitThreads * U),
+                 o_toff = take(4 * T), o_tcount = take(4 * T), o_tgid = take(4 * T), o_tkey = take(4 * T),
+                 o_cbl = take(12 * T), o_codes = take(2 * (size_t)numel), o_pieces = take(4 * (size_t)kUnitThreads * U),
                  o_bbits = take(4 * (size_t)B);
-    DevBuf<char> blk;
-    HC(blk.alloc(bytes));
-    HC(tcount.alloc(T));
-    HC(tgid.alloc(T));
-    HC(gid_tkey.alloc(T));
-    HC(cb_lists.alloc(3 * T));
-    auto at32 = [&](size_t o) { return reinterpret_cast<uint32_t *>(blk.p + o); };
-    HC(hipMemcpyAsync(blk.p, host.data(), host_bytes, hipMemcpyHostToDevice, s));
-    HC(hipMemsetAsync(flags.p, 0, 4 * kFlags, s));
+    int rc = upload();
+    if (rc != MPS_OK) return rc;
+    tcount = at32(o_tcount);
+    tgid = at32(o_tgid);
+    gid_tkey = at32(o_tkey);
+    uint32_t *cb_lists = at32(o_cbl);
     UnitArgs ua;
-    ua.units = reinterpret_cast<const Unit *>(blk.p + o_units);
+    ua.units = reinterpret_cast<const Unit *>(blk + o_units);
     ua.bf16 = sp.bf16;
     ua.q = sp.q;
     ua.m = (uint32_t)m;
     ua.qmask = qmask;
-    ua.row_offsets = sc->bucket_row_offsets.p;
-    ua.row_indices = sc->row_indices.p;
-    ua.col_start = by_scale ? nullptr : sc->bucket_col_start.p;
-    ua.col_len = sc->bucket_col_len.p;
-    ua.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    ua.row_offsets = d_row_offsets;
+    ua.row_indices = d_row_indices;
+    ua.col_start = by_scale ? nullptr : d_cols;
+    ua.col_len = d_col_len;
+    ua.row_col = by_scale ? d_cols : nullptr;
     ua.k = (uint32_t)kth;
     // every row's column range starts and ends on 8 elements (columns start at multiples of the range's width)
-    ua.vec8 = m % 8 == 0 && col_len[0] % 8 == 0 && reinterpret_cast<uintptr_t>(sp.bf16) % 16 == 0 &&
+    ua.vec8 = m % 8 == 0 && width % 8 == 0 && reinterpret_cast<uintptr_t>(sp.bf16) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(sp.q) % 8 == 0;
-    auto *lists = reinterpret_cast<uint2 *>(blk.p + o_lists);
-    auto *skeys = reinterpret_cast<uint64_t *>(blk.p + o_skeys);
-    auto *codes = reinterpret_cast<uint16_t *>(blk.p + o_codes);
+    auto *lists = reinterpret_cast<uint2 *>(blk + o_lists);
+    auto *skeys = reinterpret_cast<uint64_t *>(blk + o_skeys);
+    auto *codes = reinterpret_cast<uint16_t *>(blk + o_codes);
     hipLaunchKernelGGL(unit_hist, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, at32(o_loff), lists, at32(o_ln),
-                       flags.p);
+                       flags);
     hipLaunchKernelGGL(merge_lists, dim3(S * P), dim3(kUnitThreads), 0, s, at32(o_sunit), at32(o_uos), at32(o_loff),
-                       at32(o_ln), lists, P, (uint32_t)qvals, at32(o_poff), skeys, tcount.p, at32(o_toff), at32(o_pn),
-                       at32(o_pk), flags.p);
-    hipLaunchKernelGGL(scan_parts, dim3(1), dim3(kScanBlock), 0, s, at32(o_pk), at32(o_pn), S, P, flags.p + 8);
-    hipLaunchKernelGGL(number_keys, dim3(S), dim3(256), 0, s, tcount.p, at32(o_pk), P, Tsz, (uint32_t)qvals, tgid.p,
-                       gid_tkey.p, cb_lists.p, (uint32_t)T, flags.p + 5);
+                       at32(o_ln), lists, P, (uint32_t)qvals, at32(o_poff), skeys, tcount, at32(o_toff), at32(o_pn),
+                       at32(o_pk), flags);
+    hipLaunchKernelGGL(scan_parts, dim3(1), dim3(kScanBlock), 0, s, at32(o_pk), at32(o_pn), S, P, flags + 8);
+    hipLaunchKernelGGL(number_keys, dim3(S), dim3(256), 0, s, tcount, at32(o_pk), P, Tsz, (uint32_t)qvals, tgid,
+                       gid_tkey, cb_lists, (uint32_t)T, flags + 5);
     HC(hipGetLastError());
-    HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
     const uint32_t most = hflags[10];  // entries of the scale that has most
     if (hflags[0] || most > 12288) return kGeneral;
     G = hflags[8];
     D = hflags[9];
     cap = (uint64_t)S * P * kPairSlots;
-    int rc = alloc_tables();
-    if (rc != MPS_OK) return rc;
+    if ((rc = alloc_tables()) != MPS_OK) return rc;
     cba.toff = at32(o_toff);
     cba.cw_slot = at32(o_cw);
-    launch_codebooks(cba, skeys, nullptr, cb_lists.p, (uint32_t)T, flags.p + 5, G, s);
+    launch_codebooks(cba, skeys, nullptr, cb_lists, (uint32_t)T, flags + 5, G, s);
     HC(hipGetLastError());
     if ((rc = bucket_tables()) != MPS_OK) return rc;
-    HC(sc->bucket_thread_startbit.alloc((size_t)B * (kth + 1)));
-    HC(sc->bucket_bit_base.alloc(B + 1));
+    OUT(startbit, uint32_t, 10, (size_t)B * (kth + 1));
+    OUT(bit_base, int64_t, 11, (size_t)B + 1);
     // the smaller table (two workgroups a CU) while it is at most 3/4 full
     auto codes_pass = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)U), dim3(kUnitThreads), 0, s, ua, P, at32(o_poff), at32(o_pn), skeys,
-                         at32(o_cw), at32(o_belem), codes, at32(o_pieces), flags.p + 1);
+                         at32(o_cw), at32(o_belem), codes, at32(o_pieces), flags + 1);
     };
     if (most <= 6144) codes_pass(unit_codes<8192>);
     else codes_pass(unit_codes<16384>);
-    hipLaunchKernelGGL(bucket_starts, dim3(B), dim3(kUnitThreads), 0, s, ua.units, at32(o_bunit), d_lane_base.p,
-                       (uint32_t)kth, at32(o_pieces), sc->bucket_thread_startbit.p, at32(o_bbits));
-    hipLaunchKernelGGL(bucket_bases, dim3(1), dim3(kScanBlock), 0, s, at32(o_bbits), B, sc->bucket_bit_base.p);
+    hipLaunchKernelGGL(bucket_starts, dim3(B), dim3(kUnitThreads), 0, s, ua.units, at32(o_bunit), d_lane_base,
+                       (uint32_t)kth, at32(o_pieces), startbit, at32(o_bbits));
+    hipLaunchKernelGGL(bucket_bases, dim3(1), dim3(kScanBlock), 0, s, at32(o_bbits), B, bit_base);
     HC(hipGetLastError());
     int64_t end = 0;
-    HC(hipMemcpyAsync(&end, sc->bucket_bit_base.p + B, 8, hipMemcpyDeviceToHost, s));
-    HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(&end, bit_base + B, 8, hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
     if ((rc = check_errors()) != MPS_OK) return rc;
     W = (end + 63) >> 6;
-    HC(sc->bitstream.alloc((size_t)W));
+    OUT(bitstream, uint64_t, 12, (size_t)W);
     if (W) {
       hipLaunchKernelGGL(unit_pack, dim3((unsigned)(U + 7) / 8 * 8), dim3(kUnitThreads), 0, s, ua, (uint32_t)U,
                          at32(o_belem), codes,
-                         at32(o_pieces), sc->bucket_thread_startbit.p, sc->bucket_bit_base.p,
-                         reinterpret_cast<uint32_t *>(sc->bitstream.p));
+                         at32(o_pieces), startbit, bit_base,
+                         reinterpret_cast<uint32_t *>(bitstream));
       HC(hipGetLastError());
     }
-    HC(hipStreamSynchronize(s));  // the block goes out of scope
     return MPS_OK;
   };
 
   // --- the general path: hash tables in global memory, a work-item a substream ---
   auto general_path = [&]() -> int {
+    int rc = upload();
+    if (rc != MPS_OK) return rc;
+    std::vector<uint16_t> row_sidx, block_sidx;
+    if (scale_block2d) {
+      block_sidx.resize((size_t)(nb0 * nb1));
+      for (size_t i = 0; i < block_sidx.size(); ++i) block_sidx[i] = rank[hsc[i]];
+    } else {
+      row_sidx.resize((size_t)n);
+      for (size_t r = 0; r < row_sidx.size(); ++r) row_sidx[r] = rank[hsc[scale_scalar ? 0 : r]];
+    }
     DevBuf<uint16_t> d_row_sidx, d_block_sidx;
     HC(d_row_sidx.alloc(row_sidx.size()));
     HC(d_block_sidx.alloc(block_sidx.size()));
@@ -1772,11 +1795,11 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
       HC(counts.alloc(cap));
       HC(hipMemsetAsync(keys.p, 0xFF, sizeof(uint64_t) * cap, s));
       HC(hipMemsetAsync(counts.p, 0, sizeof(uint32_t) * cap, s));
-      HC(hipMemsetAsync(flags.p, 0, sizeof(uint32_t) * kFlags, s));
+      HC(hipMemsetAsync(flags, 0, sizeof(uint32_t) * kFlags, s));
       hipLaunchKernelGGL(hist_kernel, dim3(hist_blocks), dim3(kHistBlock), 0, s, sp.bf16, sp.q, n, m, smap,
-                         qmask, per_block, keys.p, counts.p, cap - 1, flags.p);
+                         qmask, per_block, keys.p, counts.p, cap - 1, flags);
       HC(hipGetLastError());
-      HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+      HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
       HC(hipStreamSynchronize(s));
       if (!hflags[0]) break;
       if (cap >= ((uint64_t)1 << 34)) return fail(MPS_ERR_RUNTIME, "histogram table overflow");
@@ -1792,43 +1815,45 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
       HC(ccount.alloc(cap));
       HC(cslot.alloc(cap));
       hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((cap + 255) / 256)), dim3(256), 0, s, keys.p, counts.p, cap,
-                         ckey.p, ccount.p, cslot.p, flags.p + 4);
+                         ckey.p, ccount.p, cslot.p, flags + 4);
       HC(hipGetLastError());
-      HC(hipMemcpyAsync(&D, flags.p + 4, 4, hipMemcpyDeviceToHost, s));
+      HC(hipMemcpyAsync(&D, flags + 4, 4, hipMemcpyDeviceToHost, s));
       HC(hipStreamSynchronize(s));
     }
-    DevBuf<uint32_t> toff, tfill, tnz;
-    HC(tcount.alloc(T));
+    DevBuf<uint32_t> toff, tfill, tnz, d_tcount, d_tgid, d_tkey, cb_lists;
+    HC(d_tcount.alloc(T));
+    tcount = d_tcount.p;
     HC(toff.alloc(T));
     HC(tfill.alloc(T));
     HC(tnz.alloc(T));
-    HC(tgid.alloc(T));
-    HC(hipMemsetAsync(tcount.p, 0, 4 * T, s));
+    HC(d_tgid.alloc(T));
+    tgid = d_tgid.p;
+    HC(hipMemsetAsync(tcount, 0, 4 * T, s));
     HC(hipMemsetAsync(tfill.p, 0, 4 * T, s));
-    hipLaunchKernelGGL(table_count_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, D, tcount.p);
+    hipLaunchKernelGGL(table_count_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, D, tcount);
     HC(hipGetLastError());
     uint32_t D_check = 0;
     G = 0;
-    HC(device_scan(tcount.p, toff.p, T, s, &D_check));
-    hipLaunchKernelGGL(nonzero_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, T, tnz.p);
+    HC(device_scan(tcount, toff.p, T, s, &D_check));
+    hipLaunchKernelGGL(nonzero_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount, T, tnz.p);
     HC(hipGetLastError());
-    HC(device_scan(tnz.p, tgid.p, T, s, &G));
+    HC(device_scan(tnz.p, tgid, T, s, &G));
     if (D_check != D) return fail(MPS_ERR_RUNTIME, "internal error: histogram grouping mismatch");
     DevBuf<uint16_t> seg_sym;
     DevBuf<uint32_t> seg_cnt, seg_slot, ws_off, cw_slot;
     HC(seg_sym.alloc(D));
     HC(seg_cnt.alloc(D));
     HC(seg_slot.alloc(D));
-    HC(gid_tkey.alloc(G));
+    HC(d_tkey.alloc(G));
+    gid_tkey = d_tkey.p;
     hipLaunchKernelGGL(scatter_kernel, dim3((D + 255) / 256), dim3(256), 0, s, ckey.p, ccount.p, cslot.p, D, toff.p,
                        tfill.p, seg_sym.p, seg_cnt.p, seg_slot.p);
-    hipLaunchKernelGGL(table_list_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount.p, tgid.p, T,
-                       gid_tkey.p);
+    hipLaunchKernelGGL(table_list_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, tcount, tgid, T,
+                       gid_tkey);
     HC(hipGetLastError());
 
     // --- 3. code books ---
-    int rc = alloc_tables();
-    if (rc != MPS_OK) return rc;
+    if ((rc = alloc_tables()) != MPS_OK) return rc;
     HC(cw_slot.alloc(cap));
     // Codebooks. L <= 11 (the FP8 and AWQ formats): the keys' histogram entries
     // are sorted for all keys at once, then a wave per key builds each codebook in
@@ -1848,7 +1873,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
       if (D)
         hipLaunchKernelGGL(item_keys_kernel, dim3((D + 255) / 256), dim3(256), 0, s, seg_sym.p, seg_cnt.p, (uint64_t)D,
                            keys_in.p);
-      hipLaunchKernelGGL(segment_bounds_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, toff.p, tcount.p, G,
+      hipLaunchKernelGGL(segment_bounds_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey, toff.p, tcount, G,
                          seg_beg.p, seg_end.p);
       HC(hipGetLastError());
       size_t tmp_bytes = 0;
@@ -1864,7 +1889,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     HC(ws_off.alloc(G));
     uint32_t ws_total = 0;
     if (G && !wave_cb) {
-      hipLaunchKernelGGL(ws_size_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, tcount.p, G, Tsz,
+      hipLaunchKernelGGL(ws_size_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey, tcount, G, Tsz,
                          ws_sz.p);
       HC(hipGetLastError());
       HC(device_scan(ws_sz.p, ws_off.p, G, s, &ws_total));
@@ -1880,10 +1905,10 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     cba.cw_slot = cw_slot.p;
     if (G && wave_cb) {
       HC(cb_lists.alloc(3 * (size_t)G));
-      HC(hipMemsetAsync(flags.p + 5, 0, 12, s));
-      hipLaunchKernelGGL(codebook_classes_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey.p, tcount.p, G, Tsz,
-                         cb_lists.p, flags.p + 5);
-      launch_codebooks(cba, keys_sorted.p, slots_sorted.p, cb_lists.p, G, flags.p + 5, G, s);
+      HC(hipMemsetAsync(flags + 5, 0, 12, s));
+      hipLaunchKernelGGL(codebook_classes_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey, tcount, G, Tsz,
+                         cb_lists.p, flags + 5);
+      launch_codebooks(cba, keys_sorted.p, slots_sorted.p, cb_lists.p, G, flags + 5, G, s);
     } else if (G) {
       hipLaunchKernelGGL(codebook_kernel, dim3((G + 63) / 64), dim3(64), 0, s, cba);
     }
@@ -1893,8 +1918,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     if ((rc = bucket_tables()) != MPS_OK) return rc;
 
     // --- 5. bitstream ---
-    HC(sc->bucket_thread_startbit.alloc((size_t)B * (kth + 1)));
-    HC(hipMemsetAsync(sc->bucket_thread_startbit.p, 0, 4 * (size_t)B * (kth + 1), s));
+    OUT(startbit, uint32_t, 10, (size_t)B * (kth + 1));
+    HC(hipMemsetAsync(startbit, 0, 4 * (size_t)B * (kth + 1), s));
     DevBuf<uint32_t> cw_elem, bucket_bits;
     HC(cw_elem.alloc((size_t)numel));
     HC(bucket_bits.alloc(B));
@@ -1903,30 +1928,30 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     la.bf16 = sp.bf16;
     la.fp8 = sp.q;
     la.qmask = qmask;
-    la.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    la.row_col = by_scale ? d_cols : nullptr;
     la.S = smap;
     la.m = m;
-    la.row_offsets = sc->bucket_row_offsets.p;
-    la.row_indices = sc->row_indices.p;
-    la.col_start = sc->bucket_col_start.p;
-    la.col_len = sc->bucket_col_len.p;
-    la.lane_base = d_lane_base.p;
+    la.row_offsets = d_row_offsets;
+    la.row_indices = d_row_indices;
+    la.col_start = d_cols;
+    la.col_len = d_col_len;
+    la.lane_base = d_lane_base;
     la.B = B;
     la.k = kth;
     la.keys = keys.p;
     la.cw_slot = cw_slot.p;
     la.cap_mask = cap - 1;
     la.cw_elem = cw_elem.p;
-    la.lane_bits = sc->bucket_thread_startbit.p;
-    la.err = flags.p + 1;
+    la.lane_bits = startbit;
+    la.err = flags + 1;
     if (lanes) hipLaunchKernelGGL(lane_bits_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, la);
     HC(hipGetLastError());
-    if (B) hipLaunchKernelGGL(lane_starts_kernel, dim3(B), dim3(1024), 0, s, sc->bucket_thread_startbit.p,
-                              d_lane_base.p, kth, bucket_bits.p);
+    if (B) hipLaunchKernelGGL(lane_starts_kernel, dim3(B), dim3(1024), 0, s, startbit,
+                              d_lane_base, kth, bucket_bits.p);
     HC(hipGetLastError());
     std::vector<uint32_t> h_bucket_bits(B);
     if (B) HC(hipMemcpyAsync(h_bucket_bits.data(), bucket_bits.p, 4 * (size_t)B, hipMemcpyDeviceToHost, s));
-    HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
+    HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
     if ((rc = check_errors()) != MPS_OK) return rc;
     // 64-bit aligned bucket bases (build_huffman.cu:813-818), final cursor unaligned
@@ -1939,25 +1964,25 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
     }
     bit_base[B] = pos;
     W = (pos + 63) >> 6;
-    HC(sc->bucket_bit_base.alloc(B + 1));
-    HC(hipMemcpyAsync(sc->bucket_bit_base.p, bit_base.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
-    HC(sc->bitstream.alloc((size_t)W));
-    if (W) HC(hipMemsetAsync(sc->bitstream.p, 0, 8 * (size_t)W, s));
+    OUT(d_bit_base, int64_t, 11, (size_t)B + 1);
+    HC(hipMemcpyAsync(d_bit_base, bit_base.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, s));
+    OUT(bitstream, uint64_t, 12, (size_t)W);
+    if (W) HC(hipMemsetAsync(bitstream, 0, 8 * (size_t)W, s));
     PackArgs pa;
     pa.bf16 = sp.bf16;
-    pa.row_col = by_scale ? sc->bucket_col_start.p : nullptr;
+    pa.row_col = by_scale ? d_cols : nullptr;
     pa.m = m;
-    pa.row_offsets = sc->bucket_row_offsets.p;
-    pa.row_indices = sc->row_indices.p;
-    pa.col_start = sc->bucket_col_start.p;
-    pa.col_len = sc->bucket_col_len.p;
-    pa.lane_base = d_lane_base.p;
+    pa.row_offsets = d_row_offsets;
+    pa.row_indices = d_row_indices;
+    pa.col_start = d_cols;
+    pa.col_len = d_col_len;
+    pa.lane_base = d_lane_base;
     pa.B = B;
     pa.k = kth;
     pa.cw_elem = cw_elem.p;
-    pa.startbit = sc->bucket_thread_startbit.p;
-    pa.bit_base = sc->bucket_bit_base.p;
-    pa.bits = reinterpret_cast<unsigned long long *>(sc->bitstream.p);
+    pa.startbit = startbit;
+    pa.bit_base = d_bit_base;
+    pa.bits = reinterpret_cast<unsigned long long *>(bitstream);
     if (lanes && W) hipLaunchKernelGGL(pack_kernel, dim3((lanes + 255) / 256), dim3(256), 0, s, pa);
     HC(hipGetLastError());
     HC(hipStreamSynchronize(s));
@@ -1967,26 +1992,51 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
   int path_rc = unit_path();
   if (path_rc == kGeneral) path_rc = general_path();
   if (path_rc != MPS_OK) return path_rc;
-  const int64_t shape[4] = {n, m, kth, by_scale ? (int64_t)col_len.front() : 0};
-  const int nshape = by_scale ? 4 : 3;
-  HC(sc->shape_nmk.alloc(nshape));
-  HC(hipMemcpyAsync(sc->shape_nmk.p, shape, 8 * nshape, hipMemcpyHostToDevice, s));
-  HC(hipMemcpyAsync(hflags, flags.p, sizeof(hflags), hipMemcpyDeviceToHost, s));
-  HC(hipStreamSynchronize(s));
 
   // by scale, slots 5, 6 and 8 hold the group offsets, group rows and group column starts
   const int64_t sizes[17] = {(int64_t)G * Tsz, (int64_t)G * packed, G, G, B, B + 1, (int64_t)row_indices.size(),
-                             (int64_t)B * qvals, by_scale ? (int64_t)group_col.size() : B, by_scale ? 0 : B,
-                             (int64_t)B * (kth + 1), B + 1, W, nshape, fp8 ? B : 0, fp8 ? (int64_t)B * 256 : 0,
-                             fp8 ? (int64_t)B * 256 : 0};
-  std::memcpy(sc->sizes, sizes, sizeof(sizes));
-  sc->stats[0] = hflags[2];
-  sc->stats[1] = hflags[3];
-  sc->stats[2] = D;
-  sc->stats[3] = (int64_t)cap;
+                             (int64_t)B * qvals, (int64_t)cols.size(), by_scale ? 0 : B, (int64_t)B * (kth + 1), B + 1,
+                             W, (int64_t)nshape, fp8 ? B : 0, fp8 ? (int64_t)B * 256 : 0, fp8 ? (int64_t)B * 256 : 0};
+  std::memcpy(sizes17, sizes, sizeof(sizes));
+  stats4[0] = hflags[2];
+  stats4[1] = hflags[3];
+  stats4[2] = D;
+  stats4[3] = (int64_t)cap;
+  return MPS_OK;
+#undef OUT
+#undef HC
+}
+
+// The handle's allocator: hipMalloc, outputs by slot, workspaces freed when the build ends.
+void *handle_alloc(void *ctx, int32_t slot, int64_t bytes) {
+  auto *sc = static_cast<mps_fp8_sidecar *>(ctx);
+  void *p = nullptr;
+  if (hipMalloc(&p, (size_t)bytes) != hipSuccess) return nullptr;
+  if (slot >= 0) sc->out[slot] = p;
+  else sc->work.push_back(p);
+  return p;
+}
+
+// A builder run into a new handle.
+int encode_handle(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
+  auto sc = std::make_unique<mps_fp8_sidecar>();
+  const int rc = encode_impl(sp, s, handle_alloc, sc.get(), sc->sizes, sc->stats);
+  const hipError_t e = hipStreamSynchronize(s);  // before the workspaces go, also after a failure
+  if (rc != MPS_OK) return rc;
+  if (e != hipSuccess) return hip_fail(e, "sidecar builder");
+  sc->free_work();
   *out = sc.release();
   return MPS_OK;
-#undef HC
+}
+
+// No C++ exception (a host array too large for memory) leaves a C entry.
+template <typename F>
+int no_throw(F &&f) {
+  try {
+    return f();
+  } catch (const std::exception &x) {
+    return fail(MPS_ERR_NO_MEMORY, "sidecar builder: %s", x.what());
+  }
 }
 
 }  // namespace
@@ -1994,11 +2044,11 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_fp8_sidecar **out) {
 
 extern "C" {
 
-int mps_fp8_encode(const mps_fp8_encode_in *in, void *stream, mps_fp8_sidecar **out) {
-  last_error().clear();
-  if (!in || !out) return fail(MPS_ERR_INVALID_ARGUMENT, "inputs must be defined");
-  *out = nullptr;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+}  // extern "C"
+
+namespace {
+// The argument checks of mps_fp8_encode: the run to make, or an error.
+int fp8_spec(const mps_fp8_encode_in *in, EncodeSpec *spec) {
   const int64_t L = in->max_len, kth = in->threads_per_block;
   if (L <= 0 || L > 15) return fail(MPS_ERR_INVALID_ARGUMENT, "max_len must be in [1, 15]");
   if (kth <= 0 || kth > 1024) return fail(MPS_ERR_INVALID_ARGUMENT, "threads_per_block must be in [1, 1024]");
@@ -2039,16 +2089,13 @@ int mps_fp8_encode(const mps_fp8_encode_in *in, void *stream, mps_fp8_sidecar **
                 "bucket packing requires scales to be scalar, per-row (n,), or 2D block-wise");
   if (numel != n * m) return fail(MPS_ERR_INVALID_ARGUMENT, "bf16_params and fp8_params must have same numel");
   if (numel >= (int64_t)1 << 32) return fail(MPS_ERR_INVALID_ARGUMENT, "tensor too large for the GPU builder");
-  EncodeSpec sp{in->bf16, in->fp8, in->scales, n, m, scale_numel, scale_scalar, scale_per_row, scale_block2d,
-                nb0, nb1, sb0, sb1, L, kth, 0, kFmtFp8};
-  return encode_impl(sp, s, out);
+  *spec = EncodeSpec{in->bf16, in->fp8, in->scales, n, m, scale_numel, scale_scalar, scale_per_row, scale_block2d,
+                     nb0, nb1, sb0, sb1, L, kth, 0, kFmtFp8};
+  return MPS_OK;
 }
 
-
-int mps_awq_encode(const mps_awq_encode_in *in, void *stream, mps_fp8_sidecar **out) {
-  last_error().clear();
-  if (!in || !out) return fail(MPS_ERR_INVALID_ARGUMENT, "inputs must be defined");
-  *out = nullptr;
+// The argument checks of mps_awq_encode.
+int awq_spec(const mps_awq_encode_in *in, EncodeSpec *spec) {
   // checks of build_huffman.cu:1097-1153 (by scale) and :1605-1650, in order
   const int64_t L = in->max_len, kth = in->threads_per_block, n = in->n, m = in->m;
   if (L <= 0 || L > 15) return fail(MPS_ERR_INVALID_ARGUMENT, "max_len must be in (0,15]");
@@ -2077,9 +2124,52 @@ int mps_awq_encode(const mps_awq_encode_in *in, void *stream, mps_fp8_sidecar **
   if (n * m >= (int64_t)1 << 32) return fail(MPS_ERR_INVALID_ARGUMENT, "tensor too large for the GPU builder");
   if (in->by_scale && n * (block2d ? nb1 : 1) >= (int64_t)1 << 31)
     return fail(MPS_ERR_INVALID_ARGUMENT, "too many quantisation groups for the GPU builder");
-  EncodeSpec sp{in->bf16, in->int4, in->scales, n, m, scale_numel, scalar, per_row, block2d, nb0, nb1, sb0, sb1,
-                L, kth, in->group_cap, in->by_scale ? kFmtAwqByScale : kFmtAwqBucket};
-  return encode_impl(sp, reinterpret_cast<hipStream_t>(stream), out);
+  *spec = EncodeSpec{in->bf16, in->int4, in->scales, n, m, scale_numel, scalar, per_row, block2d, nb0, nb1, sb0, sb1,
+                     L, kth, in->group_cap, in->by_scale ? kFmtAwqByScale : kFmtAwqBucket};
+  return MPS_OK;
+}
+
+template <typename In>
+int to_handle(const In *in, int (*make)(const In *, EncodeSpec *), void *stream, mps_fp8_sidecar **out) {
+  last_error().clear();
+  if (!in || !out) return fail(MPS_ERR_INVALID_ARGUMENT, "inputs must be defined");
+  *out = nullptr;
+  EncodeSpec sp;
+  const int rc = make(in, &sp);
+  return rc != MPS_OK ? rc : no_throw([&] { return encode_handle(sp, reinterpret_cast<hipStream_t>(stream), out); });
+}
+
+template <typename In>
+int to_alloc(const In *in, int (*make)(const In *, EncodeSpec *), void *stream, mps_encode_alloc alloc, void *ctx,
+             int64_t *sizes17, int64_t *stats4) {
+  last_error().clear();
+  if (!in || !alloc || !sizes17 || !stats4) return fail(MPS_ERR_INVALID_ARGUMENT, "inputs must be defined");
+  EncodeSpec sp;
+  const int rc = make(in, &sp);
+  return rc != MPS_OK ? rc : no_throw([&] {
+    return encode_impl(sp, reinterpret_cast<hipStream_t>(stream), alloc, ctx, sizes17, stats4);
+  });
+}
+}  // namespace
+
+extern "C" {
+
+int mps_fp8_encode(const mps_fp8_encode_in *in, void *stream, mps_fp8_sidecar **out) {
+  return to_handle(in, fp8_spec, stream, out);
+}
+
+int mps_awq_encode(const mps_awq_encode_in *in, void *stream, mps_fp8_sidecar **out) {
+  return to_handle(in, awq_spec, stream, out);
+}
+
+int mps_fp8_encode_alloc(const mps_fp8_encode_in *in, void *stream, mps_encode_alloc alloc, void *ctx,
+                         int64_t *sizes17, int64_t *stats4) {
+  return to_alloc(in, fp8_spec, stream, alloc, ctx, sizes17, stats4);
+}
+
+int mps_awq_encode_alloc(const mps_awq_encode_in *in, void *stream, mps_encode_alloc alloc, void *ctx,
+                         int64_t *sizes17, int64_t *stats4) {
+  return to_alloc(in, awq_spec, stream, alloc, ctx, sizes17, stats4);
 }
 
 int mps_fp8_sidecar_sizes(const mps_fp8_sidecar *sc, int64_t *sizes17) {
@@ -2097,18 +2187,12 @@ int mps_fp8_sidecar_stats(const mps_fp8_sidecar *sc, int64_t *stats4) {
 int mps_fp8_sidecar_copy(const mps_fp8_sidecar *sc, void *const *dst17, void *stream) {
   last_error().clear();
   if (!sc || !dst17) return fail(MPS_ERR_INVALID_ARGUMENT, "NULL argument");
-  const void *src[17] = {sc->decode_syms.p, sc->decode_lens.p, sc->table_scale.p, sc->table_fp8.p,
-                         sc->bucket_scale.p, sc->bucket_row_offsets.p, sc->row_indices.p, sc->bucket_table.p,
-                         sc->bucket_col_start.p, sc->bucket_col_len.p, sc->bucket_thread_startbit.p,
-                         sc->bucket_bit_base.p, sc->bitstream.p, sc->shape_nmk.p, sc->bucket_U.p,
-                         sc->bucket_unique_gid.p, sc->bucket_fp8_uidx.p};
-  const int esize[17] = {2, 1, 2, 2, 2, 4, 4, 4, 4, 4, 4, 8, 8, 8, 4, 4, 2};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   for (int i = 0; i < 17; ++i) {
-    const size_t bytes = (size_t)sc->sizes[i] * esize[i];
+    const size_t bytes = (size_t)sc->sizes[i] * kOutBytes[i];
     if (bytes == 0) continue;
     if (!dst17[i]) return fail(MPS_ERR_INVALID_ARGUMENT, "NULL destination %d", i);
-    MPS_HIP_CHECK(hipMemcpyAsync(dst17[i], src[i], bytes, hipMemcpyDefault, s));
+    MPS_HIP_CHECK(hipMemcpyAsync(dst17[i], sc->out[i], bytes, hipMemcpyDefault, s));
   }
   MPS_HIP_CHECK(hipStreamSynchronize(s));
   return MPS_OK;

@@ -1,16 +1,17 @@
 """GPU sidecar builder behind MPServe_cuda.huffman_build_fp8_decode_tables.
 
 Argument checks follow the reference entry (kernel/build_huffman.cu:298-366) in
-order and wording; the work itself runs in libmpserve_amd.so (mps_fp8_encode).
+order and wording; the work itself runs in libmpserve_amd.so (mps_fp8_encode_alloc),
+straight into tensors of torch's allocator.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Dict
 
 import torch
 
 from . import _native
+from ._common import BuilderOutputs
 
 # (key, dtype) of the 17 outputs in the reference's order (kernel/wrapper.cpp:429-446)
 _OUTPUTS = (
@@ -71,28 +72,12 @@ def build_fp8_sidecar(bf16_params: torch.Tensor, fp8_params: torch.Tensor, scale
     a.scale_numel = sc.numel()
     a.max_len = int(max_len)
     a.threads_per_block = int(threads_per_block)
-    lib = _native.lib()
-    handle = ctypes.c_void_p()
+    mem = BuilderOutputs(dev, {i: dt for i, (_, dt) in enumerate(_OUTPUTS)})
     with torch.cuda.device(dev):
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        _native.check(lib.mps_fp8_encode(ctypes.byref(a), stream, ctypes.byref(handle)))
-        try:
-            sizes = (ctypes.c_int64 * 17)()
-            _native.check(lib.mps_fp8_sidecar_sizes(handle, sizes))
-            stats = (ctypes.c_int64 * 4)()
-            _native.check(lib.mps_fp8_sidecar_stats(handle, stats))
-            G = int(sizes[2])
-            B = int(sizes[4])
-            shapes = _shapes(G, B, int(threads_per_block), int(max_len), sizes)
-            out: Dict[str, torch.Tensor] = {}
-            ptrs = (ctypes.c_void_p * 17)()
-            for i, ((key, dt), shp) in enumerate(zip(_OUTPUTS, shapes)):
-                t = torch.empty(shp, dtype=dt, device="cpu" if on_host else dev)
-                out[key] = t
-                ptrs[i] = t.data_ptr() if t.numel() else None
-            _native.check(lib.mps_fp8_sidecar_copy(handle, ptrs, stream))
-        finally:
-            lib.mps_fp8_sidecar_free(handle)
+        sizes, stats = mem.build(_native.lib().mps_fp8_encode_alloc, a, torch.cuda.current_stream(dev).cuda_stream)
+        shapes = _shapes(int(sizes[2]), int(sizes[4]), int(threads_per_block), int(max_len), sizes)
+        out: Dict[str, torch.Tensor] = {key: mem.tensor(i, shp, on_host)
+                                        for i, ((key, _), shp) in enumerate(zip(_OUTPUTS, shapes))}
     if with_stats:
         return out, {"esc_keys": int(stats[0]), "esc_collisions": int(stats[1]), "distinct_pairs": int(stats[2]),
                      "hash_slots": int(stats[3])}

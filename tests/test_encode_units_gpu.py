@@ -95,3 +95,53 @@ def test_units_awq(n, m, group, k, by_scale, cap):
     assert list(got) == list(want)
     for x, v in want.items():
         assert got[x].shape == v.shape and np.array_equal(got[x].view(v.dtype), v), x
+
+
+@pytest.mark.parametrize("L", [7, 12])
+def test_handle_calls_give_the_ops_outputs(L):
+    """The C ABI's handle (its own allocations, copied out) against the op's tensors; L = 12 takes the general path."""
+    import ctypes
+
+    from mpserve_amd import _native
+    from mpserve_amd.encode import _OUTPUTS
+
+    print(f"[units] handle L {L}", flush=True)
+    bf, q, sc = (torch.from_numpy(x).to(DEV) for x in synth(300, 520, seed=3))
+    want = MPServe_cuda.huffman_build_fp8_decode_tables(bf.view(torch.bfloat16), q, sc, L, 256)
+    a = _native.MpsFp8EncodeIn()
+    a.bf16, a.fp8, a.scales, a.numel, a.ndim, a.scale_ndim = bf.data_ptr(), q.data_ptr(), sc.data_ptr(), bf.numel(), 2, 1
+    a.dims[0], a.dims[1], a.scale_dims[0], a.scale_numel, a.max_len, a.threads_per_block = 300, 520, 300, 300, L, 256
+    lib, h, sizes, ptrs = _native.lib(), ctypes.c_void_p(), (ctypes.c_int64 * 17)(), (ctypes.c_void_p * 17)()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _native.check(lib.mps_fp8_encode(ctypes.byref(a), stream, ctypes.byref(h)))
+    _native.check(lib.mps_fp8_sidecar_sizes(h, sizes))
+    got = [torch.empty(sizes[i], dtype=dt) for i, (_, dt) in enumerate(_OUTPUTS)]
+    for i, t in enumerate(got):
+        ptrs[i] = t.data_ptr()
+    _native.check(lib.mps_fp8_sidecar_copy(h, ptrs, stream))
+    _native.check(lib.mps_fp8_sidecar_free(h))
+    for (key, _), t in zip(_OUTPUTS, got):
+        assert np.array_equal(t.numpy(), want[key].cpu().numpy().reshape(-1)), key
+
+
+def test_builder_reports_no_memory():
+    """An allocator without memory ends the build with an error, and the next build works."""
+    from mpserve_amd._common import BuilderOutputs
+
+    print("[units] no memory", flush=True)
+    bf, q, sc = (torch.from_numpy(x).to(DEV) for x in synth(64, 256, seed=4))
+    real, left = BuilderOutputs._alloc, [3]
+
+    def few(self, ctx, slot, nbytes):
+        left[0] -= 1
+        return real(self, ctx, slot, nbytes) if left[0] >= 0 else None
+
+    BuilderOutputs._alloc = few
+    try:
+        with pytest.raises(MemoryError, match="no device memory"):
+            MPServe_cuda.huffman_build_fp8_decode_tables(bf.view(torch.bfloat16), q, sc, 7, 256)
+    finally:
+        BuilderOutputs._alloc = real
+    out = MPServe_cuda.huffman_build_fp8_decode_tables(bf.view(torch.bfloat16), q, sc, 7, 256)
+    want = oracle.encode(bf.cpu().numpy(), q.cpu().numpy(), sc.cpu().numpy(), 7, 256)
+    _same({x: v.cpu().numpy() for x, v in out.items()}, want)
