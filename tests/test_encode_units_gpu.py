@@ -68,6 +68,19 @@ def test_units_table_sizes(syms, qs):
     _same(_fp8(bf, q, sc, 7, 1024), oracle.encode(bf, q, sc, 7, 1024))
 
 
+@pytest.mark.parametrize("n_sym", [2, 12, 64])
+def test_short_list_with_a_count_that_could_wrap(n_sym):
+    """A key of few symbols, one of them 2.3 million times: its merge runs in sequence."""
+    print(f"[units] {n_sym} symbols, one very frequent", flush=True)
+    rng = np.random.default_rng(n_sym)
+    bf = np.full((2304, 1024), 0x3C00, dtype=np.uint16)
+    rare = rng.choice(bf.size, 5000, replace=False)
+    bf.flat[rare] = 0x3C00 + rng.integers(1, n_sym, size=rare.size) ** 2 if n_sym > 2 else 0x3C01
+    q = np.full(bf.shape, 0x40, dtype=np.uint8)
+    sc = np.array([0x1C00], dtype=np.uint16)
+    _same(_fp8(bf, q, sc, 7, 1024), oracle.encode(bf, q, sc, 7, 1024))
+
+
 @pytest.mark.parametrize("bs", [(128, 128), (64, 40), (2, 3)])
 def test_units_blocks(bs):
     print(f"[units] blocks {bs}", flush=True)
