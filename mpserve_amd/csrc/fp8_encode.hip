@@ -640,32 +640,41 @@ __global__ void codebook_kernel(CodebookArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Codebooks with a wave per key (L <= 11). The keys' histogram entries are
-// sorted for all keys at once beforehand (a segmented radix sort of the
-// (count, symbol) keys), so a key's entries arrive in (count asc, sym asc)
-// order; one 64-lane workgroup then builds its codebook in LDS, with the same
-// results as codebook_kernel:
+// Codebooks, L <= 11. A key's histogram entries arrive sorted, in (count asc,
+// sym asc) order; one workgroup builds its codebook in LDS (keys of at most 64
+// entries: one wave, codebook_small_kernel):
 //  - the ESC keep set from the sorted counts: the entry at ni - (2^L - 1) fixes
 //    the boundary count c; every entry above c's run is kept, and the run's
 //    first ones (smallest symbols) fill the rest;
 //  - esc_sym from a 65536-bit set of the symbols in LDS;
-//  - the package-merge levels built once, bottom-up, each level's outputs split
-//    over the lanes by merge path (a lane finds how many leaves precede its
-//    first output by binary search, then merges its run), keeping a leaf bit
-//    per item; the selection then counts leaf bits top-down;
+//  - the package-merge levels built once, bottom-up. A merge is a rank an item:
+//    leaf i lands after the i leaves and the packages lighter than it, package
+//    b after the b packages and the leaves no heavier (leaf first on equal
+//    weight), both found by binary search. A bit an item says whether it is a
+//    leaf; the selection then counts leaf bits top-down;
 //  - canonical codes in list order, ranked within each length by ballots;
-//  - the decode table, and each histogram entry's code word from its list
-//    position, which follows from its sorted index.
-// NMAX bounds the coded list (min(ni, 2^L)); keys outside (lo, hi] of it are
-// left to another launch.
+//  - the decode table, entry by entry (prefix minus a length's first code,
+//    below its count, is the code's rank), and each histogram entry's code word
+//    from its list position, which follows from its sorted index.
+//
+// Weights add up as the reference's ints do. A package holds a leaf at most once
+// a level, so sums stay below 11 times the key's total; a key whose sums could
+// wrap, and leave the packages unsorted, is merged in sequence by one lane, as
+// the reference merges.
+//
+// NT work-items a key: with one wave and a merge path of 32 outputs a lane,
+// lists of up to 2048 left most of a CU idle behind one long chain. Measured on
+// the 2,500 keys of a 4096 x 4096 AWQ weight: lists past 512 343 -> 142 us,
+// past 64 104 -> 62 us.
 // ---------------------------------------------------------------------------
-constexpr int kCbLanes = 64;
 constexpr int kCbSmall = 64;  // keys of at most this many entries and no ESC: codebook_small_kernel
+constexpr int kCbMaxL = 11;
 
 __device__ __forceinline__ uint32_t cb_count(uint64_t k) { return key_count(k); }
 __device__ __forceinline__ uint32_t cb_sym(uint64_t k) { return (uint32_t)(k & 0xFFFFu); }
 
-template <int NMAX>
+// NMAX bounds the coded list, min(ni, 2^L); a level holds fewer than 2 NMAX items.
+template <int NMAX, int NT>
 struct CbShared {
   int32_t lw[NMAX];   // list weights
   int32_t sw[NMAX];   // ascending weights for the package-merge (kEscAwqByScale ESC lists)
@@ -675,31 +684,44 @@ struct CbShared {
   uint8_t lens[NMAX];
   union {
     struct {
-      int32_t A[4 * NMAX];
-      int32_t B[4 * NMAX];
-      uint32_t masks[11 * (NMAX / 8) + 16];
+      int32_t cur[2 * NMAX];   // a level's items
+      int32_t pack[NMAX];      // their pairs
+      uint32_t masks[kCbMaxL * (NMAX / 16)];
     } pm;
     uint32_t symset[65536 / 32];
-    uint8_t nibs[2048];
+    uint16_t by_code[NMAX];  // list positions in code order
   } u;
-  int32_t na[16];
-  int32_t xs[16];
-  uint32_t blc[16], ncode[16], run[16];
-  uint32_t acc, acc2, flag;
+  uint32_t red[NT / 64];
+  uint32_t cnt[NT / 64][16];  // a wave's items of each length
+  uint32_t flag;
 };
 
-// Sum over the workgroup's 64 lanes (one wave), returned to every lane.
-__device__ __forceinline__ uint32_t cb_sum(uint32_t v) {
+// Sum and minimum over the workgroup, returned to every work-item (two barriers).
+template <int NT>
+__device__ __forceinline__ uint32_t cb_sum(uint32_t *red, uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o);
+  if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) v += red[w];
+  __syncthreads();
   return v;
 }
-__device__ __forceinline__ uint32_t cb_min(uint32_t v) {
+template <int NT>
+__device__ __forceinline__ uint32_t cb_min(uint32_t *red, uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const uint32_t w = (uint32_t)__shfl_xor((int)v, o);
     v = w < v ? w : v;
   }
+  if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = red[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) v = red[w] < v ? red[w] : v;
+  __syncthreads();
   return v;
 }
 
@@ -715,11 +737,11 @@ __device__ __forceinline__ uint32_t cb_bound(const uint64_t *k, uint32_t lo, uin
   return lo;
 }
 
-template <int NMAX>
-__device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookArgs &a, uint32_t g,
-                                              const uint64_t *__restrict__ skeys,
-                                              const uint32_t *__restrict__ sslots) {
-  const int lane = threadIdx.x;
+template <int NMAX, int NT>
+__device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const CodebookArgs &a, uint32_t g,
+                                             const uint64_t *__restrict__ skeys,
+                                             const uint32_t *__restrict__ sslots) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const int L = a.L;
   const uint32_t T = 1u << L;
   const uint32_t tk = a.gid_tkey[g];
@@ -727,17 +749,12 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
   const uint32_t ni = a.tcount[tk];
   const uint64_t *keys = skeys + off;
   auto slot_of = [&](uint32_t t) { return sslots ? sslots[off + t] : off + t; };
-  uint16_t *dsyms = a.decode_syms + (uint64_t)g * T;
-  uint8_t *dlens = a.decode_lens + (uint64_t)g * (T / 2 > 0 ? T / 2 : 1);
-  if (lane == 0) {
+  uint32_t *dsyms = reinterpret_cast<uint32_t *>(a.decode_syms + (uint64_t)g * T);  // pairs of entries
+  uint8_t *dlens = a.decode_lens + (uint64_t)g * (T / 2);
+  if (tid == 0) {
     a.table_scale[g] = a.scale_values[tk >> 8];
     a.table_fp8[g] = (uint16_t)(tk & 0xFF);
-  }
-  if (ni == 1) {
-    for (uint32_t j = lane; j < T; j += kCbLanes) dsyms[j] = (uint16_t)cb_sym(keys[0]);
-    for (uint32_t j = lane; j < T / 2; j += kCbLanes) dlens[j] = 0x11;  // len 1 in both nibbles
-    if (lane == 0) a.cw_slot[slot_of(0)] = (1u << 16) | 0u;
-    return;
+    S.flag = 0;
   }
 
   // --- the coded list ---
@@ -746,7 +763,7 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
   uint32_t nl, s0 = 0, s1 = 0, r = 0, esc_sym = 0, esc_pos = 0;
   int32_t esc_w = 0;
   if (!use_esc) {
-    for (uint32_t p = lane; p < ni; p += kCbLanes) {
+    for (uint32_t p = tid; p < ni; p += NT) {
       const uint64_t k = keys[p];
       S.lw[p] = (int32_t)cb_count(k);
       S.ls[p] = (uint16_t)cb_sym(k);
@@ -760,19 +777,19 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
     s1 = cb_bound(keys, s0, ni, c, true);
     r = keep - (ni - s1);
     uint32_t tot = 0, kept = 0;
-    for (uint32_t t = lane; t < ni; t += kCbLanes) {
+    for (uint32_t t = tid; t < ni; t += NT) {
       const uint32_t cnt = cb_count(keys[t]);
       tot += cnt;
       kept += (t >= s1 || (t >= s0 && t < s0 + r)) ? cnt : 0u;
     }
-    tot = cb_sum(tot);
-    kept = cb_sum(kept);
+    tot = cb_sum<NT>(S.red, tot);
+    kept = cb_sum<NT>(S.red, kept);
     const uint32_t ew = tot - kept;  // int sums as in the reference
     // esc_sym: the smallest u16 absent from the key's symbols (kEscAwqByScale) or
     // from the kept ones (the other builders)
-    for (uint32_t i = lane; i < 65536 / 32; i += kCbLanes) S.u.symset[i] = 0u;
+    for (uint32_t i = tid; i < 65536 / 32; i += NT) S.u.symset[i] = 0u;
     __syncthreads();
-    for (uint32_t t = lane; t < ni; t += kCbLanes) {
+    for (uint32_t t = tid; t < ni; t += NT) {
       const bool in = a.esc_mode == kEscAwqByScale || t >= s1 || (t >= s0 && t < s0 + r);
       if (in) {
         const uint32_t sy = cb_sym(keys[t]);
@@ -781,18 +798,18 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
     }
     __syncthreads();
     uint32_t cand = 0xFFFFFFFFu;
-    for (uint32_t i = lane; i < 65536 / 32; i += kCbLanes) {
+    for (uint32_t i = tid; i < 65536 / 32; i += NT) {
       const uint32_t wv = ~S.u.symset[i];
       if (wv != 0u && cand == 0xFFFFFFFFu) cand = 32u * i + (uint32_t)__builtin_ctz(wv);
     }
-    cand = cb_min(cand);
+    cand = cb_min<NT>(S.red, cand);
     __syncthreads();
     if (a.esc_mode == kEscAwqByScale) {
       esc_sym = cand == 0xFFFFFFFFu ? 0xFFFFu : cand;
       esc_w = (int32_t)ew;
       // (count desc, sym asc), ESC last: an entry of a run [g0, g1) above c sits
       // at (ni - g1) + (t - g0); the boundary run's first r follow them
-      for (uint32_t t = lane; t < ni; t += kCbLanes) {
+      for (uint32_t t = tid; t < ni; t += NT) {
         uint32_t pos;
         if (t >= s1) {
           const uint32_t cc = cb_count(keys[t]);
@@ -814,17 +831,17 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
       uint32_t e_pos = 0;
       {
         uint32_t below = 0;  // kept counts < the ESC weight (as int)
-        for (uint32_t j = lane; j < keep; j += kCbLanes) {
+        for (uint32_t j = tid; j < keep; j += NT) {
           const uint32_t t = j < r ? s0 + j : s1 + (j - r);
           below += (int32_t)cb_count(keys[t]) < esc_w ? 1u : 0u;
         }
-        e_pos = cb_sum(below);
+        e_pos = cb_sum<NT>(S.red, below);
       }
-      for (uint32_t j = lane; j < keep; j += kCbLanes) {
+      for (uint32_t j = tid; j < keep; j += NT) {
         const uint32_t t = j < r ? s0 + j : s1 + (j - r);
         S.sw[j + (j >= e_pos ? 1u : 0u)] = (int32_t)cb_count(keys[t]);
       }
-      if (lane == 0) {
+      if (tid == 0) {
         S.sw[e_pos] = esc_w;
         S.lw[keep] = esc_w;
         S.ls[keep] = (uint16_t)esc_sym;
@@ -838,12 +855,12 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
       // inserted at its key's place
       const uint64_t ek = item_key((uint32_t)esc_w, esc_sym);
       uint32_t below = 0;
-      for (uint32_t j = lane; j < keep; j += kCbLanes) {
+      for (uint32_t j = tid; j < keep; j += NT) {
         const uint32_t t = j < r ? s0 + j : s1 + (j - r);
         below += item_key(cb_count(keys[t]), cb_sym(keys[t])) < ek ? 1u : 0u;
       }
-      esc_pos = cb_sum(below);
-      for (uint32_t j = lane; j < keep; j += kCbLanes) {
+      esc_pos = cb_sum<NT>(S.red, below);
+      for (uint32_t j = tid; j < keep; j += NT) {
         const uint32_t t = j < r ? s0 + j : s1 + (j - r);
         const uint32_t p = j + (j >= esc_pos ? 1u : 0u);
         const uint64_t k = keys[t];
@@ -851,172 +868,199 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
         S.ls[p] = (uint16_t)cb_sym(k);
         S.hidx[p] = (int32_t)t;
       }
-      if (lane == 0) {
+      if (tid == 0) {
         S.lw[esc_pos] = esc_w;
         S.ls[esc_pos] = (uint16_t)esc_sym;
         S.hidx[esc_pos] = -1;
       }
     }
     nl = T;
-    if (lane == 0) atomicAdd(&a.esc_stats[0], 1u);
+    if (tid == 0) atomicAdd(&a.esc_stats[0], 1u);
   }
   __syncthreads();
 
   // --- package-merge lengths (see package_merge_lengths) ---
+  const int32_t *W = (use_esc && a.esc_mode == kEscAwqByScale) ? S.sw : S.lw;
+  const uint32_t n = nl, keep_pm = 4u * (n - 1u);
+  uint32_t xs[kCbMaxL];  // leaves among each level's selected prefix
   {
-    const int32_t *W = (use_esc && a.esc_mode == kEscAwqByScale) ? S.sw : S.lw;
-    const int n = (int)nl;
-    const int keep_pm = 4 * (n - 1);
-    const int words = (keep_pm + 31) / 32;
-    int32_t *A = S.u.pm.A, *B = S.u.pm.B;
-    int cur = n < keep_pm ? n : keep_pm;
-    for (int i = lane; i < cur; i += kCbLanes) A[i] = W[i];
-    for (int i = lane; i < words; i += kCbLanes) {
-      const int b = cur - 32 * i;
-      S.u.pm.masks[i] = b >= 32 ? 0xFFFFFFFFu : (b > 0 ? (1u << b) - 1u : 0u);
+    uint32_t sum = 0;
+    for (uint32_t i = tid; i < n; i += NT) sum += (uint32_t)W[i];
+    const bool wraps = cb_sum<NT>(S.red, sum) >= (1u << 31) / 12u;
+    int32_t *cur = S.u.pm.cur, *pack = S.u.pm.pack;
+    uint32_t have = n < keep_pm ? n : keep_pm;
+    uint32_t sizes[kCbMaxL];
+    constexpr uint32_t kWords = NMAX / 16;  // of a level's mask
+    for (uint32_t i = tid; i < have; i += NT) cur[i] = W[i];
+    for (uint32_t i = tid; i < kWords; i += NT) {
+      const uint32_t lo = 32u * i;
+      S.u.pm.masks[i] = have >= lo + 32u ? 0xFFFFFFFFu : have > lo ? (1u << (have - lo)) - 1u : 0u;
     }
-    if (lane == 0) S.na[0] = cur;
+    sizes[0] = have;
     __syncthreads();
-    for (int j = 1; j < L; ++j) {
-      const int np = cur / 2;
-      const int o = keep_pm < n + np ? keep_pm : n + np;
-      const int chunk = (((o + kCbLanes - 1) / kCbLanes) + 31) & ~31;  // whole mask words per lane
-      const int k0 = lane * chunk;
-      const int k1 = k0 + chunk < o ? k0 + chunk : o;
-      uint32_t *mk = S.u.pm.masks + j * words;
-      if (k0 < k1) {
-        // leaves among the first k0 outputs: the largest a with leaf a-1 before package k0-a
-        int lo = k0 - np > 0 ? k0 - np : 0, hi = k0 < n ? k0 : n;
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          const int b = k0 - mid;
-          const bool ok = b >= np || W[mid - 1] <= (int32_t)((uint32_t)A[2 * b] + (uint32_t)A[2 * b + 1]);
-          if (ok) lo = mid;
-          else hi = mid - 1;
+#pragma unroll
+    for (int j = 1; j < kCbMaxL; ++j) {
+      sizes[j] = 0;
+      if (j >= L) continue;
+      const uint32_t np = have / 2u;
+      uint32_t *mk = S.u.pm.masks + j * kWords;
+      for (uint32_t b = tid; b < np; b += NT) pack[b] = (int32_t)((uint32_t)cur[2u * b] + (uint32_t)cur[2u * b + 1u]);
+      for (uint32_t i = tid; i < kWords; i += NT) mk[i] = 0u;
+      __syncthreads();
+      have = n + np < keep_pm ? n + np : keep_pm;
+      sizes[j] = have;
+      if (wraps) {
+        if (tid == 0) {
+          for (uint32_t o = 0, x = 0, b = 0; o < have; ++o) {
+            if (x < n && (b >= np || W[x] <= pack[b])) {
+              cur[o] = W[x++];
+              mk[o >> 5] |= 1u << (o & 31u);
+            } else {
+              cur[o] = pack[b++];
+            }
+          }
         }
-        int ai = lo, bi = k0 - lo;
-        uint32_t bits = 0;
-        for (int k = k0; k < k1; ++k) {
-          const int32_t pw = bi < np ? (int32_t)((uint32_t)A[2 * bi] + (uint32_t)A[2 * bi + 1]) : 0;
-          const bool leaf = ai < n && (bi >= np || W[ai] <= pw);
-          B[k] = leaf ? W[ai] : pw;
-          ai += leaf ? 1 : 0;
-          bi += leaf ? 0 : 1;
-          bits |= (leaf ? 1u : 0u) << (k & 31);
-          if ((k & 31) == 31 || k + 1 == k1) {
-            mk[k >> 5] = bits;
-            bits = 0;
+      } else {
+        for (uint32_t i = tid; i < n + np; i += NT) {
+          const bool leaf = i < n;
+          const uint32_t at = leaf ? i : i - n;
+          const int32_t v = leaf ? W[at] : pack[at];
+          uint32_t lo = 0, hi = leaf ? np : n;
+          const int32_t *other = leaf ? pack : W;
+          while (lo < hi) {  // packages lighter than this leaf, or leaves no heavier than this package
+            const uint32_t mid = (lo + hi) >> 1;
+            const int32_t x = other[mid];
+            if (leaf ? x < v : x <= v) lo = mid + 1u;
+            else hi = mid;
+          }
+          const uint32_t to = at + lo;
+          if (to < have) {
+            cur[to] = v;
+            if (leaf) atomicOr(&mk[to >> 5], 1u << (to & 31u));
           }
         }
       }
       __syncthreads();
-      int32_t *t = A;
-      A = B;
-      B = t;
-      cur = o;
-      if (lane == 0) S.na[j] = o;
     }
-    __syncthreads();
-    // top-down: leaves among each level's selected prefix
-    int c = 2 * (n - 1);
-    int nx = 0;
-    for (int level = L - 1; level >= 0 && c > 0; --level) {
-      const int cc = c < S.na[level] ? c : S.na[level];
-      const uint32_t *mk = S.u.pm.masks + level * words;
+    // top-down, by every wave for itself
+    uint32_t c = 2u * (n - 1u);
+#pragma unroll
+    for (int j = kCbMaxL - 1; j >= 0; --j) {
+      xs[j] = 0;
+      if (j >= L || c == 0u) continue;
+      const uint32_t cc = c < sizes[j] ? c : sizes[j];
+      const uint32_t *mk = S.u.pm.masks + j * kWords;
       uint32_t x = 0;
-      for (int i = lane; i < (cc + 31) / 32; i += kCbLanes) {
-        const uint32_t wv = mk[i];
-        const int rem = cc - 32 * i;
-        x += __popc(rem >= 32 ? wv : (wv & ((1u << rem) - 1u)));
+      for (uint32_t i = lane; i < (cc + 31u) / 32u; i += 64u) {
+        const uint32_t rem = cc - 32u * i;
+        x += (uint32_t)__popc(rem >= 32u ? mk[i] : (mk[i] & ((1u << rem) - 1u)));
       }
-      x = cb_sum(x);
-      if (lane == 0) S.xs[nx] = (int32_t)x;
-      ++nx;
-      c = 2 * (cc - (int)x);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) x += (uint32_t)__shfl_xor((int)x, o);
+      xs[j] = x;
+      c = 2u * (cc - x);
     }
-    __syncthreads();
-    for (int i = lane; i < n; i += kCbLanes) {
-      int len = 0;
-      for (int q = 0; q < nx; ++q) len += i < S.xs[q] ? 1 : 0;
-      S.lens[i] = (uint8_t)len;
-    }
-    if (lane < 16) {
-      S.blc[lane] = 0;
-      S.run[lane] = 0;
-    }
-    if (lane == 0) S.flag = 0;
-    __syncthreads();
   }
 
   // --- canonical codes (build_huffman.cu:171-203), handed out in list order ---
-  for (uint32_t p = lane; p < nl; p += kCbLanes) {
-    int len = S.lens[p];
-    if (len <= 0 || len > L) {
-      S.flag = 1;
-      continue;
+  // Wave w has the items [w * per, + per): counts first, then codes.
+  const uint32_t per = (n + NT - 1u) / NT * 64u;
+  const uint32_t p0 = wave * per, p1 = p0 + per < n ? p0 + per : n;
+  uint32_t mine = 0;  // lane v: this wave's items of length v
+  for (uint32_t b = p0; b < p1; b += 64u) {
+    const uint32_t p = b + lane;
+    int len = 0;
+    if (p < p1) {
+#pragma unroll
+      for (int j = 0; j < kCbMaxL; ++j) len += p < xs[j] ? 1 : 0;
+      if (len <= 0 || len > L) S.flag = 1;
+      if (use_esc && a.esc_mode != kEscFp8 && (uint32_t)S.ls[p] == esc_sym) len = L;  // AWQ: ESC code has length L
+      S.lens[p] = (uint8_t)len;
     }
-    if (use_esc && a.esc_mode != kEscFp8 && (uint32_t)S.ls[p] == esc_sym) {  // AWQ: ESC code has length L
-      len = L;
-      S.lens[p] = (uint8_t)L;
+#pragma unroll
+    for (int v = 1; v <= kCbMaxL; ++v) {
+      const uint32_t c = (uint32_t)__popcll(__ballot(len == v));
+      mine += lane == (uint32_t)v ? c : 0u;
     }
-    atomicAdd(&S.blc[len], 1u);
   }
-  __syncthreads();
+  if (lane < 16u) S.cnt[wave][lane] = mine;
+  __syncthreads();  // (the masks are read: by_code may take their place)
   if (S.flag) {
-    if (lane == 0) atomicOr(a.err, 2u);
+    if (tid == 0) atomicOr(a.err, 2u);
     return;
   }
-  if (lane == 0) {
-    uint32_t cd = 0;
-    S.ncode[0] = 0;
-    for (int b = 1; b < 16; ++b) {
-      cd = (cd + S.blc[b - 1]) << 1;
-      S.ncode[b] = cd;
+  uint32_t all = 0, before = 0;  // lane v: items of length v in all, and in the waves before
+  if (lane < 16u) {
+#pragma unroll
+    for (uint32_t w = 0; w < NT / 64; ++w) {
+      const uint32_t c = S.cnt[w][lane];
+      all += c;
+      before += w < wave ? c : 0u;
     }
   }
-  __syncthreads();
-  for (uint32_t base = 0; base < nl; base += kCbLanes) {
-    const uint32_t p = base + lane;
-    const int len = p < nl ? S.lens[p] : 0;
-    uint32_t rank = 0, mine = 0;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int v = 1; v <= L; ++v) {
+  uint32_t first[kCbMaxL + 1], num[kCbMaxL + 1], base[kCbMaxL + 1];  // of a length: first code, codes, codes before it
+  first[0] = num[0] = base[0] = 0;
+  uint32_t next = 0, at_code = 0;  // lane v: the wave's next code of length v, and its place in code order
+#pragma unroll
+  for (int v = 1; v <= kCbMaxL; ++v) {
+    num[v] = (uint32_t)__builtin_amdgcn_readlane((int)all, v);
+    first[v] = (first[v - 1] + num[v - 1]) << 1;
+    base[v] = base[v - 1] + num[v - 1];
+    if (lane == (uint32_t)v) {
+      next = first[v] + before;
+      at_code = base[v] + before;
+    }
+  }
+  const uint64_t below = lane == 0u ? 0ull : (~0ull >> (64u - lane));
+  for (uint32_t b = p0; b < p1; b += 64u) {
+    const uint32_t p = b + lane;
+    const int len = p < p1 ? S.lens[p] : 0;
+    uint32_t rank = 0, got = 0;
+#pragma unroll
+    for (int v = 1; v <= kCbMaxL; ++v) {
       const uint64_t m = __ballot(len == v);
       if (len == v) rank = (uint32_t)__popcll(m & below);
-      if (lane == v) mine = (uint32_t)__popcll(m);  // lane v keeps length v's count of this chunk
+      if (lane == (uint32_t)v) got = (uint32_t)__popcll(m);
     }
-    if (p < nl) S.code[p] = (uint16_t)(S.ncode[len] + S.run[len] + rank);
-    __syncthreads();
-    if (lane >= 1 && lane <= L) S.run[lane] += mine;
-    __syncthreads();
+    const uint32_t c = (uint32_t)__shfl((int)next, len) + rank, at = (uint32_t)__shfl((int)at_code, len) + rank;
+    if (p < p1) {
+      S.code[p] = (uint16_t)c;
+      S.u.by_code[at] = (uint16_t)p;
+    }
+    next += got;
+    at_code += got;
   }
+  __syncthreads();
 
-  // --- decode table ---
-  for (uint32_t j = lane; j < T; j += kCbLanes) {
-    dsyms[j] = 0;
-    S.u.nibs[j] = 0;
-  }
-  __syncthreads();
-  uint32_t esc_cw = 0;
-  for (uint32_t p = lane; p < nl; p += kCbLanes) {
-    const uint32_t len = S.lens[p];
-    const uint32_t c = S.code[p];
-    const bool is_esc = use_esc && (uint32_t)S.ls[p] == esc_sym;
-    const uint32_t nib = is_esc ? (a.esc_mode == kEscFp8 ? (len | 0x8u) : 15u) : len;
-    const uint32_t fill = 1u << (L - len);
-    const uint32_t base = c << (L - len);
-    for (uint32_t f = 0; f < fill; ++f) {
-      dsyms[base + f] = S.ls[p];
-      S.u.nibs[base + f] = (uint8_t)nib;
+  // --- decode table, two entries a work-item ---
+  for (uint32_t p = tid; p < T / 2u; p += NT) {
+    uint32_t s2 = 0, l2 = 0;
+#pragma unroll
+    for (uint32_t h = 0; h < 2u; ++h) {
+      const uint32_t e = 2u * p + h;
+      uint32_t at = 0, len = 0;
+#pragma unroll
+      for (int v = 1; v <= kCbMaxL; ++v) {
+        const uint32_t r = v <= L ? (e >> (L - v)) - first[v] : ~0u;  // wraps when the prefix lies below
+        if (r < num[v]) {
+          at = base[v] + r;
+          len = (uint32_t)v;
+        }
+      }
+      if (len) {
+        const uint32_t sy = S.ls[S.u.by_code[at]];
+        const uint32_t nib = use_esc && sy == esc_sym ? (a.esc_mode == kEscFp8 ? (len | 0x8u) : 15u) : len;
+        s2 |= sy << (16u * h);
+        l2 |= (nib & 0xFu) << (4u * h);
+      }
     }
+    dsyms[p] = s2;
+    dlens[p] = (uint8_t)l2;
   }
-  if (use_esc) esc_cw = ((uint32_t)S.lens[esc_pos] << 16) | (S.code[esc_pos] & 0xFFFFu);
-  __syncthreads();
-  for (uint32_t j = lane; j < (T / 2 > 0 ? T / 2 : 1); j += kCbLanes)
-    dlens[j] = T >= 2 ? (uint8_t)((S.u.nibs[2 * j] & 0xF) | ((S.u.nibs[2 * j + 1] & 0xF) << 4)) : 0;
+  const uint32_t esc_cw = use_esc ? ((uint32_t)S.lens[esc_pos] << 16) | (S.code[esc_pos] & 0xFFFFu) : 0u;
 
   // --- code word of every histogram entry, from its list position ---
-  for (uint32_t t = lane; t < ni; t += kCbLanes) {
+  for (uint32_t t = tid; t < ni; t += NT) {
     int32_t p = -1;
     if (!use_esc) {
       p = (int32_t)t;
@@ -1048,25 +1092,23 @@ __device__ __forceinline__ void codebook_wave(CbShared<NMAX> &S, const CodebookA
   }
 }
 
-// The codebooks of the *n keys in `list` (one of the three size classes).
-template <int NMAX>
-__global__ __launch_bounds__(kCbLanes) void codebook_wave_kernel(CodebookArgs a, const uint64_t *__restrict__ skeys,
-                                                                 const uint32_t *__restrict__ sslots,
-                                                                 const uint32_t *__restrict__ list,
-                                                                 const uint32_t *__restrict__ n) {
-  __shared__ CbShared<NMAX> S;
+// The codebooks of the *n keys in `list` (a size class).
+template <int NMAX, int NT>
+__global__ __launch_bounds__(NT) void codebook_key_kernel(CodebookArgs a, const uint64_t *__restrict__ skeys,
+                                                          const uint32_t *__restrict__ sslots,
+                                                          const uint32_t *__restrict__ list,
+                                                          const uint32_t *__restrict__ n) {
+  __shared__ CbShared<NMAX, NT> S;
   const uint32_t count = *n;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    codebook_wave<NMAX>(S, a, list[i], skeys, sslots);
+    codebook_key<NMAX, NT>(S, a, list[i], skeys, sslots);
     __syncthreads();
   }
 }
 
 // Keys of at most 64 entries and no ESC (of an FP8 weight's keys nearly all: a
 // normal bin of 8 holds 16 symbols), a wave a key and a list item a lane, held
-// in registers. codebook_wave_kernel's merge path gives a lane 32 outputs, so
-// one or two lanes walked a short list alone; here a level's merge is a rank a
-// lane: leaf i lands after the i leaves and the packages lighter than it,
+// in registers: a level's merge is a rank a lane, leaf i lands after the i leaves and the packages lighter than it,
 // package b after the b packages and the leaves no heavier (leaf first on equal
 // weight), both by binary search in LDS. The leaves' places stay in registers,
 // so the selection counts them with a ballot a level, and the canonical codes
@@ -1084,7 +1126,7 @@ __global__ __launch_bounds__(64 * kCbWaves) void codebook_small_kernel(CodebookA
                                                                        const uint32_t *__restrict__ sslots,
                                                                        const uint32_t *__restrict__ list,
                                                                        const uint32_t *__restrict__ n_list) {
-  constexpr int kMaxL = 11;
+  constexpr int kMaxL = kCbMaxL;
   __shared__ int32_t s_leaf[kCbWaves][64], s_pack[kCbWaves][64], s_cur[kCbWaves][128];
   __shared__ uint32_t s_sym[kCbWaves][64];  // symbols in code order
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -1480,14 +1522,14 @@ __global__ void pack_kernel(PackArgs a) {
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
-// The three codebook launches, a wave per key of each size class.
+// The three codebook launches, one a size class.
 void launch_codebooks(const CodebookArgs &cba, const uint64_t *skeys, const uint32_t *sslots, const uint32_t *lists,
                       uint32_t cap, const uint32_t *n3, uint32_t most, hipStream_t s) {
   hipLaunchKernelGGL(codebook_small_kernel, dim3(std::min((most + kCbWaves - 1) / kCbWaves, 2048u)),
                      dim3(64 * kCbWaves), 0, s, cba, skeys, sslots, lists, n3);
-  hipLaunchKernelGGL(codebook_wave_kernel<512>, dim3(std::min(most, 1280u)), dim3(kCbLanes), 0, s, cba, skeys, sslots,
+  hipLaunchKernelGGL((codebook_key_kernel<512, 256>), dim3(std::min(most, 2048u)), dim3(256), 0, s, cba, skeys, sslots,
                      lists + cap, n3 + 1);
-  hipLaunchKernelGGL(codebook_wave_kernel<2048>, dim3(std::min(most, 256u)), dim3(kCbLanes), 0, s, cba, skeys, sslots,
+  hipLaunchKernelGGL((codebook_key_kernel<2048, 512>), dim3(std::min(most, 512u)), dim3(512), 0, s, cba, skeys, sslots,
                      lists + 2 * (size_t)cap, n3 + 2);
 }
 
@@ -2035,9 +2077,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     if ((rc = alloc_tables()) != MPS_OK) return rc;
     HC(cw_slot.alloc(cap));
     // Codebooks. L <= 11 (the FP8 and AWQ formats): the keys' histogram entries
-    // are sorted for all keys at once, then a wave per key builds each codebook in
-    // LDS (codebook_wave_kernel; one launch for lists of up to 512 items, one for
-    // the larger). Longer codes (L up to 15, reachable through the op's max_len)
+    // are sorted for all keys at once, then built in LDS (launch_codebooks).
+    // Longer codes (L up to 15, reachable through the op's max_len)
     // keep the work-item-per-key kernel and its global workspace.
     const bool wave_cb = L <= 11;
     DevBuf<uint64_t> keys_in, keys_sorted;
