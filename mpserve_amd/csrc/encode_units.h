@@ -22,8 +22,8 @@
 // Measured against one work-item a substream over a hash table in global
 // memory (the general path of fp8_encode.hip, for the calls this one does not
 // take), one 14336 x 4096 FP8 weight, k = 1024: counting 1.89 ms -> 69 us,
-// grouping and sorting 1.38 ms -> 80 us, code words and bits 1.60 ms -> 101 us,
-// packing 0.57 -> 0.09 ms; the whole call 10.7 -> 0.8 ms with the host side of fp8_encode.hip.
+// grouping and sorting 1.38 ms -> 58 us, code words and bits 1.60 ms -> 92 us,
+// packing 0.57 -> 0.085 ms; the whole call 10.7 -> 0.6 ms with the host side of fp8_encode.hip.
 #pragma once
 
 constexpr int kUnitThreads = 1024;
@@ -169,8 +169,9 @@ __global__ __launch_bounds__(kUnitThreads) void unit_hist(UnitArgs a, const uint
 // [p * qvals / parts, (p + 1) * qvals / parts), added up over the scale's unit
 // lists and sorted by (q, count as int, symbol) into skeys[part_off ..]; the
 // keys' entry counts and first entries (tcount, toff, indexed s * 256 + q).
-// Sorted in LDS (bitonic, over the pairs found), which bounds it; the parts
-// keep the sorts short and the workgroups many when the scales are few.
+// The parts keep the sorts short and the workgroups many when the scales are
+// few. Measured on 14336 x 4096: 66 us with a list a wave, a load at a time, and
+// a barrier a sorting step; 43 us as below (1024 x 4096: 34 -> 26 us).
 __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__restrict__ scale_unit_off,
                                                             const uint32_t *__restrict__ unit_of_scale,
                                                             const uint32_t *__restrict__ list_off,
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__re
                                                             uint32_t *__restrict__ toff, uint32_t *__restrict__ part_n,
                                                             uint32_t *__restrict__ part_keys, uint32_t *overflow) {
   __shared__ __attribute__((aligned(16))) uint32_t s_pairs[2 * kPairSlots];
-  __shared__ uint32_t s_n, s_keys;
+  __shared__ uint32_t s_len[kUnitThreads], s_off[kUnitThreads], s_n, s_keys;
   uint32_t *s_key = s_pairs, *s_cnt = s_pairs + kPairSlots;
   uint64_t *s_sort = reinterpret_cast<uint64_t *>(s_pairs);
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -193,15 +194,42 @@ __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__re
   }
   if (tid == 0) s_n = s_keys = 0u;
   __syncthreads();
+  // The lists in chunks of 512 entries dealt to the waves, eight loads a lane in
+  // flight; 1024 lists' lengths at a time in LDS.
   bool ok = true;
-  for (uint32_t i = scale_unit_off[s] + wave; i < scale_unit_off[s + 1]; i += kUnitThreads / 64) {
-    const uint32_t u = unit_of_scale[i];
-    const uint32_t n = list_n[u];
-    const uint2 *l = lists + list_off[u];
-    for (uint32_t j = lane; j < n; j += 64u) {
-      const uint2 e = l[j];
-      const uint32_t q = e.x >> 16;
-      if (q >= q0 && q < q1) ok &= pair_add(s_key, s_cnt, e.x, e.y);
+  const uint32_t first_list = scale_unit_off[s], num_lists = scale_unit_off[s + 1] - first_list;
+  for (uint32_t l0 = 0; l0 < num_lists; l0 += kUnitThreads) {
+    const uint32_t nl = num_lists - l0 < kUnitThreads ? num_lists - l0 : kUnitThreads;
+    if (l0) __syncthreads();
+    if (tid < nl) {
+      const uint32_t u = unit_of_scale[first_list + l0 + tid];
+      s_len[tid] = list_n[u];
+      s_off[tid] = list_off[u];
+    }
+    __syncthreads();
+    uint32_t l = 0, chunk = wave;  // the wave's chunk: chunk `chunk` of list l
+    for (;;) {
+      uint32_t chunks = 0;
+      while (l < nl && chunk >= (chunks = (s_len[l] + 511u) >> 9)) {
+        chunk -= chunks;
+        ++l;
+      }
+      if (l >= nl) break;
+      const uint2 *from = lists + s_off[l];
+      const uint32_t n = s_len[l];
+      uint2 e[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8u; ++j) {
+        const uint32_t at = (chunk << 9) + (j << 6) + lane;
+        e[j] = from[at < n ? at : 0u];
+        if (at >= n) e[j].x = kNoPair;  // (no q range holds it)
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 8u; ++j) {
+        const uint32_t q = e[j].x >> 16;
+        if (q >= q0 && q < q1) ok &= pair_add(s_key, s_cnt, e[j].x, e[j].y);
+      }
+      chunk += kUnitThreads / 64;
     }
   }
   if (!ok) atomicOr(overflow, 1u);
@@ -226,12 +254,30 @@ __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__re
   }
   __syncthreads();
   const uint32_t n = s_n;
-  uint32_t np = 1;
+  uint32_t np = 64;
   while (np < n) np <<= 1;
   for (uint32_t i = n + tid; i < np; i += kUnitThreads) s_sort[i] = ~0ull;
   __syncthreads();
-  for (uint32_t size = 2; size <= np; size <<= 1) {
-    for (uint32_t d = size >> 1; d > 0; d >>= 1) {
+  // Bitonic: the steps of distance below 64 in a wave's registers, 64 entries at
+  // a time, the others in LDS with a barrier each.
+  auto in_wave = [&](uint32_t size_from, uint32_t size_to) {
+    for (uint32_t b = wave * 64u; b < np; b += kUnitThreads) {
+      uint64_t x = s_sort[b + lane];
+      for (uint32_t size = size_from; size <= size_to; size <<= 1) {
+        const bool up = ((b + lane) & size) == 0u;
+        for (uint32_t d = size < 64u ? size >> 1 : 32u; d > 0; d >>= 1) {
+          const uint64_t y = (uint64_t)__shfl_xor((unsigned long long)x, (int)d);
+          const bool low = (lane & d) == 0u;
+          if ((y < x) == (low == up)) x = y;  // the low lane keeps the smaller (going up)
+        }
+      }
+      s_sort[b + lane] = x;
+    }
+    __syncthreads();
+  };
+  in_wave(2u, 64u);
+  for (uint32_t size = 128; size <= np; size <<= 1) {
+    for (uint32_t d = size >> 1; d >= 64u; d >>= 1) {
       for (uint32_t i = tid; i < np / 2; i += kUnitThreads) {
         const uint32_t x = ((i & ~(d - 1u)) << 1) | (i & (d - 1u)), y = x + d;
         const uint64_t vx = s_sort[x], vy = s_sort[y];
@@ -242,6 +288,7 @@ __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__re
       }
       __syncthreads();
     }
+    in_wave(size, size);
   }
   const uint32_t off = part_off[blockIdx.x];
   for (uint32_t i = tid; i < n; i += kUnitThreads) skeys[off + i] = s_sort[i];
@@ -372,17 +419,27 @@ __global__ __launch_bounds__(kUnitThreads) void unit_codes(UnitArgs a, uint32_t 
   uint32_t bits = 0;
   bool found = true;
   uint16_t *out = codes + bucket_elem[u.bucket];
+  // The piece's element, its row (from the unit's first) and column: a step is the
+  // same for every work-item, plus a carry. (A division an element bounded the pass.)
+  const uint32_t dr = g.k_eff / g.cl, dc = g.k_eff - dr * g.cl;
+  uint32_t at = pc.lane + pc.i * g.k_eff;
+  uint32_t row = at / g.cl, col = at - row * g.cl;
+  row -= g.r0;
   constexpr int kB = 8;  // elements in flight a work-item
   for (uint32_t i = pc.i; i < pc.iend; i += kB) {
     uint32_t pair[kB], e[kB];
 #pragma unroll
     for (int j = 0; j < kB; ++j) {
-      e[j] = pc.lane + (i + j) * g.k_eff;
-      const bool in = i + j < pc.iend && e[j] < g.e1;
-      const uint32_t ee = in ? e[j] : g.e0;  // past the end: the unit's first element, not stored
-      e[j] = in ? e[j] : kNoPair;
-      const uint32_t r = ee / g.cl;
-      const uint32_t idx = s_base[r - g.r0] + (ee - r * g.cl);
+      const bool in = i + j < pc.iend && at < g.e1;
+      e[j] = in ? at : kNoPair;
+      // past the end: the unit's first row, not stored
+      const uint32_t idx = s_base[in ? row : 0u] + (in ? col : 0u);
+      at += g.k_eff;
+      row += dr;
+      col += dc;
+      const bool carry = col >= g.cl;
+      row += carry ? 1u : 0u;
+      col -= carry ? g.cl : 0u;
       pair[j] = ((uint32_t)(a.q[idx] & a.qmask) << 16) | a.bf16[idx];
     }
 #pragma unroll
@@ -475,6 +532,11 @@ __global__ __launch_bounds__(kScanBlock) void bucket_bases(const uint32_t *__res
 // with neighbouring units on one XCD (below); 4096 x 4096 AWQ 157 -> 32 us.
 // Staging the chunks in LDS to write a piece's run from eight lanes did not
 // help (313 us against 259, both with the atomics).
+// kJoin codes of at most 28 (7 x 4) or 22 (11 x 2) bits in all enter the bit
+// buffer together (14336 x 4096: 91 -> 85 us); a raw symbol among them is taken
+// up code by code. Loading a batch ahead did not help (83 us, but 4096 x 4096
+// AWQ 31 -> 36 us).
+template <int kJoin>
 __global__ __launch_bounds__(kUnitThreads) void unit_pack(UnitArgs a, uint32_t num_units,
                                                           const uint32_t *__restrict__ bucket_elem,
                                                           const uint16_t *__restrict__ codes,
@@ -530,7 +592,22 @@ __global__ __launch_bounds__(kUnitThreads) void unit_pack(UnitArgs a, uint32_t n
       w[j] = i + j < pc.iend && e < total ? in[e] : 0u;
     }
 #pragma unroll
-    for (int j = 0; j < kB; ++j) put_code(w[j], pc.lane + (i + j) * k_eff);
+    for (int j = 0; j < kB; j += kJoin) {
+      uint32_t raw = 0, v = 0, len = 0;
+#pragma unroll
+      for (int x = j; x < j + kJoin; ++x) {
+        const uint32_t l = cw16_len(w[x]);
+        raw |= w[x] & 0x8000u;
+        v = (v << l) | (w[x] & 0x7FFu);
+        len += l;
+      }
+      if (raw) {
+#pragma unroll
+        for (int x = j; x < j + kJoin; ++x) put_code(w[x], pc.lane + (i + x) * k_eff);
+      } else if (len) {
+        put(v, len);
+      }
+    }
   }
   // The rest of the last chunk.
   uint32_t lane = pc.lane, i = pc.iend;

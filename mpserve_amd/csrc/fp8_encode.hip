@@ -1968,10 +1968,13 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     W = (end + 63) >> 6;
     OUT(bitstream, uint64_t, 12, (size_t)W);
     if (W) {
-      hipLaunchKernelGGL(unit_pack, dim3((unsigned)(U + 7) / 8 * 8), dim3(kUnitThreads), 0, s, ua, (uint32_t)U,
-                         at32(o_belem), codes,
-                         at32(o_pieces), startbit, bit_base,
-                         reinterpret_cast<uint32_t *>(bitstream));
+      auto pack = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(U + 7) / 8 * 8), dim3(kUnitThreads), 0, s, ua, (uint32_t)U,
+                           at32(o_belem), codes, at32(o_pieces), startbit, bit_base,
+                           reinterpret_cast<uint32_t *>(bitstream));
+      };
+      if (L <= 7) pack(unit_pack<4>);
+      else pack(unit_pack<2>);
       HC(hipGetLastError());
     }
     return MPS_OK;
