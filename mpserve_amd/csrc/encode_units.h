@@ -8,12 +8,12 @@
 //   unit_hist    counts a unit's pairs in LDS and writes them as a list;
 //   merge_lists  adds up the lists of one scale (one q range of it) in LDS and
 //                sorts them by (q, count, symbol): the builder's item order;
-//   scan_parts, number_keys   table ids of the keys, in (scale, q) order;
+//   number_keys  table ids of the keys, in (scale, q) order;
 //   (the codebooks, from the sorted entries, fp8_encode.hip)
 //   unit_codes   maps a unit's elements to code words through an LDS table of
 //                the scale's pairs, stores them (16 bits an element, in bucket
 //                order) and sums each substream's bits within the unit;
-//   bucket_starts, bucket_bases   start bits of the substreams and buckets;
+//   bucket_starts   start bits of the substreams and buckets;
 //   unit_pack    writes each substream's piece of the unit into the bitstream.
 // Every pass has as many workgroups as units, so a tensor of few buckets, or
 // of few substreams a bucket, fills the chip too: a piece of a substream
@@ -31,6 +31,45 @@ constexpr uint32_t kPairSlots = 8192;   // LDS slots of a unit's, or a part's, p
 constexpr uint32_t kUnitRows = 1024;    // a unit spans at most this many rows (groups), + 2 partial ones
 constexpr uint32_t kNoPair = 0xFFFFFFFFu;
 constexpr uint32_t kMaxProbes = 256;
+
+// The scales' ranks among their sorted distinct values: res[0] the number of
+// values, ranks[i] of scale i, values[] ascending. One workgroup over a set of
+// 65536 bits in LDS: a few microseconds, where the host took some 80 for its
+// tables of 65536 alone (of a 1024 x 4096 weight's 360 us a build).
+__global__ __launch_bounds__(kUnitThreads) void scale_ranks(const uint16_t *__restrict__ scales, uint64_t n,
+                                                            uint32_t *__restrict__ res, uint16_t *__restrict__ ranks,
+                                                            uint16_t *__restrict__ values) {
+  constexpr uint32_t kWords = 65536 / 32, kPer = kWords / kUnitThreads;
+  __shared__ uint32_t s_set[kWords], s_before[kWords], s_tmp[16];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < kWords; i += kUnitThreads) s_set[i] = 0u;
+  __syncthreads();
+  for (uint64_t i = tid; i < n; i += kUnitThreads) {
+    const uint32_t v = scales[i], bit = 1u << (v & 31u);
+    if (!(s_set[v >> 5] & bit)) atomicOr(&s_set[v >> 5], bit);
+  }
+  __syncthreads();
+  uint32_t mine = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kPer; ++j) mine += (uint32_t)__popc(s_set[tid * kPer + j]);
+  uint32_t total = 0, at = block_exclusive_scan(mine, s_tmp, &total);
+#pragma unroll
+  for (uint32_t j = 0; j < kPer; ++j) {
+    const uint32_t w = tid * kPer + j;
+    uint32_t bits = s_set[w];
+    s_before[w] = at;
+    while (bits) {
+      values[at++] = (uint16_t)(32u * w + (uint32_t)__builtin_ctz(bits));
+      bits &= bits - 1u;
+    }
+  }
+  __syncthreads();
+  for (uint64_t i = tid; i < n; i += kUnitThreads) {
+    const uint32_t v = scales[i];
+    ranks[i] = (uint16_t)(s_before[v >> 5] + (uint32_t)__popc(s_set[v >> 5] & ((1u << (v & 31u)) - 1u)));
+  }
+  if (tid == 0) res[0] = total;
+}
 
 struct Unit {
   uint32_t bucket;
@@ -314,51 +353,47 @@ __global__ __launch_bounds__(kUnitThreads) void merge_lists(const uint32_t *__re
   }
 }
 
-// Exclusive sums of the parts' key counts (in place), and in res: [0] keys in
-// all, [1] entries in all, [2] most entries of one scale. One workgroup.
-__global__ __launch_bounds__(kScanBlock) void scan_parts(uint32_t *part_keys, const uint32_t *part_n, uint32_t scales,
-                                                         uint32_t parts, uint32_t *res) {
-  __shared__ uint32_t s_tmp[16], s_most, s_sum;
-  const uint32_t n = scales * parts, tid = threadIdx.x;
-  if (tid == 0) s_most = s_sum = 0u;
-  uint32_t run = 0;
-  for (uint32_t b = 0; b < n; b += kScanBlock) {
-    const uint32_t v = b + tid < n ? part_keys[b + tid] : 0u;
-    uint32_t total = 0;
-    const uint32_t ex = block_exclusive_scan(v, s_tmp, &total);
-    if (b + tid < n) part_keys[b + tid] = run + ex;
-    run += total;
-  }
-  __syncthreads();
-  for (uint32_t s = tid; s < scales; s += kScanBlock) {
-    uint32_t d = 0;
-    for (uint32_t p = 0; p < parts; ++p) d += part_n[s * parts + p];
-    atomicAdd(&s_sum, d);
-    atomicMax(&s_most, d);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    res[0] = run;
-    res[1] = s_sum;
-    res[2] = s_most;
-  }
-}
-
-// Table ids of scale blockIdx.x's keys, and their size classes' lists.
+// Table ids of scale blockIdx.x's keys (after the keys of the parts before its
+// own), and their size classes' lists. Workgroup 0 also sums up, in res: [0]
+// keys in all, [1] entries in all, [2] most entries of one scale.
 __global__ __launch_bounds__(256) void number_keys(const uint32_t *__restrict__ tcount,
-                                                   const uint32_t *__restrict__ part_keys, uint32_t parts, uint32_t T,
-                                                   uint32_t qvals, uint32_t *__restrict__ tgid,
+                                                   const uint32_t *__restrict__ part_keys,
+                                                   const uint32_t *__restrict__ part_n, uint32_t scales, uint32_t parts,
+                                                   uint32_t T, uint32_t qvals, uint32_t *__restrict__ tgid,
                                                    uint32_t *__restrict__ gid_tkey, uint32_t *lists, uint32_t cap,
-                                                   uint32_t *n3) {
-  __shared__ uint32_t s_tmp[16];
-  const uint32_t tk = blockIdx.x * 256u + threadIdx.x;
-  const uint32_t ni = threadIdx.x < qvals ? tcount[tk] : 0u;
-  const uint32_t gid = part_keys[blockIdx.x * parts] + block_exclusive_scan(ni ? 1u : 0u, s_tmp, nullptr);
+                                                   uint32_t *n3, uint32_t *res) {
+  __shared__ uint32_t s_tmp[16], s_before, s_all[3];
+  const uint32_t tid = threadIdx.x;
+  if (tid == 0) s_before = s_all[0] = s_all[1] = s_all[2] = 0u;
+  __syncthreads();
+  uint32_t before = 0;
+  for (uint32_t i = tid; i < blockIdx.x * parts; i += 256u) before += part_keys[i];
+  if (before) atomicAdd(&s_before, before);
+  __syncthreads();
+  const uint32_t tk = blockIdx.x * 256u + tid;
+  const uint32_t ni = tid < qvals ? tcount[tk] : 0u;
+  const uint32_t gid = s_before + block_exclusive_scan(ni ? 1u : 0u, s_tmp, nullptr);
   if (ni) {
     tgid[tk] = gid;
     gid_tkey[gid] = tk;
   }
   cb_append(gid, ni ? cb_class(ni, T) : -1, lists, cap, n3);
+  if (blockIdx.x != 0) return;
+  uint32_t keys = 0, entries = 0, most = 0;
+  for (uint32_t s = tid; s < scales; s += 256u) {
+    uint32_t d = 0;
+    for (uint32_t p = 0; p < parts; ++p) {
+      keys += part_keys[s * parts + p];
+      d += part_n[s * parts + p];
+    }
+    entries += d;
+    most = most > d ? most : d;
+  }
+  atomicAdd(&s_all[0], keys);
+  atomicAdd(&s_all[1], entries);
+  atomicMax(&s_all[2], most);
+  __syncthreads();
+  if (tid < 3u) res[tid] = s_all[tid];
 }
 
 // Code word of an element, 16 bits (L <= 11): code | length << 11 | raw16 << 15.
@@ -463,14 +498,18 @@ __global__ __launch_bounds__(kUnitThreads) void unit_codes(UnitArgs a, uint32_t 
 
 // Bucket blockIdx.x's substreams: start bits (k + 1 of them) from the pieces'
 // bits, each piece's offset from its substream's start (in place), and the
-// bucket's bits.
+// bucket's bits. The workgroup that finishes last (`done` counts them, from
+// zero) then lays out the buckets: 64-bit aligned bases, and the end of the last
+// bucket unaligned (build_huffman.cu:813-818).
 __global__ __launch_bounds__(kUnitThreads) void bucket_starts(const Unit *__restrict__ units,
                                                               const uint32_t *__restrict__ bucket_unit,
                                                               const uint32_t *__restrict__ lane_base, uint32_t k,
                                                               uint32_t *__restrict__ piece_bits,
                                                               uint32_t *__restrict__ startbit,
-                                                              uint32_t *__restrict__ bucket_bits) {
+                                                              uint32_t *bucket_bits, int64_t *__restrict__ bit_base,
+                                                              uint32_t *done) {
   __shared__ uint32_t s_tmp[16];
+  __shared__ bool s_last;
   const uint32_t b = blockIdx.x, t = threadIdx.x;
   const uint32_t k_eff = lane_base[b + 1] - lane_base[b];
   uint32_t acc = 0;
@@ -494,28 +533,25 @@ __global__ __launch_bounds__(kUnitThreads) void bucket_starts(const Unit *__rest
   uint32_t total = 0;
   const uint32_t ex = block_exclusive_scan(acc, s_tmp, &total);
   uint32_t *sb = startbit + (uint64_t)b * (k + 1u);
+  if (t < k) sb[t + 1] = t < k_eff ? ex + acc : total;
   if (t == 0) {
     sb[0] = 0u;
-    bucket_bits[b] = total;
+    __hip_atomic_store(bucket_bits + b, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
   }
-  if (t < k) sb[t + 1] = t < k_eff ? ex + acc : total;
-}
-
-// 64-bit aligned bucket bases, and the end of the last bucket unaligned
-// (build_huffman.cu:813-818). One workgroup.
-__global__ __launch_bounds__(kScanBlock) void bucket_bases(const uint32_t *__restrict__ bucket_bits, uint32_t B,
-                                                           int64_t *__restrict__ bit_base) {
-  __shared__ uint32_t s_tmp[16];
-  const uint32_t tid = threadIdx.x;
+  __syncthreads();
+  if (!s_last) return;
+  const uint32_t B = gridDim.x;
   uint64_t run = 0;  // 64-bit words
-  for (uint32_t b = 0; b < B; b += kScanBlock) {
-    const uint32_t bits = b + tid < B ? bucket_bits[b + tid] : 0u;
+  for (uint32_t b0 = 0; b0 < B; b0 += kUnitThreads) {
+    const bool in = b0 + t < B;
+    const uint32_t bits = in ? __hip_atomic_load(bucket_bits + b0 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     const uint32_t words = (uint32_t)(((uint64_t)bits + 63u) >> 6);
-    uint32_t total = 0;
-    const uint32_t ex = block_exclusive_scan(words, s_tmp, &total);
-    if (b + tid < B) bit_base[b + tid] = (int64_t)((run + ex) << 6);
-    if (b + tid + 1u == B) bit_base[B] = (int64_t)(((run + ex) << 6) + bits);
-    run += total;
+    uint32_t sum = 0;
+    const uint32_t first = block_exclusive_scan(words, s_tmp, &sum);
+    if (in) bit_base[b0 + t] = (int64_t)((run + first) << 6);
+    if (b0 + t + 1u == B) bit_base[B] = (int64_t)(((run + first) << 6) + bits);
+    run += sum;
   }
 }
 

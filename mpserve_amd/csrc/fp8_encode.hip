@@ -1522,15 +1522,19 @@ __global__ void pack_kernel(PackArgs a) {
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
-// The three codebook launches, one a size class.
+// The codebook launches, one a size class that has keys (at most most[c]; n3 on
+// the device says how many).
 void launch_codebooks(const CodebookArgs &cba, const uint64_t *skeys, const uint32_t *sslots, const uint32_t *lists,
-                      uint32_t cap, const uint32_t *n3, uint32_t most, hipStream_t s) {
-  hipLaunchKernelGGL(codebook_small_kernel, dim3(std::min((most + kCbWaves - 1) / kCbWaves, 2048u)),
-                     dim3(64 * kCbWaves), 0, s, cba, skeys, sslots, lists, n3);
-  hipLaunchKernelGGL((codebook_key_kernel<512, 256>), dim3(std::min(most, 2048u)), dim3(256), 0, s, cba, skeys, sslots,
-                     lists + cap, n3 + 1);
-  hipLaunchKernelGGL((codebook_key_kernel<2048, 512>), dim3(std::min(most, 512u)), dim3(512), 0, s, cba, skeys, sslots,
-                     lists + 2 * (size_t)cap, n3 + 2);
+                      uint32_t cap, const uint32_t *n3, const uint32_t *most, hipStream_t s) {
+  if (most[0])
+    hipLaunchKernelGGL(codebook_small_kernel, dim3(std::min((most[0] + kCbWaves - 1) / kCbWaves, 2048u)),
+                       dim3(64 * kCbWaves), 0, s, cba, skeys, sslots, lists, n3);
+  if (most[1])
+    hipLaunchKernelGGL((codebook_key_kernel<512, 256>), dim3(std::min(most[1], 2048u)), dim3(256), 0, s, cba, skeys,
+                       sslots, lists + cap, n3 + 1);
+  if (most[2])
+    hipLaunchKernelGGL((codebook_key_kernel<2048, 512>), dim3(std::min(most[2], 512u)), dim3(512), 0, s, cba, skeys,
+                       sslots, lists + 2 * (size_t)cap, n3 + 2);
 }
 
 template <typename T>
@@ -1655,21 +1659,24 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
       return fail(MPS_ERR_NO_MEMORY, "no device memory for output %d of the sidecar builder", slot); \
   }
 
-  // --- scales to host, dense scale index (sorted unique values) ---
-  std::vector<uint16_t> hsc((size_t)scale_numel);
-  HC(hipMemcpyAsync(hsc.data(), sp.scales, sizeof(uint16_t) * scale_numel, hipMemcpyDeviceToHost, s));
-  HC(hipStreamSynchronize(s));
-  std::vector<uint16_t> rank(65536, 0), uniq_sc;
+  // --- the scales' ranks among their sorted distinct values, to the host ---
+  // [0] how many values; then the scales' ranks, then the values, ascending
+  const size_t o_ranks = 256, o_values = o_ranks + 2 * (size_t)scale_numel;
+  const size_t most_values = std::min<size_t>((size_t)scale_numel, 65536);
+  std::vector<char> ranked(o_values + 2 * most_values);
   {
-    std::vector<uint8_t> seen(65536, 0);
-    for (uint16_t v : hsc) seen[v] = 1;
-    for (uint32_t v = 0; v < 65536; ++v)
-      if (seen[v]) {
-        rank[v] = (uint16_t)uniq_sc.size();
-        uniq_sc.push_back((uint16_t)v);
-      }
+    char *d = static_cast<char *>(alloc(ctx, -1, (int64_t)ranked.size()));
+    if (!d) return fail(MPS_ERR_NO_MEMORY, "no device memory for the sidecar builder's scales");
+    hipLaunchKernelGGL(scale_ranks, dim3(1), dim3(kUnitThreads), 0, s, sp.scales, (uint64_t)scale_numel,
+                       reinterpret_cast<uint32_t *>(d), reinterpret_cast<uint16_t *>(d + o_ranks),
+                       reinterpret_cast<uint16_t *>(d + o_values));
+    HC(hipGetLastError());
+    HC(hipMemcpyAsync(ranked.data(), d, ranked.size(), hipMemcpyDeviceToHost, s));
+    HC(hipStreamSynchronize(s));
   }
-  const uint32_t S = (uint32_t)uniq_sc.size();
+  const uint16_t *rank = reinterpret_cast<const uint16_t *>(ranked.data() + o_ranks);  // of scale i
+  const uint16_t *uniq_sc = reinterpret_cast<const uint16_t *>(ranked.data() + o_values);
+  const uint32_t S = *reinterpret_cast<const uint32_t *>(ranked.data());
 
   // --- buckets (build_huffman.cu:611-696), host ---
   // Rows (groups, by scale) are dealt to their scales by counting: ascending
@@ -1684,10 +1691,10 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
   if (by_scale || !scale_block2d) {
     std::vector<int64_t> at(S + 1, 0);  // first row (group) of each scale
     if (scale_block2d)
-      for (uint16_t v : hsc) at[rank[v] + 1] += sb0;
+      for (int64_t i = 0; i < scale_numel; ++i) at[rank[i] + 1] += sb0;
     else if (scale_scalar) at[1] = n;
     else
-      for (uint16_t v : hsc) at[rank[v] + 1] += 1;
+      for (int64_t i = 0; i < scale_numel; ++i) at[rank[i] + 1] += 1;
     const int64_t cap_rows = by_scale ? sp.group_cap : 128;
     for (uint32_t i = 0; i < S; ++i) {
       const int64_t rows = at[i + 1];
@@ -1699,10 +1706,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     }
     row_indices.resize((size_t)(n * per_row));
     if (by_scale) cols.resize(row_indices.size());
-    std::vector<uint16_t> ranks(hsc.size());
-    for (size_t i = 0; i < ranks.size(); ++i) ranks[i] = rank[hsc[i]];
     for (int64_t r = 0; r < n; ++r) {
-      const uint16_t *rk = ranks.data() + (scale_scalar ? 0 : scale_block2d ? r / sb0 * nb1 : r);
+      const uint16_t *rk = rank + (scale_scalar ? 0 : scale_block2d ? r / sb0 * nb1 : r);
       for (int64_t c = 0; c < per_row; ++c) {
         const size_t to = (size_t)at[rk[c]]++;
         row_indices[to] = (int32_t)r;
@@ -1716,7 +1721,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
         for (int64_t off = 0; off < sb0; off += 128) {
           const int64_t take = std::min<int64_t>(128, sb0 - off);
           for (int64_t q = 0; q < take; ++q) row_indices.push_back((int32_t)(br * sb0 + off + q));
-          bucket_sidx.push_back(rank[hsc[(size_t)(br * nb1 + bc)]]);
+          bucket_sidx.push_back(rank[br * nb1 + bc]);
           cols.push_back((int32_t)(bc * sb1));
           row_offsets.push_back((int32_t)row_indices.size());
         }
@@ -1736,7 +1741,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
 
   // --- one device block: the host-built arrays (`put`), then work memory (`take`) ---
   // flags: [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count, [5..7] codebook
-  // classes, [8..10] keys, entries and most entries of a scale (scan_parts)
+  // classes, [8..10] keys, entries and most entries of a scale (number_keys), [11] finished
+  // workgroups (bucket_starts)
   constexpr int kFlags = 16;
   uint32_t hflags[kFlags] = {};
   std::vector<char> host;
@@ -1752,7 +1758,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     std::memcpy(host.data() + at, src, sz);
     return at;
   };
-  const size_t o_flags = put(hflags, sizeof(hflags)), o_scale_values = put(uniq_sc.data(), 2 * (size_t)S),
+  const size_t o_flags = put(hflags, sizeof(hflags)), o_scale_values = put(uniq_sc, 2 * (size_t)S),
                o_sidx = put(bucket_sidx.data(), 2 * (size_t)B), o_lane_base = put(lane_base.data(), 4 * lane_base.size()),
                o_bscale = put(bucket_scale.data(), 2 * (size_t)B),
                o_rowoff = put(row_offsets.data(), 4 * row_offsets.size()),
@@ -1930,9 +1936,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     hipLaunchKernelGGL(merge_lists, dim3(S * P), dim3(kUnitThreads), 0, s, at32(o_sunit), at32(o_uos), at32(o_loff),
                        at32(o_ln), lists, P, (uint32_t)qvals, at32(o_poff), skeys, tcount, at32(o_toff), at32(o_pn),
                        at32(o_pk), flags);
-    hipLaunchKernelGGL(scan_parts, dim3(1), dim3(kScanBlock), 0, s, at32(o_pk), at32(o_pn), S, P, flags + 8);
-    hipLaunchKernelGGL(number_keys, dim3(S), dim3(256), 0, s, tcount, at32(o_pk), P, Tsz, (uint32_t)qvals, tgid,
-                       gid_tkey, cb_lists, (uint32_t)T, flags + 5);
+    hipLaunchKernelGGL(number_keys, dim3(S), dim3(256), 0, s, tcount, at32(o_pk), at32(o_pn), S, P, Tsz, (uint32_t)qvals,
+                       tgid, gid_tkey, cb_lists, (uint32_t)T, flags + 5, flags + 8);
     HC(hipGetLastError());
     HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
@@ -1944,7 +1949,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     if ((rc = alloc_tables()) != MPS_OK) return rc;
     cba.toff = at32(o_toff);
     cba.cw_slot = at32(o_cw);
-    launch_codebooks(cba, skeys, nullptr, cb_lists, (uint32_t)T, flags + 5, G, s);
+    launch_codebooks(cba, skeys, nullptr, cb_lists, (uint32_t)T, flags + 5, hflags + 5, s);
     HC(hipGetLastError());
     if ((rc = bucket_tables()) != MPS_OK) return rc;
     OUT(startbit, uint32_t, 10, (size_t)B * (kth + 1));
@@ -1957,8 +1962,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     if (most <= 6144) codes_pass(unit_codes<8192>);
     else codes_pass(unit_codes<16384>);
     hipLaunchKernelGGL(bucket_starts, dim3(B), dim3(kUnitThreads), 0, s, ua.units, at32(o_bunit), d_lane_base,
-                       (uint32_t)kth, at32(o_pieces), startbit, at32(o_bbits));
-    hipLaunchKernelGGL(bucket_bases, dim3(1), dim3(kScanBlock), 0, s, at32(o_bbits), B, bit_base);
+                       (uint32_t)kth, at32(o_pieces), startbit, at32(o_bbits), bit_base, flags + 11);
     HC(hipGetLastError());
     int64_t end = 0;
     HC(hipMemcpyAsync(&end, bit_base + B, 8, hipMemcpyDeviceToHost, s));
@@ -1987,10 +1991,10 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     std::vector<uint16_t> row_sidx, block_sidx;
     if (scale_block2d) {
       block_sidx.resize((size_t)(nb0 * nb1));
-      for (size_t i = 0; i < block_sidx.size(); ++i) block_sidx[i] = rank[hsc[i]];
+      for (size_t i = 0; i < block_sidx.size(); ++i) block_sidx[i] = rank[i];
     } else {
       row_sidx.resize((size_t)n);
-      for (size_t r = 0; r < row_sidx.size(); ++r) row_sidx[r] = rank[hsc[scale_scalar ? 0 : r]];
+      for (size_t r = 0; r < row_sidx.size(); ++r) row_sidx[r] = rank[scale_scalar ? 0 : r];
     }
     DevBuf<uint16_t> d_row_sidx, d_block_sidx;
     HC(d_row_sidx.alloc(row_sidx.size()));
@@ -2131,7 +2135,8 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
       HC(hipMemsetAsync(flags + 5, 0, 12, s));
       hipLaunchKernelGGL(codebook_classes_kernel, dim3((G + 255) / 256), dim3(256), 0, s, gid_tkey, tcount, G, Tsz,
                          cb_lists.p, flags + 5);
-      launch_codebooks(cba, keys_sorted.p, slots_sorted.p, cb_lists.p, G, flags + 5, G, s);
+      const uint32_t any[3] = {G, G, G};
+      launch_codebooks(cba, keys_sorted.p, slots_sorted.p, cb_lists.p, G, flags + 5, any, s);
     } else if (G) {
       hipLaunchKernelGGL(codebook_kernel, dim3((G + 63) / 64), dim3(64), 0, s, cba);
     }
