@@ -187,20 +187,17 @@ def _launch(int4, bitstream, syms, lens, table, col_start, col_len, offsets, row
     d.n, d.m, d.out = n, m, out.data_ptr()
     if n * m >= (1 << 31):
         raise ValueError("tensor too large for the AWQ decode kernel (n*m >= 2^31)")
-    # From its second call on a sidecar that the slab path can take (k = 1024: by-scale
-    # with 128-column groups, or row buckets; k = 256 or 512: by-scale with 128-column
-    # groups, or row buckets when m is a multiple of 4k, whose buckets the plan splits
-    # into ranges decoded side by side) the op launches the sidecar's cached plan; other
-    # sidecars (whose plans would take the per-lane path, slower than this kernel's two
-    # workgroups per bucket when a tensor has fewer buckets than CUs) and the first call
-    # decode over whole buckets, as the reference does.
+    # From its second call on a sidecar that the slab paths can take (k = 256, 512 or
+    # 1024: row buckets, or by-scale groups of a power of two of 64 columns up to k, or of
+    # 1024 columns or more) the op launches the sidecar's cached plan; other sidecars
+    # (whose plans would take the per-lane path, slower than this kernel's two workgroups
+    # per bucket when a tensor has fewer buckets than CUs) and the first call decode over
+    # whole buckets, as the reference does.
     key_tensors = tuple(t for t in (int4, bitstream, syms, lens, table, col_start, col_len, offsets, rows, group_col,
                                     startbit, bit_base) if t is not None)
     k = startbit.size(1) - 1
-    if group_col is None:
-        slab = k == 1024 or (k in (256, 512) and m % (4 * k) == 0)
-    else:
-        slab = k in (256, 512, 1024) and int(group_size) == 128
+    gs = int(group_size)
+    slab = k in (256, 512, 1024) and (group_col is None or gs >= 1024 or (64 <= gs <= k and gs & (gs - 1) == 0))
     with torch.cuda.device(dev):
         stream = _stream_handle(dev)
         plan = None
