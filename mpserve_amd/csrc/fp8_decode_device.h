@@ -92,7 +92,12 @@ constexpr int32_t kMultiRange = 0x10;
 // A flat item (a whole bucket, a range of its slabs, or several ranges side by
 // side): `rows` holds its elements, bits 8.. of `path` the column its first
 // element has in its first row, and bits 12.. of `k_eff` the slabs a range
-// (kMultiRange).
+// (kMultiRange). A run (kFlatRun) is several small whole buckets with the same
+// tables, which are staged once: the item is the first of them, bits 8.. of
+// `path` hold how many there are, and bits 12.. of `k_eff` where the others'
+// records start among the plan's followers. The work-items' groups of k_eff
+// take the run's buckets in turn.
+constexpr int32_t kFlatRun = 0x20;
 constexpr int kFlatColBits = 24, kFlatSlabShift = 12;
 
 struct BucketShape {
@@ -1068,9 +1073,10 @@ __device__ __forceinline__ WorkItem bucket_item(const mps_fp8_tensor &T, int64_t
 // kFlat: flat items (their paths' registers and code stay out of the kernels of
 // launches that have none).
 template <bool kQueue, bool kSlabK, bool kFlat>
-__device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t *out, const WorkItem &w,
+__device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t *out, const WorkItem &item,
                                               uint32_t *lds, uint32_t *status, uint32_t *queue,
-                                              uint32_t &ticket, int32_t wg_part, int32_t wg_parts MPS_TR_PARAM) {
+                                              uint32_t &ticket, int32_t wg_part, int32_t wg_parts,
+                                              const WorkItem *__restrict__ followers MPS_TR_PARAM) {
   uint32_t *qregion = lds;
   uint32_t *lut = lds + kQWords;
   int32_t *s_rows = reinterpret_cast<int32_t *>(qregion) + 6 * kBlock;    // queue slot 6 (generic path)
@@ -1081,8 +1087,25 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
   int tid;
   __asm__ volatile("v_mov_b32 %0, %1" : "=v"(tid) : "v"((int)threadIdx.x));
 
-  const int32_t path = w.path & 0xF;
-  const int32_t c0 = w.c0, cl = w.cl, k_eff = kFlat ? w.k_eff & ((1 << kFlatSlabShift) - 1) : w.k_eff;
+  const int32_t path = item.path & 0xF;
+  // A run: this work-item's group of k_eff starts with the run's bucket `r_at`, whose
+  // record takes the item's place here (the tables are the same).
+  const bool run = kFlat && (item.path & kFlatRun) != 0;
+  const uint32_t run_k = kFlat ? (uint32_t)item.k_eff & ((1u << kFlatSlabShift) - 1u) : 0u;
+  const uint32_t run_n = run ? (uint32_t)item.path >> 8 : 1u, run_from = (uint32_t)item.k_eff >> kFlatSlabShift;
+  uint32_t r_at = run ? uni((uint32_t)tid / run_k) : 0u;
+  const bool spare = r_at >= run_n;
+  auto own_item = [&]() -> decltype(auto) {
+    if constexpr (kFlat) {
+      WorkItem x = item;
+      if (run && r_at > 0 && !spare) x = followers[run_from + r_at - 1u];
+      return x;
+    } else {
+      return (item);
+    }
+  };
+  decltype(auto) w = own_item();
+  const int32_t c0 = w.c0, cl = w.cl, k_eff = kFlat ? (int32_t)run_k : w.k_eff;
   const bool bucket_ok = path != kPathBad;
   const bool k1024 = path == kPathK1024;
   const bool fast = path == kPathFast;
@@ -1090,7 +1113,7 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
   // A multi-range item (fast path, k_eff 256 or 512): work-items
   // [sub * k_eff, (sub + 1) * k_eff) decode its sub-th range, whose rows,
   // start bits and end bits follow the previous range's (uniform per wave).
-  const bool multi = (w.path & kMultiRange) != 0;
+  const bool multi = (item.path & kMultiRange) != 0;
   const int32_t mrr = (w.path >> 8) & 0xFF;
   const int32_t sub = multi ? (int32_t)uni((uint32_t)(tid >> (k_eff == 256 ? 8 : 9))) : 0;
   int32_t rows = multi ? max(0, min(mrr, w.rows - sub * mrr)) : w.rows;
@@ -1099,9 +1122,9 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
   uint32_t f_elems = 0, f_col = 0, f_row0 = 0;
   if (flat) {
     const uint32_t step = multi ? ((uint32_t)w.k_eff >> kFlatSlabShift) * (uint32_t)k_eff : 0u;  // elements a range
-    const uint32_t at = (uint32_t)sub * step, all = (uint32_t)w.rows;
+    const uint32_t at = (uint32_t)sub * step, all = spare ? 0u : (uint32_t)w.rows;
     f_elems = uni(at < all ? (multi ? min(step, all - at) : all) : 0u);
-    const uint32_t x = ((uint32_t)w.path >> 8) + at;
+    const uint32_t x = (run ? 0u : (uint32_t)w.path >> 8) + at;
     f_row0 = uni(x / (uint32_t)cl);
     f_col = uni(x - f_row0 * (uint32_t)cl);
     rows = (int32_t)uni((f_col + f_elems + (uint32_t)cl - 1u) / (uint32_t)cl);
@@ -1109,7 +1132,8 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
   }
   const int64_t total = (int64_t)rows * cl;
   const uint64_t nm = (uint64_t)T.n * (uint64_t)T.m;
-  const int lane = multi ? (tid & (k_eff - 1)) : tid;  // the lane's substream (work-item within its range)
+  // the lane's substream (work-item within its range, or its bucket of a run)
+  const int lane = multi || run ? (tid & (k_eff - 1)) : tid;
   // Substream of this work-item: the k = 1024 paths give wave w's 16-lane row
   // R, position v the column 64w + 4v + R (see decode_slab4); the others, the lane.
   // A fast-path bucket with k_eff 256 or 512 takes the slab path too (kSlabK).
@@ -1331,7 +1355,8 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
   tr[0] = __builtin_amdgcn_s_memrealtime();
 #endif
 
-  if (!bucket_ok || any_bad_row) {
+  // (In a run, a bad row skips its bucket only: below, wave by wave.)
+  if (!bucket_ok || (any_bad_row && !run)) {
     if (tid == 0) flag(status, !bucket_ok ? MPS_STATUS_BAD_BUCKET : MPS_STATUS_BAD_ROW);
     return;
   }
@@ -1365,17 +1390,57 @@ __device__ __forceinline__ void decode_bucket(const mps_fp8_tensor &T, uint16_t 
 #undef MPS_SLAB
   } else if (kFlat && flat) {
     const uint32_t ks = k_eff == 1024 ? 10u : k_eff == 512 ? 9u : 8u;
-#define MPS_FLAT(WRAP, ESC)                                                                                        \
-  decode_slab4<WRAP, ESC, 0>(T, out, lut, qregion, (uint32_t)tid, (uint32_t)lane, ks, f_elems, (uint32_t)cl, rowoff_lo, \
-                             rowoff_hi, base, first, pos, pos_end, status, f_col)
-    if (cl % 4 == 0) {
-      if (has_esc) MPS_FLAT(3, true);
-      else MPS_FLAT(3, false);
-    } else {
-      if (has_esc) MPS_FLAT(4, true);
-      else MPS_FLAT(4, false);
-    }
+    uint32_t cl_at = (uint32_t)cl, lo_at = rowoff_lo, hi_at = rowoff_hi;
+    uint64_t base_at = base;
+    bool bad = run && __builtin_amdgcn_ballot_w64(bad_row) != 0;
+    if (bad && wl == 0) flag(status, MPS_STATUS_BAD_ROW);
+    for (;;) {
+#define MPS_FLAT(WRAP, ESC)                                                                                          \
+  decode_slab4<WRAP, ESC, 0>(T, out, lut, qregion, (uint32_t)tid, (uint32_t)lane, ks, f_elems, cl_at, lo_at, hi_at,   \
+                             base_at, first, pos, pos_end, status, f_col)
+      if (bad) {
+      } else if (cl_at % 4u == 0u) {
+        if (has_esc) MPS_FLAT(3, true);
+        else MPS_FLAT(3, false);
+      } else {
+        if (has_esc) MPS_FLAT(4, true);
+        else MPS_FLAT(4, false);
+      }
 #undef MPS_FLAT
+      if (!run) return;
+      // The run's next bucket of this group, wave by wave: a lane's queue column is
+      // its own and the tables stay, so nothing here meets the other waves.
+      do {
+        r_at += (uint32_t)kBlock >> ks;
+        if (r_at >= run_n) return;
+        const WorkItem x = followers[run_from + r_at - 1u];
+        cl_at = (uint32_t)x.cl;
+        f_elems = (uint32_t)x.rows;
+        base_at = (uint64_t)x.bit_base;
+        const uint32_t nr = f_elems / cl_at;  // whole rows
+        const __amdgpu_buffer_rsrc_t r_rw = make_rsrc(x.row_idx, nr * 4u);
+        const int32_t lo = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(r_rw, (uint32_t)wl * 4u, 0, 0);
+        const int32_t hi = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(r_rw, (uint32_t)(wl + 64) * 4u, 0, 0);
+        const __amdgpu_buffer_rsrc_t r_bits = make_rsrc(x.startbits, ((uint32_t)k_eff + 1u) * 4u);
+        pos = __builtin_amdgcn_raw_buffer_load_b32(r_bits, (uint32_t)col * 4u, 0, 0);
+        pos_end = __builtin_amdgcn_raw_buffer_load_b32(r_bits, (uint32_t)col * 4u + 4u, 0, 0);
+        const uint64_t bs_bytes = bs_words > 0 ? (uint64_t)bs_words * 8u : 0u, base_byte = base_at >> 3;
+        const __amdgpu_buffer_rsrc_t r_bs =
+            make_rsrc(bs_ptr + (base_byte < bs_bytes ? base_byte : 0), base_byte < bs_bytes ? (uint32_t)(bs_bytes - base_byte) : 0u);
+        const uint32_t o = ((pos >> 5) & ~1u) * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b128(r_bs, o + 16u * (uint32_t)i, 0, 0);
+          first[2 * i] = make_uint2(v[0], v[1]);
+          first[2 * i + 1] = make_uint2(v[2], v[3]);
+        }
+        const bool in_lo = (uint32_t)wl < nr, in_hi = (uint32_t)wl + 64u < nr;
+        bad = __builtin_amdgcn_ballot_w64((in_lo && (lo < 0 || lo >= T.n)) || (in_hi && (hi < 0 || hi >= T.n))) != 0;
+        lo_at = in_lo ? (uint32_t)lo * (uint32_t)T.m + (uint32_t)x.c0 : 0u;
+        hi_at = in_hi ? (uint32_t)hi * (uint32_t)T.m + (uint32_t)x.c0 : 0u;
+        if (bad && wl == 0) flag(status, MPS_STATUS_BAD_ROW);
+      } while (bad);
+    }
   } else if (kSlabK && slab) {
     // k_eff 256 / 512 (col_len % k_eff == 0 on the fast path): work-item tid
     // decodes substream `col` of its range, over slabs of k_eff columns
@@ -1438,12 +1503,12 @@ __global__ __launch_bounds__(kBlock) void fp8_decode_one(mps_fp8_tensor T, uint3
     const int64_t b = (int64_t)blockIdx.x / parts;
     if (b < T.num_buckets)
       decode_bucket<false, kSlabK, kFlat>(T, T.out, bucket_item(T, b, kFlat), lds, status, nullptr, ticket,
-                                          (int32_t)(blockIdx.x % parts), parts MPS_TR_ARG);
+                                          (int32_t)(blockIdx.x % parts), parts, nullptr MPS_TR_ARG);
     return;
   }
   for (int64_t b = blockIdx.x; b < T.num_buckets; b += gridDim.x) {
-    decode_bucket<false, kSlabK, kFlat>(T, T.out, bucket_item(T, b, kFlat), lds, status, nullptr, ticket, 0,
-                                        1 MPS_TR_ARG);
+    decode_bucket<false, kSlabK, kFlat>(T, T.out, bucket_item(T, b, kFlat), lds, status, nullptr, ticket, 0, 1,
+                                        nullptr MPS_TR_ARG);
     end_bucket();
   }
 }
@@ -1496,7 +1561,7 @@ __global__ __launch_bounds__(kBlock) void fp8_decode_plan(const mps_fp8_tensor *
       uint64_t tr[4] = {0, 0, 0, 0};
 #endif
       const mps_fp8_tensor &T = tensors[w.tensor];
-      decode_bucket<!kEndTicket, kSlabK, kFlat>(T, T.out + out_delta, w, lds, status, queue, ticket, 0, 1 MPS_TR_ARG);
+      decode_bucket<!kEndTicket, kSlabK, kFlat>(T, T.out + out_delta, w, lds, status, queue, ticket, 0, 1, work + nwork MPS_TR_ARG);
 #if MPS_TRACE_ITEMS
       const uint64_t tr_wave = __builtin_amdgcn_s_memrealtime();
 #endif

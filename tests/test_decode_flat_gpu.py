@@ -90,3 +90,25 @@ def test_flat_ranges(m):
     sides = [oracle.encode(bf, q, sc[:1].copy(), 7, k) for k in (256, 512, 1024)]
     for s in sides:
         assert _check(bf, q, [s]) > s["bucket_table_i32"].shape[0]
+
+
+@pytest.mark.parametrize("k", [256, 1024])
+def test_flat_runs_share_tables(k):
+    """More blocks of three scales than CUs: a plan decodes several after one table set-up. A row
+    index out of range costs its own block only."""
+    print(f"[flat] runs k{k}", flush=True)
+    bs, g = 64, 30
+    bf, q, _ = synth(bs * g, bs * g, seed=k)
+    sc = np.random.default_rng(k).integers(0x2000, 0x2003, size=(g, g), dtype=np.uint16)
+    side = oracle.encode(bf, q, sc, 7, k)
+    assert _check(bf, q, [side]) < g * g
+    side["row_indices_i32"] = side["row_indices_i32"].copy()
+    hit = 17 * g + 5  # a bucket's index: block row 17, block column 5
+    side["row_indices_i32"][hit * bs + 3] = bs * g
+    out = torch.zeros(q.shape, dtype=torch.bfloat16, device=DEV)
+    plan = DecodePlan([(torch.from_numpy(q).to(DEV), to_torch(side, DEV), out)])
+    plan.decode()
+    assert plan.read_status() == _native.MPS_STATUS_BAD_ROW
+    want = bf.copy()
+    want[17 * bs:18 * bs, 5 * bs:6 * bs] = 0
+    np.testing.assert_array_equal(out.view(torch.uint16).cpu().numpy(), want)
