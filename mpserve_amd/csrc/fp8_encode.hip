@@ -647,25 +647,27 @@ __global__ void codebook_kernel(CodebookArgs a) {
 //    the boundary count c; every entry above c's run is kept, and the run's
 //    first ones (smallest symbols) fill the rest;
 //  - esc_sym from a 65536-bit set of the symbols in LDS;
-//  - the package-merge levels built once, bottom-up. A merge is a rank an item:
-//    leaf i lands after the i leaves and the packages lighter than it, package
-//    b after the b packages and the leaves no heavier (leaf first on equal
-//    weight), both found by binary search. A bit an item says whether it is a
-//    leaf; the selection then counts leaf bits top-down;
+//  - the package-merge levels built once, bottom-up. A merge is a merge path of
+//    four outputs a work-item (leaf first on equal weight): one binary search,
+//    four items in turn, their two pairs written as the next level's packages
+//    and their leaf bits as half a byte. So a level is some fifteen LDS reads in
+//    a chain and one barrier. The selection then counts leaf bits top-down;
 //  - canonical codes in list order, ranked within each length by ballots;
 //  - the decode table, entry by entry (prefix minus a length's first code,
-//    below its count, is the code's rank), and each histogram entry's code word
-//    from its list position, which follows from its sorted index.
+//    below its count, is the code's rank), and the code word of the histogram
+//    entry behind each list item.
+// What bounds it is the chain of one key: a tensor has few long lists (128 past
+// 512 entries of the AWQ weight below), so a key gets the work-items that make
+// the chain short, and everything searched is in LDS.
 //
 // Weights add up as the reference's ints do. A package holds a leaf at most once
 // a level, so sums stay below 11 times the key's total; a key whose sums could
 // wrap, and leave the packages unsorted, is merged in sequence by one lane, as
 // the reference merges.
 //
-// NT work-items a key: with one wave and a merge path of 32 outputs a lane,
-// lists of up to 2048 left most of a CU idle behind one long chain. Measured on
-// the 2,500 keys of a 4096 x 4096 AWQ weight: lists past 512 343 -> 142 us,
-// past 64 104 -> 62 us.
+// Measured on the 2,600 keys of a 4096 x 4096 AWQ weight: lists past 512 with a
+// wave a key (32 outputs a lane) 343 us, with 512 work-items a key and each item
+// ranked by a search of its own 142, so 39; lists past 64 104, 60, 27 us.
 // ---------------------------------------------------------------------------
 constexpr int kCbSmall = 64;  // keys of at most this many entries and no ESC: codebook_small_kernel
 constexpr int kCbMaxL = 11;
@@ -684,8 +686,7 @@ struct CbShared {
   uint8_t lens[NMAX];
   union {
     struct {
-      int32_t cur[2 * NMAX];   // a level's items
-      int32_t pack[NMAX];      // their pairs
+      int32_t pack[2][NMAX];  // a level's items in pairs, this level's and the last one's
       uint32_t masks[kCbMaxL * (NMAX / 16)];
     } pm;
     uint32_t symset[65536 / 32];
@@ -725,13 +726,13 @@ __device__ __forceinline__ uint32_t cb_min(uint32_t *red, uint32_t v) {
   return v;
 }
 
-// First index in [lo, hi) of the sorted keys whose count is >= c (lower) or > c (upper).
-__device__ __forceinline__ uint32_t cb_bound(const uint64_t *k, uint32_t lo, uint32_t hi, uint32_t c, bool upper) {
-  const int32_t ci = (int32_t)c;
+// First of n ascending counts in LDS that is >= c (lower) or > c (upper).
+__device__ __forceinline__ uint32_t cb_bound(const int32_t *counts, uint32_t n, int32_t c, bool upper) {
+  uint32_t lo = 0, hi = n;
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
-    const int32_t x = (int32_t)cb_count(k[mid]);
-    if (upper ? x <= ci : x < ci) lo = mid + 1;
+    const int32_t x = counts[mid];
+    if (upper ? x <= c : x < c) lo = mid + 1;
     else hi = mid;
   }
   return lo;
@@ -767,23 +768,24 @@ __device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const Codebo
       const uint64_t k = keys[p];
       S.lw[p] = (int32_t)cb_count(k);
       S.ls[p] = (uint16_t)cb_sym(k);
-      S.hidx[p] = (int32_t)p;
     }
     nl = ni;
   } else {
     // kept: [s0, s0 + r) and [s1, ni), the top 2^L - 1 by (count desc, sym asc)
     const uint32_t c = cb_count(keys[ni - keep]);
-    s0 = cb_bound(keys, 0, ni, c, false);
-    s1 = cb_bound(keys, s0, ni, c, true);
-    r = keep - (ni - s1);
     uint32_t tot = 0, kept = 0;
     for (uint32_t t = tid; t < ni; t += NT) {
       const uint32_t cnt = cb_count(keys[t]);
       tot += cnt;
-      kept += (t >= s1 || (t >= s0 && t < s0 + r)) ? cnt : 0u;
+      kept += (int32_t)cnt > (int32_t)c ? cnt : 0u;
+      s0 += (int32_t)cnt < (int32_t)c ? 1u : 0u;
+      s1 += (int32_t)cnt <= (int32_t)c ? 1u : 0u;
     }
+    s0 = cb_sum<NT>(S.red, s0);
+    s1 = cb_sum<NT>(S.red, s1);
+    r = keep - (ni - s1);
     tot = cb_sum<NT>(S.red, tot);
-    kept = cb_sum<NT>(S.red, kept);
+    kept = cb_sum<NT>(S.red, kept) + r * c;
     const uint32_t ew = tot - kept;  // int sums as in the reference
     // esc_sym: the smallest u16 absent from the key's symbols (kEscAwqByScale) or
     // from the kept ones (the other builders)
@@ -807,39 +809,27 @@ __device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const Codebo
     if (a.esc_mode == kEscAwqByScale) {
       esc_sym = cand == 0xFFFFFFFFu ? 0xFFFFu : cand;
       esc_w = (int32_t)ew;
-      // (count desc, sym asc), ESC last: an entry of a run [g0, g1) above c sits
-      // at (ni - g1) + (t - g0); the boundary run's first r follow them
-      for (uint32_t t = tid; t < ni; t += NT) {
-        uint32_t pos;
-        if (t >= s1) {
-          const uint32_t cc = cb_count(keys[t]);
-          const uint32_t g0 = cb_bound(keys, s1, t + 1, cc, false);
-          const uint32_t g1 = cb_bound(keys, t, ni, cc, true);
-          pos = (ni - g1) + (t - g0);
-        } else if (t >= s0 && t < s0 + r) {
-          pos = (ni - s1) + (t - s0);
-        } else {
-          continue;
-        }
-        const uint64_t k = keys[t];
-        S.lw[pos] = (int32_t)cb_count(k);
-        S.ls[pos] = (uint16_t)cb_sym(k);
-        S.hidx[pos] = (int32_t)t;
+      // The kept counts, ascending: entry j of a run [j0, j1) of one count sits at
+      // keep - j1 + (j - j0) in the list, which is (count desc, sym asc), ESC last.
+      // The package-merge's weights are the same counts with the ESC weight merged
+      // in (ties: any order gives the same list).
+      int32_t *asc = S.u.pm.pack[0];
+      uint32_t e_pos = 0;  // kept counts < the ESC weight (as int)
+      for (uint32_t j = tid; j < keep; j += NT) {
+        const int32_t c = (int32_t)cb_count(keys[j < r ? s0 + j : s1 + (j - r)]);
+        asc[j] = c;
+        e_pos += c < esc_w ? 1u : 0u;
       }
-      // the package-merge's weights, ascending: the kept counts in sorted order
-      // with the ESC weight merged in (ties: any order gives the same list)
-      uint32_t e_pos = 0;
-      {
-        uint32_t below = 0;  // kept counts < the ESC weight (as int)
-        for (uint32_t j = tid; j < keep; j += NT) {
-          const uint32_t t = j < r ? s0 + j : s1 + (j - r);
-          below += (int32_t)cb_count(keys[t]) < esc_w ? 1u : 0u;
-        }
-        e_pos = cb_sum<NT>(S.red, below);
-      }
+      e_pos = cb_sum<NT>(S.red, e_pos);
       for (uint32_t j = tid; j < keep; j += NT) {
         const uint32_t t = j < r ? s0 + j : s1 + (j - r);
-        S.sw[j + (j >= e_pos ? 1u : 0u)] = (int32_t)cb_count(keys[t]);
+        const int32_t c = asc[j];
+        const uint32_t j0 = cb_bound(asc, keep, c, false), j1 = cb_bound(asc, keep, c, true);
+        const uint32_t pos = keep - j1 + (j - j0);
+        S.sw[j + (j >= e_pos ? 1u : 0u)] = c;
+        S.lw[pos] = c;
+        S.ls[pos] = (uint16_t)cb_sym(keys[t]);
+        S.hidx[pos] = (int32_t)t;
       }
       if (tid == 0) {
         S.sw[e_pos] = esc_w;
@@ -887,11 +877,12 @@ __device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const Codebo
     uint32_t sum = 0;
     for (uint32_t i = tid; i < n; i += NT) sum += (uint32_t)W[i];
     const bool wraps = cb_sum<NT>(S.red, sum) >= (1u << 31) / 12u;
-    int32_t *cur = S.u.pm.cur, *pack = S.u.pm.pack;
+    int32_t *from = S.u.pm.pack[0], *to = S.u.pm.pack[1];
     uint32_t have = n < keep_pm ? n : keep_pm;
     uint32_t sizes[kCbMaxL];
     constexpr uint32_t kWords = NMAX / 16;  // of a level's mask
-    for (uint32_t i = tid; i < have; i += NT) cur[i] = W[i];
+    static_assert(4 * NT == 2 * NMAX, "four outputs of a level a work-item");
+    for (uint32_t b = tid; b < have / 2u; b += NT) from[b] = (int32_t)((uint32_t)W[2u * b] + (uint32_t)W[2u * b + 1u]);
     for (uint32_t i = tid; i < kWords; i += NT) {
       const uint32_t lo = 32u * i;
       S.u.pm.masks[i] = have >= lo + 32u ? 0xFFFFFFFFu : have > lo ? (1u << (have - lo)) - 1u : 0u;
@@ -903,43 +894,56 @@ __device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const Codebo
       sizes[j] = 0;
       if (j >= L) continue;
       const uint32_t np = have / 2u;
-      uint32_t *mk = S.u.pm.masks + j * kWords;
-      for (uint32_t b = tid; b < np; b += NT) pack[b] = (int32_t)((uint32_t)cur[2u * b] + (uint32_t)cur[2u * b + 1u]);
-      for (uint32_t i = tid; i < kWords; i += NT) mk[i] = 0u;
-      __syncthreads();
+      uint8_t *mk = reinterpret_cast<uint8_t *>(S.u.pm.masks + j * kWords);
       have = n + np < keep_pm ? n + np : keep_pm;
       sizes[j] = have;
       if (wraps) {
         if (tid == 0) {
+          uint32_t bits = 0, last = 0;
           for (uint32_t o = 0, x = 0, b = 0; o < have; ++o) {
-            if (x < n && (b >= np || W[x] <= pack[b])) {
-              cur[o] = W[x++];
-              mk[o >> 5] |= 1u << (o & 31u);
-            } else {
-              cur[o] = pack[b++];
-            }
+            const bool leaf = x < n && (b >= np || W[x] <= from[b]);
+            const uint32_t v = (uint32_t)(leaf ? W[x++] : from[b++]);
+            bits = (bits >> 1) | (leaf ? 0x80u : 0u);
+            if (o & 1u) to[o >> 1] = (int32_t)(last + v);
+            last = v;
+            if ((o & 7u) == 7u) mk[o >> 3] = (uint8_t)bits;
+            else if (o + 1u == have) mk[o >> 3] = (uint8_t)((bits & 0xFFu) >> (7u - (o & 7u)));
           }
         }
       } else {
-        for (uint32_t i = tid; i < n + np; i += NT) {
-          const bool leaf = i < n;
-          const uint32_t at = leaf ? i : i - n;
-          const int32_t v = leaf ? W[at] : pack[at];
-          uint32_t lo = 0, hi = leaf ? np : n;
-          const int32_t *other = leaf ? pack : W;
-          while (lo < hi) {  // packages lighter than this leaf, or leaves no heavier than this package
+        const uint32_t o = 4u * tid;  // this work-item's outputs: [o, o + 4)
+        uint32_t bits = 0;
+        if (o < have) {
+          uint32_t lo = o > np ? o - np : 0u, hi = o < n ? o : n;
+          while (lo < hi) {  // how many leaves are among the first o
             const uint32_t mid = (lo + hi) >> 1;
-            const int32_t x = other[mid];
-            if (leaf ? x < v : x <= v) lo = mid + 1u;
+            if (W[mid] <= from[o - 1u - mid]) lo = mid + 1u;
             else hi = mid;
           }
-          const uint32_t to = at + lo;
-          if (to < have) {
-            cur[to] = v;
-            if (leaf) atomicOr(&mk[to >> 5], 1u << (to & 31u));
+          uint32_t x = lo, b = o - lo;
+          int32_t wv = W[x < n ? x : n - 1u], pv = from[b], v[4];
+#pragma unroll
+          for (uint32_t i = 0; i < 4u; ++i) {
+            const bool leaf = x < n && (b >= np || wv <= pv);
+            v[i] = leaf ? wv : pv;
+            bits |= leaf ? 1u << i : 0u;
+            x += leaf ? 1u : 0u;
+            b += leaf ? 0u : 1u;
+            if (i < 3u) {
+              const int32_t next = *(leaf ? W + (x < n ? x : n - 1u) : from + (b < np ? b : 0u));
+              wv = leaf ? next : wv;
+              pv = leaf ? pv : next;
+            }
           }
+          if (o + 1u < have) to[2u * tid] = v[0] + v[1];
+          if (o + 3u < have) to[2u * tid + 1u] = v[2] + v[3];
         }
+        const uint32_t other = (uint32_t)__shfl_xor((int)bits, 1);
+        if (!(tid & 1u)) mk[tid >> 1] = (uint8_t)(bits | (other << 4));
       }
+      int32_t *const swap = from;
+      from = to;
+      to = swap;
       __syncthreads();
     }
     // top-down, by every wave for itself
@@ -1060,35 +1064,16 @@ __device__ __forceinline__ void codebook_key(CbShared<NMAX, NT> &S, const Codebo
   const uint32_t esc_cw = use_esc ? ((uint32_t)S.lens[esc_pos] << 16) | (S.code[esc_pos] & 0xFFFFu) : 0u;
 
   // --- code word of every histogram entry, from its list position ---
-  for (uint32_t t = tid; t < ni; t += NT) {
-    int32_t p = -1;
-    if (!use_esc) {
-      p = (int32_t)t;
-    } else if (a.esc_mode == kEscAwqByScale) {
-      if (t >= s1) {
-        const uint32_t cc = cb_count(keys[t]);
-        const uint32_t g0 = cb_bound(keys, s1, t + 1, cc, false);
-        const uint32_t g1 = cb_bound(keys, t, ni, cc, true);
-        p = (int32_t)((ni - g1) + (t - g0));
-      } else if (t >= s0 && t < s0 + r) {
-        p = (int32_t)((ni - s1) + (t - s0));
-      }
-    } else {
-      int32_t j = -1;
-      if (t >= s0 && t < s0 + r) j = (int32_t)(t - s0);
-      else if (t >= s1) j = (int32_t)(r + (t - s1));
-      if (j >= 0) p = j + (j >= (int32_t)esc_pos ? 1 : 0);
-    }
-    uint32_t cw;
-    if (p >= 0) {
-      cw = ((uint32_t)S.lens[p] << 16) | (S.code[p] & 0xFFFFu);
-    } else if (cb_sym(keys[t]) == esc_sym) {
-      cw = esc_cw;  // a data symbol equal to esc_sym: the ESC code alone
-      atomicAdd(&a.esc_stats[1], cb_count(keys[t]));
-    } else {
-      cw = esc_cw | kRaw;  // outside the map: ESC code + raw16
-    }
-    a.cw_slot[slot_of(t)] = cw;
+  for (uint32_t p = tid; p < n; p += NT) {
+    const int32_t t = use_esc ? S.hidx[p] : (int32_t)p;
+    if (t >= 0) a.cw_slot[slot_of((uint32_t)t)] = ((uint32_t)S.lens[p] << 16) | (S.code[p] & 0xFFFFu);
+  }
+  if (!use_esc) return;
+  for (uint32_t i = tid; i < ni - keep; i += NT) {  // the entries left out: [0, s0) and [s0 + r, s1)
+    const uint32_t t = i < s0 ? i : i + r;
+    const bool coded = cb_sym(keys[t]) == esc_sym;  // a data symbol equal to esc_sym: the ESC code alone
+    if (coded) atomicAdd(&a.esc_stats[1], cb_count(keys[t]));
+    a.cw_slot[slot_of(t)] = coded ? esc_cw : esc_cw | kRaw;  // else ESC code + raw16
   }
 }
 
@@ -1533,7 +1518,7 @@ void launch_codebooks(const CodebookArgs &cba, const uint64_t *skeys, const uint
     hipLaunchKernelGGL((codebook_key_kernel<512, 256>), dim3(std::min(most[1], 2048u)), dim3(256), 0, s, cba, skeys,
                        sslots, lists + cap, n3 + 1);
   if (most[2])
-    hipLaunchKernelGGL((codebook_key_kernel<2048, 512>), dim3(std::min(most[2], 512u)), dim3(512), 0, s, cba, skeys,
+    hipLaunchKernelGGL((codebook_key_kernel<2048, 1024>), dim3(std::min(most[2], 512u)), dim3(1024), 0, s, cba, skeys,
                        sslots, lists + 2 * (size_t)cap, n3 + 2);
 }
 
