@@ -35,19 +35,42 @@ constexpr uint32_t kMaxProbes = 256;
 // The scales' ranks among their sorted distinct values: res[0] the number of
 // values, ranks[i] of scale i, values[] ascending. One workgroup over a set of
 // 65536 bits in LDS: a few microseconds, where the host took some 80 for its
-// tables of 65536 alone (of a 1024 x 4096 weight's 360 us a build).
+// tables of 65536 alone (of a 1024 x 4096 weight's 360 us a build). What bounds
+// it is the latency of one CU's loads, so they are 16 bytes wide where the array
+// is aligned, four in flight: 131,072 scales of a 4096 x 4096 weight 70 -> 20 us.
 __global__ __launch_bounds__(kUnitThreads) void scale_ranks(const uint16_t *__restrict__ scales, uint64_t n,
                                                             uint32_t *__restrict__ res, uint16_t *__restrict__ ranks,
                                                             uint16_t *__restrict__ values) {
-  constexpr uint32_t kWords = 65536 / 32, kPer = kWords / kUnitThreads;
-  __shared__ uint32_t s_set[kWords], s_before[kWords], s_tmp[16];
+  constexpr uint32_t kWords = 65536 / 32, kPer = kWords / kUnitThreads, kLoads = 4;
+  __shared__ uint32_t s_set[kWords], s_tmp[16];
+  __shared__ uint2 s_rank[kWords];  // a word of the set, and the values before it
   const uint32_t tid = threadIdx.x;
+  const uint64_t n8 = reinterpret_cast<uintptr_t>(scales) % 16 == 0 ? n / 8 : 0;  // 16-byte loads; the rest one by one
+  const uint4 *scales8 = reinterpret_cast<const uint4 *>(scales);
   for (uint32_t i = tid; i < kWords; i += kUnitThreads) s_set[i] = 0u;
   __syncthreads();
-  for (uint64_t i = tid; i < n; i += kUnitThreads) {
-    const uint32_t v = scales[i], bit = 1u << (v & 31u);
+  auto mark = [&](uint32_t v) {
+    const uint32_t bit = 1u << (v & 31u);
     if (!(s_set[v >> 5] & bit)) atomicOr(&s_set[v >> 5], bit);
+  };
+  for (uint64_t i = tid; i < n8; i += kLoads * kUnitThreads) {
+    uint4 v[kLoads];
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; ++j) {
+      const uint64_t at = i + j * kUnitThreads;
+      v[j] = scales8[at < n8 ? at : i];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; ++j) {
+      const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+      for (uint32_t h = 0; h < 4u; ++h) {
+        mark(w[h] & 0xFFFFu);
+        mark(w[h] >> 16);
+      }
+    }
   }
+  for (uint64_t i = 8 * n8 + tid; i < n; i += kUnitThreads) mark(scales[i]);
   __syncthreads();
   uint32_t mine = 0;
 #pragma unroll
@@ -57,17 +80,34 @@ __global__ __launch_bounds__(kUnitThreads) void scale_ranks(const uint16_t *__re
   for (uint32_t j = 0; j < kPer; ++j) {
     const uint32_t w = tid * kPer + j;
     uint32_t bits = s_set[w];
-    s_before[w] = at;
+    s_rank[w] = make_uint2(bits, at);
     while (bits) {
       values[at++] = (uint16_t)(32u * w + (uint32_t)__builtin_ctz(bits));
       bits &= bits - 1u;
     }
   }
   __syncthreads();
-  for (uint64_t i = tid; i < n; i += kUnitThreads) {
-    const uint32_t v = scales[i];
-    ranks[i] = (uint16_t)(s_before[v >> 5] + (uint32_t)__popc(s_set[v >> 5] & ((1u << (v & 31u)) - 1u)));
+  auto rank = [&](uint32_t v) {
+    const uint2 r = s_rank[v >> 5];
+    return r.y + (uint32_t)__popc(r.x & ((1u << (v & 31u)) - 1u));
+  };
+  for (uint64_t i = tid; i < n8; i += kLoads * kUnitThreads) {
+    uint4 v[kLoads];
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; ++j) {
+      const uint64_t at = i + j * kUnitThreads;
+      v[j] = scales8[at < n8 ? at : i];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kLoads; ++j) {
+      const uint64_t at = i + j * kUnitThreads;
+      uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+      for (uint32_t h = 0; h < 4u; ++h) w[h] = rank(w[h] & 0xFFFFu) | (rank(w[h] >> 16) << 16);
+      if (at < n8) reinterpret_cast<uint4 *>(ranks)[at] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
   }
+  for (uint64_t i = 8 * n8 + tid; i < n; i += kUnitThreads) ranks[i] = (uint16_t)rank(scales[i]);
   if (tid == 0) res[0] = total;
 }
 
