@@ -158,3 +158,44 @@ def test_builder_reports_no_memory():
     out = MPServe_cuda.huffman_build_fp8_decode_tables(bf.view(torch.bfloat16), q, sc, 7, 256)
     want = oracle.encode(bf.cpu().numpy(), q.cpu().numpy(), sc.cpu().numpy(), 7, 256)
     _same({x: v.cpu().numpy() for x, v in out.items()}, want)
+
+
+@pytest.mark.parametrize("entries", [65, 66, 127, 129, 511, 512, 513, 1025, 2046, 2047, 2048, 2049, 2300, 5000])
+def test_long_lists(entries):
+    """One key's list at the edges of the codebook kernels' sizes: few ties and many, with ESC past 2^L."""
+    print(f"[units] list of {entries}", flush=True)
+    rng = np.random.default_rng(entries)
+    vals = np.concatenate([np.arange(entries), (entries * rng.random(90000) ** (1.5 + entries % 7)).astype(np.int64)])
+    vals = vals[:vals.size // 64 * 64] if entries != 513 else np.repeat(np.arange(entries), 128)  # 513: all counts tie
+    bf = rng.permutation(vals).astype(np.uint16).reshape(-1, 64)
+    q = np.full(bf.shape, 5, dtype=np.uint8)
+    sc = np.array([0x1C00], dtype=np.uint16)
+    for L in (7, 11):
+        _same(_fp8(bf, q, sc, L, 256), oracle.encode(bf, q, sc, L, 256))
+    rows = np.full(bf.shape[0], 0x3C00, dtype=np.uint16)
+    args = (torch.from_numpy(bf).to(DEV).view(torch.bfloat16), torch.from_numpy(q).to(DEV), torch.from_numpy(rows), 11, 256)
+    for by_scale in (True, False):
+        op = ("huffman_build_awq_int4_bucket_decode_tables" + ("_by_scale" if by_scale else ""))
+        got = getattr(MPServe_cuda, op)(*args, *((1024,) if by_scale else ()))
+        _same({x: v.cpu().numpy() for x, v in got.items()}, oracle.awq_encode(bf, q, rows, 11, 256, 1024, by_scale))
+
+
+@pytest.mark.parametrize("n,shift,distinct", [
+    (1, 0, 8), (7, 0, 8), (8, 0, 8), (9, 0, 8), (8192, 0, 8), (33000, 0, 8), (33000, 1, 1), (33001, 8, 300),
+    (8191, 0, 4095), (8192, 0, 1), (8193, 0, 4096),    # from 8192 rows they are dealt to their scales on the GPU
+    (9000, 0, 4096), (9000, 0, 4097), (20000, 0, 20000),  # with up to 4096 distinct scales
+    (600000, 0, 1000),                                 # tiles of more than 2048 rows
+])
+def test_scales_ranked_and_dealt(n, shift, distinct):
+    """Scales in memory at an offset, in numbers that leave loads, waves and tiles incomplete."""
+    print(f"[units] {n} scales of {distinct}, shift {shift}", flush=True)
+    rng = np.random.default_rng(n)
+    bf, q = rng.integers(0, 50, size=(n, 2)).astype(np.uint16), rng.integers(0, 4, size=(n, 2)).astype(np.uint8)
+    sc = rng.choice(65536, size=distinct, replace=False).astype(np.uint16)
+    sc = rng.permutation(np.concatenate([sc, rng.choice(sc, size=max(0, n - distinct))])[:n])
+    base = torch.zeros(n + shift, dtype=torch.int16, device=DEV)
+    base[shift:] = torch.from_numpy(sc.view(np.int16)).to(DEV)
+    got = MPServe_cuda.huffman_build_fp8_decode_tables(
+        torch.from_numpy(bf.view(np.int16)).to(DEV).view(torch.bfloat16), torch.from_numpy(q).to(DEV),
+        base[shift:].view(torch.uint16), 7, 64)
+    _same({x: v.cpu().numpy() for x, v in got.items()}, oracle.encode(bf, q, sc, 7, 64))
