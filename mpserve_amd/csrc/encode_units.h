@@ -656,7 +656,7 @@ __global__ __launch_bounds__(kUnitThreads) void bucket_starts(const Unit *__rest
                                                               uint32_t *__restrict__ piece_bits,
                                                               uint32_t *__restrict__ startbit,
                                                               uint32_t *bucket_bits, int64_t *__restrict__ bit_base,
-                                                              uint32_t *done) {
+                                                              uint32_t *done, int64_t *__restrict__ end) {
   __shared__ uint32_t s_tmp[16];
   __shared__ bool s_last;
   const uint32_t b = blockIdx.x, t = threadIdx.x;
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(kUnitThreads) void bucket_starts(const Unit *__rest
     uint32_t sum = 0;
     const uint32_t first = block_exclusive_scan(words, s_tmp, &sum);
     if (in) bit_base[b0 + t] = (int64_t)((run + first) << 6);
-    if (b0 + t + 1u == B) bit_base[B] = (int64_t)(((run + first) << 6) + bits);
+    if (b0 + t + 1u == B) bit_base[B] = *end = (int64_t)(((run + first) << 6) + bits);
     run += sum;
   }
 }

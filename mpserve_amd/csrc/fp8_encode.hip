@@ -1771,7 +1771,7 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
   // --- one device block: the host-built arrays (`put`), then work memory (`take`) ---
   // flags: [0] overflow, [1] error bits, [2..3] esc stats, [4] compact count, [5..7] codebook
   // classes, [8..10] keys, entries and most entries of a scale (number_keys), [11] finished
-  // workgroups (bucket_starts)
+  // workgroups and [12..13] the stream's end (bucket_starts)
   constexpr int kFlags = 16;
   uint32_t hflags[kFlags] = {};
   std::vector<char> host;
@@ -1998,13 +1998,14 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     if (most <= 6144) codes_pass(unit_codes<8192>);
     else codes_pass(unit_codes<16384>);
     hipLaunchKernelGGL(bucket_starts, dim3(B), dim3(kUnitThreads), 0, s, ua.units, at32(o_bunit), d_lane_base,
-                       (uint32_t)kth, at32(o_pieces), startbit, at32(o_bbits), bit_base, flags + 11);
+                       (uint32_t)kth, at32(o_pieces), startbit, at32(o_bbits), bit_base, flags + 11,
+                       reinterpret_cast<int64_t *>(flags + 12));
     HC(hipGetLastError());
-    int64_t end = 0;
-    HC(hipMemcpyAsync(&end, bit_base + B, 8, hipMemcpyDeviceToHost, s));
     HC(hipMemcpyAsync(hflags, flags, sizeof(hflags), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
     if ((rc = check_errors()) != MPS_OK) return rc;
+    int64_t end = 0;  // of the bitstream, in bits
+    std::memcpy(&end, hflags + 12, sizeof(end));
     W = (end + 63) >> 6;
     OUT(bitstream, uint64_t, 12, (size_t)W);
     if (W) {
