@@ -76,12 +76,14 @@ int mps_fp8_decode(const mps_fp8_tensor *tensor, int64_t max_len, void *stream);
  * column ranges and bit bases to order the work largest first and to build
  * one work record per bucket, and copies the descriptors into one device
  * allocation the plan owns (with its own status word). When the buckets are
- * few or uneven for the device's CUs, large buckets are split into row
- * ranges: a kernel on `stream` walks their substreams' code lengths once and
- * records each substream's bit position at every range's first row (the lane
- * checkpoints, also owned by the plan). A sidecar whose bucket metadata, row
- * indices, start bits, tables, FP8 bytes or bitstream is rewritten needs a
- * new plan in that case. The pointed-to sidecars must stay alive while the
+ * few or uneven for the device's CUs, large buckets are split into ranges of
+ * rows (of steps of k elements, where the columns are no multiple of k): a
+ * kernel on `stream` walks their substreams' code lengths once and records
+ * each substream's bit position at every range's start (the lane checkpoints,
+ * also owned by the plan). Small buckets whose table ids are equal (128 x 128
+ * blocks of one scale) are grouped into items that set the tables up once. A
+ * sidecar whose bucket metadata, row indices, start bits, tables, FP8 bytes or
+ * bitstream is rewritten needs a new plan in either case. The pointed-to sidecars must stay alive while the
  * plan is used. Launches are persistent: one workgroup per CU takes work
  * items from a queue in the plan's memory, which each launch leaves as it
  * found it. The plan holds 32 such queues and gives each stream that launches
@@ -107,8 +109,8 @@ int mps_fp8_plan_decode(mps_fp8_plan *plan, void *stream);
  * This serves the drop-in decode op's per-sidecar plan cache and the vLLM
  * method's scratch slots. */
 int mps_fp8_plan_decode_into(mps_fp8_plan *plan, uint16_t *out, void *stream);
-/* The plan's work list (for profiling tools): work items (buckets, and the row
- * ranges of the buckets it split), bytes of LDS per workgroup. */
+/* The plan's work list (for profiling tools): work items (buckets, runs of
+ * them, and the ranges of the buckets it split), bytes of LDS per workgroup. */
 int mps_fp8_plan_info(const mps_fp8_plan *plan, int64_t *work_items, int64_t *lds_bytes);
 /* Read and clear the plan's MPS_STATUS_* flags; synchronises `stream` first. */
 int mps_fp8_plan_read_status(mps_fp8_plan *plan, void *stream, uint32_t *status_out);
@@ -120,7 +122,7 @@ int mps_fp8_plan_destroy(mps_fp8_plan *plan);
  * allocating routine and does not synchronise: the descriptors (copied from
  * the host array on `stream`) and one work record per bucket go into a static
  * device array of 4 MiB that each device holds from library load to the end
- * of the process. Buckets are not split into row ranges. Flags go to the
+ * of the process. Buckets are neither split nor grouped. Flags go to the
  * device status word (mps_fp8_read_status). Calls that overlap on one device
  * share that array and race: issue them on one stream, or order them.
  * Larger inputs, and a `stream` that is capturing a graph (the descriptor

@@ -12,7 +12,7 @@ The reference binds two builders and two decoders for AWQ int4 weights
   kernel :477-589).
 
 Same op and argument names, defaults, dict keys, argument checks in order and
-wording. The builders run on the GPU (libmpserve_amd.so, mps_awq_encode) and
+wording. The builders run on the GPU (libmpserve_amd.so, mps_awq_encode_alloc) and
 give the reference builders' bytes; CPU inputs come back as CPU tensors. The
 decoders run on the current stream of the int4 tensor's device (mps_awq_decode).
 """
