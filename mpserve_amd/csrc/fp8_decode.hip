@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <queue>
+#include <numeric>
 #include <vector>
 
 #include "fp8_decode_device.h"
@@ -476,7 +477,7 @@ int mps_fp8_plan_create(const mps_fp8_tensor *tensors, int64_t count, void *stre
   // on the k = 1024 and fast paths larger than total / (2 * CUs) elements are
   // split into row ranges of at most that size (and at least 64 elements per
   // substream, 16 groups, so that a range's set-up stays small beside its
-  // decode). Each range starts from lane checkpoints (fp8_checkpoints).
+  // decode; fewer where CUs would be idle, min_lane below). Each range starts from lane checkpoints (fp8_checkpoints).
   //
   // A fast-path bucket with k_eff 256 or 512 fills only k_eff of a
   // workgroup's 1024 work-items, and its tables allow one workgroup per CU. So
@@ -519,13 +520,20 @@ int mps_fp8_plan_create(const mps_fp8_tensor *tensors, int64_t count, void *stre
   auto per_cut = [&](size_t i) { return is_flat(i) ? 1 : bucket[i].cl / bucket[i].k_eff; };
   // cost of `rows` rows (slabs) of split-capable bucket i decoded by one group of work-items
   auto rows_cost = [&](size_t i, int64_t rows) { return rows * (int64_t)per_cut(i) * 1024 + kItemSetup; };
+  // Fewest elements per substream of a range: 64 where that gives every CU one
+  // (4096 x 4096), fewer below, since a set-up costs a CU that would be idle
+  // nothing; at least 16. Measured, k = 1024, a plan of one tensor, with 64 and now:
+  // 512 x 4096 15.7 -> 10.0 us, 1024 x 4096 20.0 -> 12.3 (32: 13.5), 1000 x 3000
+  // 20.1 -> 12.1, 2048 x 4096 19.6 -> 16.6; 2048 x 2048, k = 256: 20.8 -> 12.4 us.
+  const int64_t all = std::accumulate(elems.begin(), elems.end(), (int64_t)0);
+  const int64_t min_lane = std::min<int64_t>(64, std::max<int64_t>(16, all / (1024 * ncu)));
   for (size_t i = 0; i < bucket.size(); ++i) {
     const WorkItem &w = bucket[i];
     const int64_t ke = std::max<int64_t>(w.k_eff, 1);
     whole_cost[i] = (elems[i] + ke - 1) / ke * 1024 + kItemSetup;
     if ((w.path != kPathK1024 && w.path != kPathFast && !is_flat(i)) || cuts(i) < 2) continue;
     const int32_t P = per_cut(i);
-    const int32_t min_rows = std::max<int32_t>(1, (64 + P - 1) / P);
+    const int32_t min_rows = std::max<int32_t>(1, ((int32_t)min_lane + P - 1) / P);
     const int64_t maxr = std::max<int64_t>(1, cuts(i) / min_rows);
     const int64_t S = w.path != kPathK1024 && (w.k_eff == 256 || w.k_eff == 512) ? 1024 / w.k_eff : 1;
     // range rows ride in 8 bits of the work record (fast buckets hold <= 128 rows), slabs in 19
@@ -550,7 +558,7 @@ int mps_fp8_plan_create(const mps_fp8_tensor *tensors, int64_t count, void *stre
   };
   int64_t total = 0;
   for (size_t i = 0; i < bucket.size(); ++i) total += whole_cost[i] - kItemSetup;
-  const int64_t cap = std::max<int64_t>(total / (MPS_SPLIT_DIV * ncu), 65536);
+  const int64_t cap = std::max<int64_t>(total / (MPS_SPLIT_DIV * ncu), 1024 * min_lane);
   std::vector<int64_t> ni(bucket.size(), 1);  // items of each bucket
   for (size_t i = 0; i < bucket.size(); ++i) {
     const int64_t c = whole_cost[i] - kItemSetup;

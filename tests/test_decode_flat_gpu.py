@@ -112,3 +112,18 @@ def test_flat_runs_share_tables(k):
     want = bf.copy()
     want[17 * bs:18 * bs, 5 * bs:6 * bs] = 0
     np.testing.assert_array_equal(out.view(torch.uint16).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n,m,k", [
+    (256, 1024, 1024), (300, 3072, 1024), (512, 4096, 1024), (140, 14336, 1024),  # P of 1, 3, 4, 14 blocks a row
+    (1000, 3000, 1024), (257, 2001, 512),                                         # flat
+    (512, 256, 256), (700, 1536, 512), (512, 4096, 256),                          # ranges side by side
+])
+def test_small_tensors_in_short_ranges(n, m, k):
+    """A tensor of fewer than 64 elements a lane and CU: ranges of down to 16 elements a lane."""
+    print(f"[flat] short ranges {n}x{m} k{k}", flush=True)
+    bf, q, sc = synth(n, m, seed=n + m)
+    sc[:] = sc[0]  # buckets of 128 rows
+    side = oracle.encode(bf, q, sc, 7, k)
+    items = _check(bf, q, [side])
+    assert items > side["bucket_table_i32"].shape[0]
