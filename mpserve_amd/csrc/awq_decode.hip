@@ -453,11 +453,20 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
   }
   // Row ranges: a slab-path row bucket with more than total / (2 * CUs) elements
   // is split into row ranges of at least 64 elements a lane, each started from
-  // lane checkpoints that one walk over the bucket's substreams finds.
+  // lane checkpoints that one walk over the bucket's substreams finds (16: 1024 x
+  // 4096, k = 1024, 20.2 -> 24.0 us: more table set-ups than CUs).
   // A bucket with k 256 or 512 (k_of_rec) is always cut, into up to 1024 / k
   // ranges a record (one record per total / (2 * CUs) elements), which share
   // the record's set-up.
   const int64_t target = std::max<int64_t>(1, total / (2 * (int64_t)std::max(cus, 1)));
+  // Fewest elements a lane of a range that shares its record's set-up, or of a flat
+  // one: 64 where that gives every CU one (4096 x 4096), fewer in smaller plans,
+  // whose idle CUs pay a set-up for nothing; at least 16, below which a range is all
+  // set-up. One weight's plan, the per-record rule of 64 and now: 1024 x 4096, k =
+  // 256, 27.8 -> 17.7 us; 2048 x 2048, k = 256, 28.0 -> 17.5; 2048 x 4096, k = 512,
+  // 26.5 -> 20.6; 128-column groups, 1024 x 4096, k = 256, 25.7 -> 22.6 us.
+  const int64_t min_lane =
+      std::min<int64_t>(64, std::max<int64_t>(16, total / (kAwqBlock * (int64_t)std::max(cus, 1))));
   std::vector<AwqSplitJob> jobs;
   std::vector<size_t> job_rec;  // the base record each job splits
   int64_t ck_words = 0;
@@ -467,13 +476,13 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
     if (k_of_rec[r] > 0) {
       // units: rows, or slabs of k / 128 groups (by-scale, at most 128 a range: the
       // slab path keeps a wave's 128 group bases in two registers)
-      // More than one record only while each range keeps >= 64 elements a lane.
+      // More than one record only while each range keeps >= min_lane elements a lane.
       const int64_t S = kAwqBlock / k_of_rec[r];
       // (flat: slabs of k elements, at most P a range)
       const bool flat = gps_of_rec[r] < 0;
       const int64_t gps = gps_of_rec[r];
       const int64_t units = flat || P > 0 ? rows : (rows + gps - 1) / gps;
-      const int64_t min_units = flat ? 64 : P > 0 ? (64 + P - 1) / P : 64;
+      const int64_t min_units = P > 0 && !flat ? (min_lane + P - 1) / P : min_lane;
       const int64_t recs = std::min(std::max<int64_t>(1, (w.elems + target - 1) / target),
                                     std::max<int64_t>(1, units / (S * min_units)));
       int64_t ranges = std::min<int64_t>(units, S * recs);

@@ -99,3 +99,18 @@ def test_by_scale_groups(n, m, group, k, cap, monkeypatch):
     s = w.scale_u16.view(torch.int16)
     s.copy_(torch.where(torch.arange(s.numel(), device=DEV).view(s.shape) % 3 == 0, s, s.reshape(-1)[0]))  # large buckets
     _check(w.bf16, w.int4_u8, w.scale_u16, k, True, cap, monkeypatch, False)
+
+
+@pytest.mark.parametrize("n,m,group,k", [
+    (512, 4096, None, 1024), (140, 14336, None, 1024),                             # 4 and 14 blocks a row
+    (512, 1024, None, 256), (300, 2048, None, 512),                                # ranges side by side
+    (700, 3000, None, 1024), (257, 2001, None, 512),                               # flat
+    (512, 4096, 128, 256), (512, 4096, 128, 1024), (512, 2048, 64, 512),           # slabs of groups
+])
+def test_small_weights_in_short_ranges(n, m, group, k, monkeypatch):
+    """A weight of fewer than 64 elements a lane and CU: ranges of down to 16 elements a lane."""
+    print(f"[awq flat] short ranges {n}x{m} group {group} k{k}", flush=True)
+    w = make_awq_weight(n, m, group, seed=n + m, device=DEV)
+    s = w.scale_u16.view(torch.int16)
+    s.copy_(s.reshape(-1)[0].clone().expand_as(s))  # buckets of 128 rows, or of 1024 groups
+    _check(w.bf16, w.int4_u8, w.scale_u16, k, group is not None, 1024, monkeypatch, False)
