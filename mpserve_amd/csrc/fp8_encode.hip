@@ -2411,10 +2411,14 @@ int to_alloc(const In *in, int (*make)(const In *, EncodeSpec *), void *stream, 
   last_error().clear();
   if (!in || !alloc || !sizes17 || !stats4) return fail(MPS_ERR_INVALID_ARGUMENT, "inputs must be defined");
   EncodeSpec sp;
-  const int rc = make(in, &sp);
-  return rc != MPS_OK ? rc : no_throw([&] {
-    return encode_impl(sp, reinterpret_cast<hipStream_t>(stream), alloc, ctx, sizes17, stats4);
-  });
+  int rc = make(in, &sp);
+  if (rc != MPS_OK) return rc;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  rc = no_throw([&] { return encode_impl(sp, s, alloc, ctx, sizes17, stats4); });
+  // Complete on return, also after a failure: the outputs and the inputs may then be
+  // used, rewritten or freed on any stream, as after the handle's calls.
+  const hipError_t e = hipStreamSynchronize(s);
+  return rc == MPS_OK && e != hipSuccess ? hip_fail(e, "sidecar builder") : rc;
 }
 }  // namespace
 
