@@ -270,12 +270,13 @@ int mps_awq_encode(const mps_awq_encode_in *in, void *stream, mps_fp8_sidecar **
  * aligned: each non-empty output once, by its slot (0..16, the handle's order),
  * and workspaces as slot -1; it returns NULL when it has none (then
  * MPS_ERR_NO_MEMORY). Called on the calling thread. sizes17 and stats4 are as
- * mps_fp8_sidecar_sizes and mps_fp8_sidecar_stats give them. `stream` is
- * synchronised before the return, also after an error: outputs, inputs and
- * workspaces may then be used or freed on any stream. No counterpart in the
- * reference, whose outputs are host tensors; it spares a serving or compressing
- * program, whose allocator caches memory, the builder's own device allocations
- * and the copies out of a handle. */
+ * mps_fp8_sidecar_sizes and mps_fp8_sidecar_stats give them. The last passes may
+ * still be running on `stream` after MPS_OK: the caller synchronises it before it
+ * uses outputs or inputs on another stream or on the host (the Python ops do so
+ * before they return), and frees workspaces in stream order. After an error the
+ * stream is idle. No counterpart in the reference, whose outputs are host tensors;
+ * it spares a serving or compressing program, whose allocator caches memory, the
+ * builder's own device allocations and the copies out of a handle. */
 typedef void *(*mps_encode_alloc)(void *ctx, int32_t slot, int64_t bytes);
 int mps_fp8_encode_alloc(const mps_fp8_encode_in *in, void *stream, mps_encode_alloc alloc, void *ctx,
                          int64_t *sizes17, int64_t *stats4);

@@ -78,6 +78,13 @@ class BuilderOutputs:
         _native.check(rc)
         return sizes, stats
 
+    def complete(self) -> None:
+        """Waits for the build's last passes: its outputs and inputs may then be used, rewritten
+        or freed on any stream (as after the reference's host builders). Called with the result
+        made up, so that the passes run beside that work (14336 x 4096: 547 us a build; waiting in the
+        native call 565; not waiting, which raced with work on other streams, 515)."""
+        torch.cuda.current_stream(self._device).synchronize()
+
     def tensor(self, slot: int, shape, on_host: bool) -> torch.Tensor:
         t = self._out.get(slot)
         if t is None:

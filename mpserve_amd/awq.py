@@ -105,6 +105,7 @@ def _build(bf16, int4, scales, max_len, threads, group_cap, by_scale: bool, with
         shape = {0: (G, 1 << L), 1: (G, max(1, (1 << L) // 2)), 7: (B, 16), 10: (B, int(threads) + 1)}
         out: Dict[str, torch.Tensor] = {key: mem.tensor(slot, shape.get(slot, (int(sizes[slot]),)), on_host)
                                         for key, slot, _ in keys}
+        mem.complete()
     if with_stats:
         return out, {"esc_keys": int(stats[0]), "esc_collisions": int(stats[1])}
     return out

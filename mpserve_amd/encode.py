@@ -78,6 +78,7 @@ def build_fp8_sidecar(bf16_params: torch.Tensor, fp8_params: torch.Tensor, scale
         shapes = _shapes(int(sizes[2]), int(sizes[4]), int(threads_per_block), int(max_len), sizes)
         out: Dict[str, torch.Tensor] = {key: mem.tensor(i, shp, on_host)
                                         for i, ((key, _), shp) in enumerate(zip(_OUTPUTS, shapes))}
+        mem.complete()
     if with_stats:
         return out, {"esc_keys": int(stats[0]), "esc_collisions": int(stats[1]), "distinct_pairs": int(stats[2]),
                      "hash_slots": int(stats[3])}
