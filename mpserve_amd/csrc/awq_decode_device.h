@@ -1060,7 +1060,11 @@ __device__ __forceinline__ void awq_slab_bucket(const mps_awq_tensor &T, const A
   auto gbase = [&](uint32_t gi, int32_t row, int32_t col, bool &bad) -> uint32_t {
     if (gi >= (uint32_t)nr) return 0u;
     bad |= row < 0 || (int64_t)row >= T.n || col < 0 || (int64_t)col + cl > T.m;
-    return (uint32_t)row * m + (uint32_t)col + (slabs ? wcol : 0u);
+    // (128 columns spelt out: what this lambda captures moves the compiler's register choices, and
+    // with wcol in every kernel awq_decode_plan<3> and <5> reloaded 5788 and 5314 spilled scalars
+    // instead of 3554 and 3370: layers that mix row ranges with k = 256 or tiny buckets 238 -> 229 us.)
+    if constexpr (kAnyGroup) return (uint32_t)row * m + (uint32_t)col + (slabs ? wcol : 0u);
+    else return (uint32_t)row * m + (uint32_t)col + (by_scale ? ((w & 1u) << 6) : 0u);
   };
   bool bad_row = kFlat && nr > kFlatMaxRows;
   const uint32_t base_lo = gbase(gi0, row0, col0, bad_row);
