@@ -25,7 +25,7 @@ LIB = os.path.join(HERE, "libmpserve_amd.so")
 ARCH = os.environ.get("MPS_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["fp8_decode.hip", "fp8_decode_flat.hip", "fp8_encode.hip", "awq_decode.hip",
-           "awq_decode_flat.hip"]
+           *(f"awq_decode_flat_{m}.hip" for m in (31, 11, 30, 13, 14))]
 
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",

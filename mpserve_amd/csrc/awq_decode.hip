@@ -13,14 +13,10 @@
 #include <vector>
 
 #include "awq_decode_device.h"
+#include "awq_decode_flat.h"
 #include "mps_common.h"
 
 namespace mps {
-
-// The plan launch that also takes flat ranges (awq_decode_flat.hip; work: AwqWork records).
-void launch_awq_flat_plan(const mps_awq_tensor *tensors, const void *work, int64_t nwork, const uint32_t *ckpt,
-                          uint32_t *status, int64_t out_delta, uint32_t *queue, unsigned grid, hipStream_t stream);
-
 namespace {
 
 template <int kSplit>
@@ -212,7 +208,8 @@ struct mps_awq_plan {
   uint32_t *d_ckpt = nullptr;  // lane checkpoints of the row buckets split into ranges
   int64_t splits = 0;          // row buckets split into ranges
   // bit 0: some work record is a row range (kind 2); bit 1: ranges side by side
-  // (kind 3); bit 2: tiny buckets (kind 0 with `tiny`); bit 3: flat ranges (kind 4)
+  // (kind 3); bit 2: tiny buckets (kind 0 with `tiny`); bit 3: flat ranges (kind 4);
+  // bit 4: by-scale groups of other sizes than 128 columns
   int ranges_mode = 0;
 };
 
@@ -593,11 +590,11 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
   plan->ranges_mode = (std::any_of(items.begin(), items.end(), [](const AwqWork &w) { return w.tiny != 0; }) ? 4 : 0) |
                       (std::any_of(items.begin(), items.end(), [](const AwqWork &w) { return w.kind == 2; }) ? 1 : 0) |
                       (std::any_of(items.begin(), items.end(), [](const AwqWork &w) { return w.kind == 3; }) ? 2 : 0) |
+                      (std::any_of(items.begin(), items.end(), [](const AwqWork &w) { return w.kind == 4; }) ? 8 : 0) |
                       (std::any_of(items.begin(), items.end(), [&](const AwqWork &w) {
-                         return w.kind == 4 || ((w.kind == 1 || w.kind == 3) && tensors[w.tensor].group_col_start &&
-                                                tensors[w.tensor].group_size != 128);
+                         return w.kind != 0 && tensors[w.tensor].group_col_start && tensors[w.tensor].group_size != 128;
                        })
-                           ? 8
+                           ? 16
                            : 0);
   *plan_out = plan;
   return MPS_OK;
@@ -627,10 +624,17 @@ static int awq_plan_launch(mps_awq_plan *plan, int64_t out_delta, uint32_t *stat
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kAwqBlock), 0, reinterpret_cast<hipStream_t>(stream), plan->d_tensors,
                        plan->d_work, plan->nwork, plan->d_ckpt, status, out_delta, queue);
   };
-  if (plan->ranges_mode & 8)
-    launch_awq_flat_plan(plan->d_tensors, plan->d_work, plan->nwork, plan->d_ckpt, status, out_delta, queue, grid,
-                         reinterpret_cast<hipStream_t>(stream));
-  else switch (plan->ranges_mode) {
+  if (plan->ranges_mode & (8 | 16)) {
+    const AwqFlatLaunch a{plan->d_tensors, plan->d_work, plan->nwork, plan->d_ckpt, status, out_delta, queue, grid,
+                          reinterpret_cast<hipStream_t>(stream)};
+    const int mode = plan->ranges_mode;
+    auto within = [&](int paths) { return (mode & ~paths) == 0; };
+    if (within(13)) launch_awq_flat_13(a);
+    else if (within(14)) launch_awq_flat_14(a);
+    else if (within(11)) launch_awq_flat_11(a);
+    else if (within(30)) launch_awq_flat_30(a);
+    else launch_awq_flat_31(a);
+  } else switch (plan->ranges_mode) {
     case 0: launch(awq_decode_plan<0>); break;
     case 1: launch(awq_decode_plan<1>); break;
     case 2: launch(awq_decode_plan<2>); break;

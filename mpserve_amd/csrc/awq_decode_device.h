@@ -27,7 +27,7 @@
 // 512-work-item workgroups per bucket, each with its own copy of the tables.
 //
 // Included by awq_decode.hip (the host side and the kernels without flat ranges)
-// and awq_decode_flat.hip (the plan kernel with every path).
+// and awq_decode_flat_*.hip (the plan kernels with them, awq_decode_flat.h).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -859,12 +859,12 @@ __device__ __forceinline__ void awq_slab_decode(const mps_awq_tensor &T, const u
 // and end bits; (2) the tables' slices and the lane's first bitstream words.
 // Thread tid expands entries 32c .. 32c+31 of the table of int4 value tid / 64
 // (c = tid % 64).
-// kRanged 3: flat ranges side by side (kind 4: k 256, 512 or 1024, rows of any
-// width), a range being slabs [range * range_rows, + range_rows) of the bucket.
 // kRanged: 0 a whole bucket, 1 a row range (kind 2), 2 row ranges side by side
 // (kind 3: k 256 or 512, the work-items [s k, (s + 1) k) decode range
 // wk.range + s, from checkpoint rows range + s and range + s + 1 of a full
-// [ranges + 1][k] set); whole buckets compile without the range logic.
+// [ranges + 1][k] set), 3 flat ranges side by side (kind 4: k 256, 512 or 1024,
+// rows of any width, a range being slabs [range * range_rows, + range_rows) of
+// the bucket); whole buckets compile without the range logic.
 // A by-scale record may hold a run of buckets b with identical table ids: the
 // first that gets past its checks (`tables`) loads and expands the tables and
 // records in run_flags that it did (kRunTables) and whether they have an ESC
@@ -1229,7 +1229,7 @@ __device__ __forceinline__ void awq_slab_bucket_wave(const mps_awq_tensor &T, in
 // buffer laid out like, but other than, the one it was created with).
 // kRanges: bit 0, the plan has row ranges (kind 2 records); bit 1, row ranges
 // side by side (kind 3); bit 2, tiny buckets (awq_tiny_lane); bit 3, flat ranges
-// (kind 4) and by-scale groups of other sizes than 128 columns. Plans without
+// (kind 4); bit 4, by-scale groups of other sizes than 128 columns, flat or not. Plans without
 // them launch the instantiation that leaves that path out: the range path's
 // code in the same kernel measured 4.6% slower on a by-scale layer, the tiny
 // path's 4.4% slower on a row-bucket layer.
@@ -1280,7 +1280,7 @@ __device__ __forceinline__ void awq_plan_record(const mps_awq_tensor *__restrict
                                                 const uint32_t *__restrict__ ckpt, uint32_t *status,
                                                 int64_t out_delta, uint32_t *__restrict__ lut,
                                                 uint32_t *__restrict__ s_base) {
-  constexpr bool kAny = (kRanges & 8) != 0;
+  constexpr bool kAny = (kRanges & 16) != 0;
   const int4 w = make_int4(wk.tensor, wk.bucket, wk.nsub, wk.kind);
   mps_awq_tensor T = tensors[w.x];
   T.out += out_delta;

@@ -1,10 +1,14 @@
 """Plans of weights that take different paths in one launch: each set of paths has a kernel of
 its own (awq_decode_plan<kRanges>, fp8_decode_plan), and every weight decodes as in a plan alone."""
+import numpy as np
 import pytest
 import torch
 
+import oracle
 from mpserve_amd import awq
+from mpserve_amd.decode import DecodePlan
 from mpserve_amd.synthetic import make_awq_weight
+from tests.helpers import synth, to_torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -48,3 +52,44 @@ def _check_awq(shapes, monkeypatch):
 def test_awq_aligned_weights_of_several_kinds(shapes, monkeypatch):
     print(f"[mixed] awq {shapes}", flush=True)
     _check_awq(shapes, monkeypatch)
+
+
+FLAT = (300, 1000, None, 1024)     # rows that are no multiple of the substreams
+FLAT256 = (140, 1021, None, 256)
+OTHER = (512, 1024, 64, 1024)      # groups of another size than 128 columns
+OTHER256 = (600, 1024, 64, 256)
+
+
+@pytest.mark.parametrize("shapes", [
+    (ROWS, FLAT), (GROUPS, FLAT, TINY), (ROWS, TINY, FLAT256),           # <13>
+    (BESIDE, FLAT256), (BESIDE, TINY, FLAT),                             # <14>
+    (ROWS, BESIDE, FLAT),                                                # <11>
+    (GROUPS, OTHER), (GROUPS, OTHER, FLAT, TINY), (BESIDE, OTHER256), (OTHER, OTHER256, FLAT256),  # <30>
+    (ROWS, BESIDE, TINY, FLAT), (ROWS, OTHER, FLAT), (ROWS, BESIDE, OTHER, TINY),                  # <31>
+])
+def test_awq_aligned_and_flat_weights(shapes, monkeypatch):
+    print(f"[mixed] awq {shapes}", flush=True)
+    _check_awq(shapes, monkeypatch)
+
+
+@pytest.mark.parametrize("shapes", [
+    ((512, 4096, 1024), (140, 5000, 1024)),                        # a large flat share
+    ((512, 4096, 1024), (2, 1000, 1024)), ((512, 4096, 256), (2, 1021, 256)),  # few and short flat buckets
+    ((512, 4096, 1024), (1, 10000, 512)),                          # few, but long
+    ((512, 4096, 1024), (512, 1024, 256), (300, 1021, 512), (3, 700, 1024)),
+])
+def test_fp8_aligned_and_flat_weights(shapes):
+    print(f"[mixed] fp8 {shapes}", flush=True)
+    items = []
+    for n, m, k in shapes:
+        bf, q, sc = synth(n, m, seed=n + m + k)
+        sc[:] = sc[0]
+        side = to_torch(oracle.encode(bf, q, sc, 7, k), DEV)
+        out = torch.full((n, m), float("nan"), dtype=torch.bfloat16, device=DEV)
+        items.append((bf, (torch.from_numpy(q).to(DEV), side, out)))
+    plan = DecodePlan([x for _, x in items])
+    for _ in range(2):
+        plan.decode()
+    assert plan.read_status() == 0
+    for (bf, (_, _, out)), s in zip(items, shapes):
+        np.testing.assert_array_equal(out.view(torch.uint16).cpu().numpy(), bf, err_msg=str(s))
