@@ -19,6 +19,7 @@ decoders run on the current stream of the int4 tensor's device (mps_awq_decode).
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Dict
 
 import torch
@@ -165,6 +166,43 @@ def _plan_cache():
     return _AWQ_PLANS
 
 
+@functools.lru_cache(maxsize=None)
+def _compute_units(index: int) -> int:
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
+def _op_takes_plan(k: int, n: int, m: int, buckets: int, rows: int, group_size: int, cus: int) -> bool:
+    """Does a decoder launch the sidecar's cached plan from its second call on? Else, and on
+    the first call, it decodes over whole buckets, as the reference does: the kernel with two
+    workgroups a bucket up to half as many buckets as CUs, with one past it.
+
+    ``rows``: entries of the row (group) list; ``group_size``: 0 for row sidecars. Sidecars of
+    whole blocks (k = 1024 rows, rows of a multiple of 4k columns, 128-column groups) always do.
+    For the others, by measurement on 256 CUs (direct, plan in us):
+    - up to 128 buckets a plan's set-up pays from about 6 elements a substream in the mean
+      bucket: k = 256, 8 x 1500 rows (5.9) 11.1, 11.7; 300 x 300 (5.1) 14.5, 13.0; 600 x 300
+      (7.2) 17.3, 13.5; k = 512, 8 x 3000 (5.9) 11.2, 12.7; 40 x 3000 (7.3) 15.0, 13.7;
+    - 129 to 256 buckets take the direct kernel two rounds, and the plan pays in any case:
+      k = 256, 1000 x 60 (131 buckets) 18.4, 13.3; past 256 the first rule holds again: 4096 x 8
+      (279 buckets) 12.5, 21.6; 4096 x 4096 in groups of 64 (407) 163, 43;
+    - rows too narrow for flat ranges (a range holds at most 126 rows and should span 32
+      slabs) stay on the plan's per-lane path, which only pays in the second case: k = 512,
+      1024 x 128 rows (110 buckets) 11.6, 13.0; k = 256, 600 x 60 (124) 10.6, 13.2."""
+    if k not in (256, 512, 1024) or buckets <= 0:
+        return False
+    if group_size:
+        if group_size == 128:
+            return True
+        slab = group_size >= 1024 or (64 <= group_size <= k and group_size & (group_size - 1) == 0)
+        if not slab:
+            return False
+    else:
+        if k == 1024 or m % (4 * k) == 0:
+            return True
+        slab = 126 * (n * m // max(1, rows)) // k >= 32  # (the mean row's columns: m, or a block's)
+    return cus // 2 < buckets <= cus or (slab and n * m >= 6 * k * buckets)
+
+
 def _launch(int4, bitstream, syms, lens, table, col_start, col_len, offsets, rows, group_col, group_size,
             startbit, bit_base, n, m, max_len, out) -> torch.Tensor:
     dev = int4.device
@@ -188,21 +226,14 @@ def _launch(int4, bitstream, syms, lens, table, col_start, col_len, offsets, row
     d.n, d.m, d.out = n, m, out.data_ptr()
     if n * m >= (1 << 31):
         raise ValueError("tensor too large for the AWQ decode kernel (n*m >= 2^31)")
-    # From its second call on a sidecar that the slab paths can take (k = 256, 512 or
-    # 1024: row buckets, or by-scale groups of a power of two of 64 columns up to k, or of
-    # 1024 columns or more) the op launches the sidecar's cached plan; other sidecars
-    # (whose plans would take the per-lane path, slower than this kernel's two workgroups
-    # per bucket when a tensor has fewer buckets than CUs) and the first call decode over
-    # whole buckets, as the reference does.
     key_tensors = tuple(t for t in (int4, bitstream, syms, lens, table, col_start, col_len, offsets, rows, group_col,
                                     startbit, bit_base) if t is not None)
-    k = startbit.size(1) - 1
-    gs = int(group_size)
-    slab = k in (256, 512, 1024) and (group_col is None or gs >= 1024 or (64 <= gs <= k and gs & (gs - 1) == 0))
+    slab = table.size(0) > 0 and _op_takes_plan(startbit.size(1) - 1, n, m, table.size(0), rows.numel(), int(group_size),
+                                                _compute_units(dev.index or 0))
     with torch.cuda.device(dev):
         stream = _stream_handle(dev)
         plan = None
-        if slab and table.size(0) > 0 and out.data_ptr() % 8 == 0:
+        if slab and out.data_ptr() % 8 == 0:
             plan = _plan_cache().get(key_tensors, n, m, d, dev, stream, extra=(int(group_size),))
         if plan is not None:
             plan.decode_into(out, stream)
