@@ -73,8 +73,18 @@ class BuilderOutputs:
         """Runs ``entry`` (mps_*_encode_alloc); (sizes, stats) of its outputs."""
         sizes, stats = (ctypes.c_int64 * 17)(), (ctypes.c_int64 * 4)()
         rc = entry(ctypes.byref(args), ctypes.c_void_p(stream), _native.ENCODE_ALLOC(self._alloc), None, sizes, stats)
-        if self._error is not None:
-            raise self._error
+        error, self._error = self._error, None
+        if error is not None or rc != 0:
+            # The stream is idle. The error's traceback holds _alloc's frame and so this object:
+            # it must hold neither the error (a cycle) nor the build's memory, which a caller
+            # that tries again would find still taken.
+            self._out.clear()
+            self._work.clear()
+        if error is not None:
+            try:
+                raise error
+            finally:
+                del error
         _native.check(rc)
         return sizes, stats
 
