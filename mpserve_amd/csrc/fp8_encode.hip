@@ -1794,12 +1794,14 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
                o_rows = put(row_indices.data(), 4 * row_indices.size()), o_cols = put(cols.data(), 4 * cols.size()),
                o_clen = put(col_len.data(), 4 * (size_t)B), o_shape = put(shape, 8 * nshape);
   char *blk = nullptr;
-  bool placed = false;  // the outputs among the host-built arrays are made once
   uint32_t *flags = nullptr, *d_lane_base = nullptr, *tcount = nullptr, *tgid = nullptr, *gid_tkey = nullptr;
   int32_t *d_row_offsets = nullptr, *d_row_indices = nullptr, *d_cols = nullptr, *d_col_len = nullptr;
   auto at32 = [&](size_t o) { return reinterpret_cast<uint32_t *>(blk + o); };
   // Allocates the block as laid out so far, uploads it and places the outputs it holds.
+  // (Where the unit passes gave up after theirs, that block stays: the general path
+  // uses its host-built arrays, and clears the flags itself.)
   auto upload = [&]() -> int {
+    if (blk) return MPS_OK;
     if (!(blk = static_cast<char *>(alloc(ctx, -1, (int64_t)bytes))))
       return fail(MPS_ERR_NO_MEMORY, "no device memory for the sidecar builder's workspace (%zu bytes)", bytes);
     HC(hipMemcpyAsync(blk, host.data(), host.size(), hipMemcpyHostToDevice, s));
@@ -1809,8 +1811,6 @@ int encode_impl(const EncodeSpec &sp, hipStream_t s, mps_encode_alloc alloc, voi
     d_row_indices = dealt ? dealt_rows : reinterpret_cast<int32_t *>(blk + o_rows);
     d_cols = dealt && by_scale ? dealt_cols : reinterpret_cast<int32_t *>(blk + o_cols);
     d_col_len = reinterpret_cast<int32_t *>(blk + o_clen);
-    if (placed) return MPS_OK;
-    placed = true;
     OUT(x4, uint16_t, 4, (size_t)B);
     OUT(x5, int32_t, 5, row_offsets.size());
     int32_t *x6 = dealt_rows, *x8 = dealt_cols;  // (or their buffers, where the sort had too many scales)

@@ -55,3 +55,26 @@ def test_awq_build_on_a_side_stream_is_complete(by_scale):
         with torch.cuda.stream(side):
             build(w.bf16, w.int4_u8, w.scale_u16, 11, 1024)
         assert side.query()
+
+
+@pytest.mark.parametrize("n_sym", [3000, 65536])
+def test_general_path_takes_the_unit_passes_block(n_sym, monkeypatch):
+    """A build whose pairs overflow the unit passes' tables (random bits) asks for one block of work
+    memory beside the scales', as one that stays on them does."""
+    from mpserve_amd._common import BuilderOutputs
+
+    print(f"[streams] work memory, {n_sym} symbols", flush=True)
+    real, work = BuilderOutputs._alloc, []
+
+    def count(self, ctx, slot, nbytes):
+        if slot < 0:
+            work.append(nbytes)
+        return real(self, ctx, slot, nbytes)
+
+    monkeypatch.setattr(BuilderOutputs, "_alloc", count)
+    g = torch.Generator(device=DEV).manual_seed(n_sym)
+    w = torch.randint(0, n_sym, (256, 900), generator=g, device=DEV).to(torch.int16).view(torch.bfloat16)
+    q = torch.randint(0, 256 if n_sym == 65536 else 2, (256, 900), generator=g, device=DEV, dtype=torch.uint8)
+    s = torch.full((1,), 0x1C00, dtype=torch.int16, device=DEV).view(torch.uint16)
+    MPServe_cuda.huffman_build_fp8_decode_tables(w, q, s, 7, 1024)
+    assert len(work) == 2
