@@ -199,3 +199,63 @@ def test_scales_ranked_and_dealt(n, shift, distinct):
         torch.from_numpy(bf.view(np.int16)).to(DEV).view(torch.bfloat16), torch.from_numpy(q).to(DEV),
         base[shift:].view(torch.uint16), 7, 64)
     _same({x: v.cpu().numpy() for x, v in got.items()}, oracle.encode(bf, q, sc, 7, 64))
+
+
+@pytest.mark.parametrize("n,m,group,distinct", [
+    (1100, 512, 64, 150), (1100, 512, 64, 4096),  # 8800 groups dealt to their scales on the GPU
+    (1100, 512, 64, 4097), (1100, 512, 64, 8800),  # with too many scales for that: the host's loop into the same outputs
+    (2731, 24, 8, 7),                              # 8193 groups, three a row
+])
+@pytest.mark.parametrize("cap", [1024, 37])
+def test_groups_dealt_to_their_scales(n, m, group, distinct, cap):
+    """By-scale builds of 8192 groups and more: rows and columns of every bucket's groups, in order."""
+    print(f"[units] awq {n}x{m} group {group}, {distinct} scales, cap {cap}", flush=True)
+    rng = np.random.default_rng(distinct)
+    bf = (0x3C00 + rng.integers(0, 40, size=(n, m))).astype(np.uint16)
+    q = rng.integers(0, 16, size=(n, m)).astype(np.uint8)
+    sc = rng.choice(65536, size=distinct, replace=False).astype(np.uint16)
+    groups = n * (m // group)
+    sc = rng.permutation(np.concatenate([sc, rng.choice(sc, size=groups - distinct)])).reshape(n, m // group)
+    got = MPServe_cuda.huffman_build_awq_int4_bucket_decode_tables_by_scale(
+        torch.from_numpy(bf.view(np.int16)).to(DEV).view(torch.bfloat16), torch.from_numpy(q).to(DEV),
+        torch.from_numpy(sc.view(np.int16)).view(torch.uint16), 11, 64, cap)
+    want = oracle.awq_encode(bf, q, sc, 11, 64, cap, True)
+    got = {x: v.cpu().numpy() for x, v in got.items()}
+    assert list(got) == list(want)
+    for x, v in want.items():
+        assert got[x].shape == v.shape and np.array_equal(got[x].view(v.dtype), v), x
+
+
+@pytest.mark.parametrize("L,n_sym", [(7, 65), (7, 128), (11, 513), (11, 2048)])
+def test_long_list_with_sums_that_could_wrap(L, n_sym):
+    """A key of 179.5 million elements (past (2^31 - 1) / 12): its list's merge runs in sequence, in each of the
+    workgroup-a-key kernels. Code lengths against the oracle's package-merge of the counts."""
+    print(f"[units] {n_sym} symbols, 179.5 million elements", flush=True)
+    n, m = 13000, 13808
+    rng = np.random.default_rng(n_sym)
+    counts = np.maximum(1, (rng.random(n_sym) ** 6 * 1e6).astype(np.int64))
+    counts = np.maximum(1, counts * (n * m) // counts.sum())
+    counts[counts.argmax()] += n * m - counts.sum()
+    assert counts.sum() == n * m and counts.min() >= 1
+    syms = 0x3C00 + np.arange(n_sym)
+    bf = torch.repeat_interleave(torch.from_numpy(syms.astype(np.int16)).to(DEV), torch.from_numpy(counts).to(DEV))
+    q = torch.full((n, m), 0x40, dtype=torch.uint8, device=DEV)
+    sc = torch.full((1,), 0x1C00, dtype=torch.int16, device=DEV).view(torch.uint16)
+    got = MPServe_cuda.huffman_build_fp8_decode_tables(bf.view(n, m).view(torch.bfloat16), q, sc, L, 1024)
+    order = np.lexsort((syms, counts))
+    lens = np.empty(n_sym, dtype=np.int64)
+    lens[order] = oracle.package_merge([int(c) for c in counts[order]], L)
+    table = got["decode_syms_u16"].cpu().numpy()
+    packed = got["decode_lens_u8"].cpu().numpy()
+    assert table.shape == (1, 1 << L)
+    nib = np.stack([packed & 15, packed >> 4], axis=-1).reshape(-1)
+    entry = table[0].astype(np.int64) - 0x3C00
+    assert np.array_equal(np.bincount(entry, minlength=n_sym), 1 << (L - lens)) and np.array_equal(nib, lens[entry])
+    # codes of a length in list order, ascending
+    starts = np.concatenate([[True], entry[1:] != entry[:-1]])
+    want = order[np.argsort(lens[order], kind="stable")]
+    assert np.array_equal(entry[starts], want)
+    assert int(got["bucket_bit_base_i64"][-1]) > 0
+    total = int((counts * lens).sum())
+    bits = got["bucket_thread_startbit_u32"].cpu().numpy().astype(np.int64)[:, -1].sum()
+    assert bits == total
