@@ -1538,7 +1538,8 @@ constexpr int64_t kMaxQueueItems = (int64_t(1) << 30) - 65536;
 // half), its tables' return (word 7 high half), the end of its table expansion
 // (word 8 low half), the set-up's first barrier (word 8 high half) and the
 // last wave's tables (word 9). Threads 0 and 960 write them with ordinary
-// stores after the barrier; words 10 and 11 are spare.
+// stores after the barrier; words 10 and 11 are spare. (Each translation unit has its
+// own; the host reads fp8_decode.hip's, whose kernels see no flat items.)
 #if MPS_TRACE_ITEMS
 constexpr int kTraceWgs = 256, kTraceItems = 128, kTraceWords = 12;
 __device__ uint64_t g_item_trace[kTraceWgs * kTraceItems * kTraceWords];

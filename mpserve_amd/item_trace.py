@@ -47,6 +47,15 @@ def _lib(path: str) -> ctypes.CDLL:
     return lib
 
 
+def _require_records(valid: np.ndarray) -> None:
+    """The trace's memory belongs to the kernels of aligned plans. A plan with flat buckets (columns
+    that are no multiple of the substreams) or other AWQ group sizes launches kernels of other
+    translation units, whose records nothing here reads."""
+    if not valid.any():
+        raise RuntimeError("no items were traced: plans with flat buckets or AWQ groups of other sizes than 128 "
+                           "columns run kernels outside the trace")
+
+
 def fp8_trace(lib_path: str, workload: str, k: int) -> Dict:
     import torch
 
@@ -92,6 +101,7 @@ def fp8_trace(lib_path: str, workload: str, k: int) -> Dict:
         lib.mps_fp8_plan_destroy(plan)
     a = np.frombuffer(buf, dtype=np.uint64).reshape(256, 128, 12).astype(np.int64)
     valid = a[:, :, 1] > 0
+    _require_records(valid)
     t0 = int(a[:, :, 0][valid].min())
     rec = a[valid]
     dur = (rec[:, 1] - rec[:, 0]) / 100.0  # us
@@ -184,6 +194,7 @@ def awq_trace(lib_path: str, k: int) -> Dict:
         finally:
             lib.mps_awq_plan_destroy(plan)
         a = np.frombuffer(buf, dtype=np.uint64).reshape(8192, 4).astype(np.int64)
+        _require_records(a[:, 1] > 0)
         a = a[a[:, 1] > 0]
         t0 = int(a[:, 0].min())
         dur = (a[:, 1] - a[:, 0]) / 100.0
