@@ -103,6 +103,12 @@ __global__ __launch_bounds__(kAwqBlock) void awq_checkpoints(const mps_awq_tenso
     const int32_t dr = K / cl, dc = K - dr * cl;
     int32_t rr = tid / cl, cc = tid - rr * cl, seen = -1;
     int64_t base = 0;
+    // The walk stops at the last range's start; the rows after it are checked here, so that a
+    // bucket with a bad one keeps its per-lane record, which drops that row alone.
+    for (int32_t r = tid; r < T.bucket_row_offsets[J.bucket + 1] - ra; r += K) {
+      const int32_t row = T.row_indices[ra + r], c0 = T.group_col_start ? T.group_col_start[ra + r] : J.c0;
+      if (row < 0 || row >= T.n || c0 < 0 || (int64_t)c0 + cl > T.m) failed[blockIdx.x] = 1u;
+    }
     for (int j = 1; j < J.ranges; ++j) {
       for (int32_t i = (j - 1) * J.range_rows; i < j * J.range_rows; ++i) {
         if (rr != seen) {
@@ -272,7 +278,7 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
   // at most kRowSlots / 4 rows each, so they can share a workgroup's tables
   // (kind 0).
   std::vector<AwqWork> base;
-  std::vector<int32_t> roff, clen, cst, btab, gcol;
+  std::vector<int32_t> roff, clen, cst, btab, gcol, grow;
   // Elements a by-scale slab record's run of buckets may hold: a CU's share
   // of the plan (records go out largest first, so the large ones run early
   // and small ones fill the end; half a share measured 0.9% slower on an 8B
@@ -319,7 +325,16 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
     if ((slab_tensor || bmulti_tensor) && T.group_col_start && T.num_row_indices > 0) {
       gcol.resize((size_t)T.num_row_indices);
       MPS_HIP_CHECK(hipMemcpy(gcol.data(), T.group_col_start, sizeof(int32_t) * T.num_row_indices, hipMemcpyDefault));
-      const bool aligned = std::all_of(gcol.begin(), gcol.end(), [](int32_t c) { return (c & 3) == 0; });
+      bool aligned = std::all_of(gcol.begin(), gcol.end(), [](int32_t c) { return (c & 3) == 0; });
+      // The slab path drops a bucket (a range, a wave's groups) with a bad group. Other sizes than
+      // 128 columns came to it from the per-lane path, which drops that group alone: with a bad
+      // group among them they stay there.
+      if (aligned && T.group_size != 128) {
+        grow.resize(gcol.size());
+        MPS_HIP_CHECK(hipMemcpy(grow.data(), T.row_indices, sizeof(int32_t) * T.num_row_indices, hipMemcpyDefault));
+        for (size_t g = 0; g < grow.size() && aligned; ++g)
+          aligned = grow[g] >= 0 && grow[g] < T.n && gcol[g] >= 0 && gcol[g] + T.group_size <= T.m;
+      }
       slab_tensor = slab_tensor && aligned;
       bmulti_tensor = bmulti_tensor && aligned;
     }

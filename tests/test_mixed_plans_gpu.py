@@ -93,3 +93,29 @@ def test_fp8_aligned_and_flat_weights(shapes):
     assert plan.read_status() == 0
     for (bf, (_, _, out)), s in zip(items, shapes):
         np.testing.assert_array_equal(out.view(torch.uint16).cpu().numpy(), bf, err_msg=str(s))
+
+
+@pytest.mark.parametrize("n,m,group,k", [
+    (40, 1500, None, 1024), (300, 4099, None, 256),   # flat: one range; several side by side
+    (256, 1024, 64, 1024), (512, 1024, 256, 256), (40, 1500, 1500, 512),
+])
+@pytest.mark.parametrize("at", [0.0, 0.99])
+def test_awq_bad_row_is_dropped_alone(n, m, group, k, at, monkeypatch):
+    """A row (group) index out of range in sidecars that left the per-lane path: flagged, and the other
+    rows decode as they do there."""
+    print(f"[mixed] bad row {n}x{m} group {group} k{k} at {at}", flush=True)
+    from mpserve_amd._native import MPS_STATUS_BAD_ROW
+
+    q, sc = _awq_item(n, m, group, k)
+    key = "group_rows_i32" if group else "row_indices_i32"
+    sc[key] = sc[key].clone()
+    sc[key][int(at * sc[key].numel())] = n
+    outs = []
+    for slab in ("0", "1"):
+        monkeypatch.setenv("MPSERVE_AWQ_SLAB", slab)
+        out = torch.zeros((n, m), dtype=torch.bfloat16, device=DEV)
+        plan = awq.AwqDecodePlan([(q, sc, out)])
+        plan.decode()
+        assert plan.read_status() & MPS_STATUS_BAD_ROW
+        outs.append(out.view(torch.int16))
+    assert torch.equal(outs[0], outs[1]) and int((outs[0] != 0).any(dim=1).sum()) >= n - 1
