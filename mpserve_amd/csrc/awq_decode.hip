@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kAwqBlock) void awq_decode_kernel(mps_awq_tensor T,
 // (the plan then keeps the bucket whole, and its decode reports them). A `full`
 // job (ranges side by side, k 256 or 512) also writes rows 0 (the substreams'
 // start bits) and `ranges` (their end bits). A by-scale job's ranges are ranges
-// of slabs (`range_rows` slabs of k / 128 groups each; `rows`: the groups).
+// of slabs (`range_rows` slabs of k / group_size groups each; `rows`: the groups).
 struct AwqSplitJob {
   int32_t tensor, bucket, P, rows;
   int32_t c0, range_rows, ranges;
@@ -311,14 +311,14 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
       clen.resize((size_t)B);
       MPS_HIP_CHECK(hipMemcpy(clen.data(), T.bucket_col_len, sizeof(int32_t) * B, hipMemcpyDefault));
     }
-    // The slab path (k = 1024: by-scale with 128-column groups, or row buckets of
+    // The slab path (k = 1024: by-scale with groups slab_group takes, or row buckets of
     // 1..128 rows over P >= 4 blocks of 1024 columns) loads int4 bytes as dwords
     // and stores 8 bytes a lane: every group or column range must start on a
     // 4-element boundary and the buffers must be aligned to match.
     bool slab_tensor = slab_on && T.k == kAwqBlock && (!T.group_col_start || slab_group(T.group_size, T.k)) &&
                        T.m % 4 == 0 && (reinterpret_cast<uintptr_t>(T.int4) & 3u) == 0 && (reinterpret_cast<uintptr_t>(T.out) & 7u) == 0;
-    // By-scale sidecars with k 256 or 512 and 128-column groups: buckets cut into
-    // ranges of slabs (k / 128 groups each), 1024 / k ranges side by side a record.
+    // By-scale sidecars with k 256 or 512 and such groups: buckets cut into ranges
+    // of slabs (k / group_size groups each), 1024 / k ranges side by side a record.
     bool bmulti_tensor = slab_on && (T.k == 256 || T.k == 512) && T.group_col_start &&
                          slab_group(T.group_size, T.k) && T.m % 4 == 0 && (reinterpret_cast<uintptr_t>(T.int4) & 3u) == 0 &&
                          (reinterpret_cast<uintptr_t>(T.out) & 7u) == 0;
@@ -486,7 +486,7 @@ int mps_awq_plan_create(const mps_awq_tensor *tensors, int64_t count, void *stre
     const AwqWork &w = base[r];
     const int32_t rows = rows_of_rec[r], P = p_of_rec[r];
     if (k_of_rec[r] > 0) {
-      // units: rows, or slabs of k / 128 groups (by-scale, at most 128 a range: the
+      // units: rows, or slabs of k / group_size groups (by-scale, at most 128 a range: the
       // slab path keeps a wave's 128 group bases in two registers)
       // More than one record only while each range keeps >= min_lane elements a lane.
       const int64_t S = kAwqBlock / k_of_rec[r];

@@ -318,7 +318,8 @@ __device__ __forceinline__ void awq_bucket(const mps_awq_tensor &T, int64_t b, i
 }
 
 // ---------------------------------------------------------------------------
-// Slab path: by-scale buckets with k = 1024 substreams and groups of 128
+// Slab path, told here for k = 1024 substreams and groups of 128 columns (other
+// sizes, slab_group, and k 256 and 512 likewise): by-scale buckets with groups of 128
 // columns (8 to 1024 groups). Element e of such a bucket is column e % 128 of
 // its group e / 128, and substream t codes e = t, t + 1024, ...: the i-th
 // element of every substream lies in *slab* i, the bucket's groups 8i .. 8i+7.
@@ -851,9 +852,9 @@ __device__ __forceinline__ void awq_slab_decode(const mps_awq_tensor &T, const u
   if (0u - np - 64u != pos_end) flag(status, MPS_STATUS_DESYNC);
 }
 
-// One slab-path bucket, checked by the plan: k = 1024 and either by-scale
-// with 128-column groups and 8 .. 1024 groups, or a row bucket of 1 .. 128 rows
-// whose column range is P >= 4 blocks of 1024. Set-up in two levels of loads,
+// One slab-path bucket, checked by the plan: by-scale with one to 128 slabs of
+// whole groups, or a row bucket of 1 .. 128 rows whose column range is P >= 4
+// blocks of k, or flat (kRanged 3). Set-up in two levels of loads,
 // each issued in full before any result is used: (1) the table ids, the
 // wave's group rows and column starts (or the bucket's rows), the lane's start
 // and end bits; (2) the tables' slices and the lane's first bitstream words.

@@ -4,10 +4,11 @@
 // huffman_build_fp8_decode_tables_entry (kernel/build_huffman.cu:292-969) produces:
 //   1. histogram of (scale, fp8) keys x BF16 symbols    (:392-401)
 //   2. keys in ascending order -> table id (gid)         (:403-412)
-//   3. per key: ESC selection, package-merge lengths,    (:445-578)   -> one wave per key, in LDS
+//   3. per key: ESC selection, package-merge lengths,    (:445-578)   -> a wave or a workgroup per key, in LDS
 //      canonical codes in (count asc, sym asc) order,
 //      decode LUT and packed 4-bit lengths
-//   4. row buckets, bucket_table, U/uniq/uidx            (:582-783)   -> host (O(rows)) + a kernel
+//   4. row buckets, bucket_table, U/uniq/uidx            (:582-783)   -> rows dealt to their scales by a counting
+//                                                                        sort (few: on the host), tables by a kernel
 //   5. per-lane bit counts, u32 lane starts, 64-bit      (:786-925)
 //      aligned bucket bases, MSB-first packing
 // Steps 1, 2 and 5 run on units of one bucket over tables in LDS
@@ -249,7 +250,7 @@ __global__ void table_list_kernel(const uint32_t *tcount, const uint32_t *tgid, 
 }
 
 // ---------------------------------------------------------------------------
-// 3. Code book of one key (one work-item per key)
+// 3. Code book of one key, L >= 12 (one work-item per key; L <= 11 further down)
 // ---------------------------------------------------------------------------
 // Items (count, sym) compare as the reference's std::pair<int, uint16_t>.
 // Items are ordered by (count, symbol) with counts compared as int, as the
@@ -2307,10 +2308,6 @@ int no_throw(F &&f) {
 
 }  // namespace
 }  // namespace mps
-
-extern "C" {
-
-}  // extern "C"
 
 namespace {
 // The argument checks of mps_fp8_encode: the run to make, or an error.
