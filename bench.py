@@ -96,8 +96,8 @@ def parse_args(argv=None):
                         "one process, launches interleaved in rounds; prints one JSON line of medians")
     p.add_argument("--compare-rounds", type=int, default=6, help="--compare-libs: rounds (20 launches per library each)")
     p.add_argument("--vram-pretouch-gib", type=int, default=48, metavar="GIB",
-                   help="before anything else, allocate, fill and free this much device memory (0: skip); on a "
-                        "fresh box the decode of buffers placed on never-used memory runs about 6%% slower")
+                   help="before anything else, allocate, fill and free this much device memory (0: skip): part "
+                        "of what sets where the buffers land")
     p.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
                    help="after the timed steps, run 3 plain int32 elementwise copies of MIB MiB each "
                         "(reference kernel of known bytes for scaling rocprofv3 FETCH_SIZE/WRITE_SIZE)")
@@ -678,11 +678,10 @@ def headline(entries, dev, args, build_s: float):
 
 def vram_pretouch(dev, gib: int) -> int:
     """Allocate, fill and free ``gib`` GiB of device memory, and return it to
-    the driver. On a freshly assigned box, a process whose model sits on memory
-    no earlier allocation used decodes at one level for its whole life (5.75 ms
-    for the model); after this the same process measures 5.30-5.50 ms, as every
-    later process on the box does without it. It runs before the inputs exist,
-    outside every timed region. Returns the GiB it touched (0: skipped)."""
+    the driver: one of the things that set where the model's buffers land, and so
+    the level a process decodes at (5.1-5.8 ms for the model, by layout). It runs
+    before the inputs exist, outside every timed region. Returns the GiB it
+    touched (0: skipped)."""
     import torch
 
     if gib <= 0:
